@@ -16,7 +16,10 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <type_traits>
+
 #include "gs_common.h"
+#include "gs_wave.h"
 
 namespace gs {
 
@@ -90,6 +93,7 @@ struct DenseK {
   int which;
   Phys<T> P;
   int rain_mode;  // 0 none, 1 uniform, 2 gridded
+  int wave;       // kWave* flags of P
   const S* rain_frames;
   int64_t frame_stride, rain_pitch;
   int stage;
@@ -129,33 +133,375 @@ __device__ __forceinline__ ColMap col_map(int c, int ny, int bc) {
   return m;
 }
 
-// h, hu, hv of cell (i, column map cm); the row map is uniform across the wavefront.
-template <typename T, typename S>
-__device__ __forceinline__ void load_q(const DenseK<T, S>& a, S* const* q, int i, const ColMap& cm, T& h, T& hu,
-                                       T& hv) {
-  bool zx = false, fx = false;
-  const int mi = map_state(i, a.nx, a.bc_x, zx, fx);
-  const int64_t idx = (int64_t)mi * a.pitch + cm.mj;
-  h = (T)q[0][idx];
-  hu = (T)q[1][idx];
-  hv = (T)q[2][idx];
-  if (fx) hu = -hu;
-  if (cm.flip) hv = -hv;
-  if (zx || cm.zero) { h = T(0); hu = T(0); hv = T(0); }
+// Element at byte offset `off` of a row that starts at `row` (uniform): the row's address stays
+// in scalar registers and the lane adds a 32-bit offset, so an access costs no vector address
+// arithmetic. O is uint32_t unless a row spans 4 GiB or more.
+template <typename P, typename O>
+__device__ __forceinline__ GS_G P& row_at(GS_G P* row, O off) {
+  // a value of its own, widened beside the access: a widening hoisted out of the row loop would
+  // make the lane's address a 64-bit vector add
+  if (sizeof(O) == 4) __asm__("" : "+v"(off));
+  typedef typename std::conditional<std::is_const<P>::value, const char, char>::type B;
+  return *(GS_G P*)((GS_G B*)row + off);
 }
 
+// What a tile's rows read besides the kernel argument.
 template <typename T, typename S>
-__device__ __forceinline__ T load_b(const DenseK<T, S>& a, int i, const ColMap& cm) {
-  const int mi = map_bed(i, a.nx, a.bc_x);
-  return (T)a.bed[(int64_t)mi * a.pitch + cm.mjb];
+struct DenseTile {
+  const S* qi[3];
+  S* qo[3];
+  const S* frame;      // gridded rain frame of this step
+  const T* ntab;       // Manning n per class (LDS)
+  T rain, eta, n0;     // n0: the Manning n of a domain with no classes
+  int c;               // the lane's column
+  bool col_ok;         // the lane writes its cell
+  bool edge;           // the tile's stencils reach ghost rows or columns
+  ColMap cm;
+};
+
+// One row of a lane's column as it lies in memory. The loads of a row are issued one row ahead of
+// its use; what the row then needs (the ghost rules, a conversion) waits until then.
+template <typename S>
+struct RawRow {
+  S h, hu, hv;
+};
+
+template <typename O, typename T, typename S>
+__device__ __forceinline__ void load_q(const DenseK<T, S>& a, const DenseTile<T, S>& x, int i, RawRow<S>& r) {
+  int mi = i;
+  if (x.edge) {
+    bool zx = false, fx = false;
+    mi = map_state(i, a.nx, a.bc_x, zx, fx);
+  }
+  const int64_t row = (int64_t)mi * a.pitch;
+  const O off = (O)(uint32_t)x.cm.mj * (O)sizeof(S);
+  r.h = row_at(row_base(x.qi[0] + row), off);
+  r.hu = row_at(row_base(x.qi[1] + row), off);
+  r.hv = row_at(row_base(x.qi[2] + row), off);
+}
+// The cell's state from the loaded row i.
+template <typename T, typename S>
+__device__ __forceinline__ void use_q(const DenseK<T, S>& a, const DenseTile<T, S>& x, int i, const RawRow<S>& r, T& h,
+                                      T& hu, T& hv) {
+  h = (T)r.h;
+  hu = (T)r.hu;
+  hv = (T)r.hv;
+  if (x.edge) {
+    bool zx = false, fx = false;
+    (void)map_state(i, a.nx, a.bc_x, zx, fx);
+    if (fx) hu = -hu;
+    if (x.cm.flip) hv = -hv;
+    if (zx || x.cm.zero) { h = T(0); hu = T(0); hv = T(0); }
+  }
 }
 
+template <typename O, typename T, typename S>
+__device__ __forceinline__ S load_b(const DenseK<T, S>& a, const DenseTile<T, S>& x, int i) {
+  const int mi = x.edge ? map_bed(i, a.nx, a.bc_x) : i;
+  return row_at(row_base(a.bed + (int64_t)mi * a.pitch), (O)(uint32_t)x.cm.mjb * (O)sizeof(S));
+}
 
-// MODE 0: residual into a.rhs; MODE 1: fused step.
-template <typename T, int MODE, typename S = T>
-__global__ __launch_bounds__(kBlock) void k_dense_sweep(DenseK<T, S> a) {
+// The four faces of a cell in the reference's order. A face gated off (both cells dry) adds
+// zeros: the sums start at +0 and IEEE addition yields -0 only from two -0 terms, so they never
+// hold -0, and x + 0 = x - 0 = x for every other x.
+template <typename T>
+__device__ __forceinline__ void sum_faces(const FaceProd<T>& up, const FaceProd<T>& dn, const FaceProd<T>& right,
+                                          T lFh, T lFN, T lFT, T lsR, T& rh, T& rhu, T& rhv) {
+  rh = T(0); rhu = T(0); rhv = T(0);
+  rh = rh - up.Fh;
+  rhu = rhu - up.FN;
+  rhv = rhv - up.FT;
+  rhu = rhu - up.sL;
+  rh = rh + dn.Fh;
+  rhu = rhu + dn.FN;
+  rhv = rhv + dn.FT;
+  rhu = rhu + dn.sR;
+  rh = rh - right.Fh;
+  rhu = rhu - right.FT;
+  rhv = rhv - right.FN;
+  rhv = rhv - right.sL;
+  rh = rh + lFh;
+  rhu = rhu + lFT;
+  rhv = rhv + lFN;
+  rhv = rhv + lsR;
+}
+
+// face() as the products its cells add, zero where it is gated off.
+template <typename T>
+__device__ __forceinline__ void face_prod(T bL, T bR, T gzL, T gzR, T hL, T hR, T uNL, T uTL, T uNR, T uTR, T half,
+                                          T inv, T g, T hm, FaceProd<T>& f) {
+  Face<T> q;
+  face<T>(bL, bR, gzL, gzR, hL, hR, uNL, uTL, uNR, uTR, half, g, hm, q);
+  f.Fh = q.gate ? q.Fh * inv : T(0);
+  f.FN = q.gate ? q.FN * inv : T(0);
+  f.FT = q.gate ? q.FT * inv : T(0);
+  f.sL = q.gate ? q.srcL * inv : T(0);
+  f.sR = q.gate ? q.srcR * inv : T(0);
+}
+
+// What a cell's update reads from its planes. Lanes that write nothing read nothing. LEAN: the
+// domain has no flags, Manning, class and running-max plane and no gridded rain.
+template <bool LEAN, typename T, typename S>
+__device__ __forceinline__ void cell_inputs(const DenseK<T, S>& a, const DenseTile<T, S>& x, int i, T& rh, T& rhu,
+                                            T& rhv, T& rr0, T& n, uint8_t& fl) {
+  fl = 0;
+  rr0 = rh;
+  n = T(0);
+  if (LEAN) {
+    rr0 = rr0 + x.rain;   // + 0 without rain: rh is not -0
+    n = x.n0;
+    return;
+  }
+  const int64_t idx = (int64_t)i * a.pitch + x.c;
+  if (a.flags) {
+    if (x.col_ok) fl = a.flags[idx];
+    if (fl & GS_FLAG_INACTIVE) { rh = T(0); rhu = T(0); rhv = T(0); }
+    rr0 = rh;
+  }
+  if (a.rain_mode == 1) {
+    rr0 = rr0 + x.rain;
+  } else if (a.rain_mode == 2) {
+    if (x.col_ok) rr0 = rr0 + (T)x.frame[(int64_t)i * a.rain_pitch + x.c];
+  }
+  if (a.flags && (fl & GS_FLAG_INACTIVE)) rr0 = rh;
+  if (a.P.friction) {
+    if (a.n_field || a.cls) {
+      if (x.col_ok) n = a.n_field ? (T)a.n_field[idx] : x.ntab[a.cls[idx]];
+    } else {
+      n = x.ntab[fl & GS_FLAG_CLASS_MASK];
+    }
+  }
+}
+
+template <bool LEAN, typename O, typename T, typename S>
+__device__ __forceinline__ void cell_store(const DenseK<T, S>& a, const DenseTile<T, S>& x, int i, S h, S hu, S hv) {
+  const int64_t row = (int64_t)i * a.pitch;
+  const O out = (O)(uint32_t)x.c * (O)sizeof(S);
+  GS_G S* r0 = row_base(x.qo[0] + row);
+  GS_G S* r1 = row_base(x.qo[1] + row);
+  GS_G S* r2 = row_base(x.qo[2] + row);
+  if (x.col_ok) {
+    if (!LEAN && a.max_h && h > a.max_h[row + x.c]) a.max_h[row + x.c] = h;
+    row_at(r0, out) = h;
+    row_at(r1, out) = hu;
+    row_at(r2, out) = hv;
+  }
+}
+
+// Rows i0 .. i_end-1 of a tile by the wavefront forms (gs_wave.h). Returns the first row that it
+// leaves to dense_rows_general: one whose stencil or update holds an operand outside their
+// bounds, before anything of that row is written; i_end where there is none.
+template <typename T, int MODE, bool LEAN, typename S, typename O>
+__device__ __forceinline__ int dense_rows(const DenseK<T, S>& a, const DenseTile<T, S>& x, const WaveC<T>& w, int i0,
+                                          int i_end, lam_t<T>& lam) {
+  // lanes whose cell is written, whose y-face is used and whose cell a used face reads
+  const lmask act = lm_of(x.col_ok);
+  const lmask yuse = act | (act >> 1), cuse = yuse | (act << 1);
+  lmask odd = 0;
+  const Lanes ln = lanes_of(threadIdx.x & 63);
+
+  const S sm2 = load_b<O>(a, x, i0 - 2), sm1 = load_b<O>(a, x, i0 - 1), s0 = load_b<O>(a, x, i0),
+          s1 = load_b<O>(a, x, i0 + 1);
+  RawRow<S> rP, rC, rN;   // rN: the next row of the state, and sp2 the bed of the row after it
+  load_q<O>(a, x, i0 - 1, rP);
+  load_q<O>(a, x, i0, rC);
+  load_q<O>(a, x, i0 + 1, rN);
+  S sp2 = load_b<O>(a, x, i0 + 2);
+  const T bm2 = (T)sm2, bm1 = (T)sm1;
+  T b0 = (T)s0, bp1 = (T)s1;
+  T hP, huP, hvP, uP, vP, hC, huC, hvC, uC, vC;
+  use_q<T>(a, x, i0 - 1, rP, hP, huP, hvP);
+  use_q<T>(a, x, i0, rC, hC, huC, hvC);
+  lmask dryP, dryC;
+  prims_w<T>(hP, huP, hvP, vabs(bm2) + vabs(bm1), cuse, w, uP, vP, dryP, odd);
+  prims_w<T>(hC, huC, hvC, vabs(b0) + vabs(bp1), cuse, w, uC, vC, dryC, odd);
+  const T zxP = w.hdx * ((T(0.5) * (b0 - bm2)) * w.ix);
+  T zxC = w.hdx * ((T(0.5) * (bp1 - bm1)) * w.ix);
+  FaceProd<T> fx;   // the x-face below the current row
+  face_w<T>(bm1, b0, zxP, zxC, hP, hC, uP, vP, uC, vC, dryP, dryC, act, w.ix, w, fx, odd);
+
+  // where the written lanes' results go (offsets of 32 bits within the tile)
+  const StoreBase st0 = store_base(x.qo[0] + (int64_t)i0 * a.pitch), st1 = store_base(x.qo[1] + (int64_t)i0 * a.pitch),
+                  st2 = store_base(x.qo[2] + (int64_t)i0 * a.pitch);
+  const uint32_t lane_st = x.col_ok ? (uint32_t)x.c * (uint32_t)sizeof(S) : kNoStore;
+  const uint32_t pitch_st = (uint32_t)a.pitch * (uint32_t)sizeof(S);
+  take_loaded(rN.h, rN.hu, rN.hv, sp2);   // nothing is in flight when the rows begin
+
+  // one row; false if it is left to the general functions
+  auto row = [&](int i) __attribute__((always_inline)) -> bool {
+    T hN, huN, hvN;
+    RawRow<S> r = rN;
+    S sb = sp2;
+    take_loaded(r.h, r.hu, r.hv, sb);
+    const int ipf = min(i + 2, i_end);   // the last rows load again what they have
+    load_q<O>(a, x, ipf, rN);
+    sp2 = load_b<O>(a, x, ipf + 1);
+    use_q<T>(a, x, i + 1, r, hN, huN, hvN);
+    const T bp2 = (T)sb;
+
+    T uN, vN;
+    lmask dryN;
+    prims_w<T>(hN, huN, hvN, bp2, cuse, w, uN, vN, dryN, odd);
+    // y faces of row i: lane computes its upper face (c, c+1)
+    const T bl = lane_get(ln.dn, b0), br = lane_get(ln.up, b0);
+    const T zy = w.hdy * ((T(0.5) * (br - bl)) * w.iy);
+    const T hR = lane_get(ln.up, hC), uR = lane_get(ln.up, uC), vR = lane_get(ln.up, vC);
+    const T zyR = lane_get(ln.up, zy);
+    const T zxN = w.hdx * ((T(0.5) * (bp2 - b0)) * w.ix);
+    FaceProd<T> fn, fy;
+    face_w<T>(b0, br, zy, zyR, hC, hR, vC, uC, vR, uR, dryC, lm_upper(dryC), yuse, w.iy, w, fy, odd);
+    const T lFh = lane_get(ln.dn, fy.Fh), lFN = lane_get(ln.dn, fy.FN), lFT = lane_get(ln.dn, fy.FT), lsR = lane_get(ln.dn, fy.sR);
+    face_w<T>(b0, bp1, zxC, zxN, hC, hN, uC, vC, uN, vN, dryC, dryN, act, w.ix, w, fn, odd);
+    T rh, rhu, rhv, rr0, n;
+    uint8_t fl;
+    sum_faces<T>(fn, fx, fy, lFh, lFN, lFT, lsR, rh, rhu, rhv);
+    cell_inputs<LEAN, T>(a, x, i, rh, rhu, rhv, rr0, n, fl);
+    if (MODE == 0) {
+      if (lm_any(odd)) return false;
+      if (x.col_ok) {
+        const int64_t idx = (int64_t)i * a.pitch + x.c;
+        a.rhs[0][idx] = rh;
+        a.rhs[1][idx] = rhu;
+        a.rhs[2][idx] = rhv;
+      }
+    } else {
+      T h, hu, hv, speed;
+      update_w<T>(hC, huC, hvC, rr0, rhu, rhv, n, act, a.P, w, h, hu, hv, speed, odd);
+      if (sizeof(O) == 8 && lm_any(odd)) return false;
+      bool quick = sizeof(S) == sizeof(T) && (w.flags & kWaveLam);
+      if (!LEAN && a.flags) {
+        const lmask stage = lm_of((fl & GS_FLAG_STAGE) != 0);
+        if (lm_any(stage)) {
+          quick = false;
+          const T hs = x.eta - b0;
+          h = lm_sel(stage, hs > T(0) ? hs : T(0), h);
+          hu = lm_sel(stage, T(0), hu);
+          hv = lm_sel(stage, T(0), hv);
+        }
+      }
+      // the stored values (one rounding each when S is narrower than T) are the state the
+      // running max and the next step's wave speed see
+      const S hS = (S)h, huS = (S)hu, hvS = (S)hv;
+      const lam_t<T> key = quick ? lam_key_w<T>(speed) : lam_key<T>((T)hS, (T)huS, (T)hvS, a.P);
+      if (sizeof(O) == 8) {
+        cell_store<LEAN, O>(a, x, i, hS, huS, hvS);
+        if (x.col_ok && (LEAN || !(fl & GS_FLAG_CFL_SKIP))) lam = key > lam ? key : lam;
+      } else {
+        // a row with an odd lane is left through the same stores, each lane's out of range, so
+        // that every way to the next row's loads holds the same stores
+        const bool left = lm_any(odd);
+        const uint32_t at = lane_st | (left ? kNoStore : 0u), row_st = (uint32_t)(i - i0) * pitch_st;
+        if (!LEAN && a.max_h && x.col_ok && !left) {
+          const int64_t idx = (int64_t)i * a.pitch + x.c;
+          if (hS > a.max_h[idx]) a.max_h[idx] = hS;
+        }
+        row_store(st0, at, row_st, hS);
+        row_store(st1, at, row_st, huS);
+        row_store(st2, at, row_st, hvS);
+        if (left) return false;
+        if (x.col_ok && (LEAN || !(fl & GS_FLAG_CFL_SKIP))) lam = key > lam ? key : lam;
+      }
+    }
+
+    // slide the window one row down
+    hC = hN; huC = huN; hvC = hvN; uC = uN; vC = vN; zxC = zxN; dryC = dryN;
+    b0 = bp1; bp1 = bp2;
+    fx = fn;
+    return true;
+  };
+  // two rows per trip, so that half of the window's moves are names instead
+  int i = i0;
+  while (i < i_end) {
+    if (!row(i)) break;
+    if (++i == i_end) break;
+    if (!row(i)) break;
+    ++i;
+  }
+  return i;
+}
+
+// The same rows by the general functions of gs_device.h, for every operand.
+template <typename T, int MODE, bool LEAN, typename S, typename O>
+__device__ __forceinline__ void dense_rows_general(const DenseK<T, S>& a, const DenseTile<T, S>& x, T dt, int i0,
+                                                   int i_end, lam_t<T>& lam) {
+  const Phys<T>& P = a.P;
+  const T ix = P.inv_dx, iy = P.inv_dy, hdx = P.half_dx, hdy = P.half_dy, g = P.g, hm = P.h_min;
+  const T bm2 = (T)load_b<O>(a, x, i0 - 2), bm1 = (T)load_b<O>(a, x, i0 - 1);
+  T b0 = (T)load_b<O>(a, x, i0), bp1 = (T)load_b<O>(a, x, i0 + 1);
+  RawRow<S> r;
+  T hP, huP, hvP, uP, vP, hC, huC, hvC, uC, vC;
+  load_q<O>(a, x, i0 - 1, r);
+  use_q<T>(a, x, i0 - 1, r, hP, huP, hvP);
+  prims(hP, huP, hvP, hm, uP, vP);
+  const T gzxP = (T(0.5) * (b0 - bm2)) * ix;
+  load_q<O>(a, x, i0, r);
+  use_q<T>(a, x, i0, r, hC, huC, hvC);
+  prims(hC, huC, hvC, hm, uC, vC);
+  T gzxC = (T(0.5) * (bp1 - bm1)) * ix;
+  FaceProd<T> fx;
+  face_prod<T>(bm1, b0, gzxP, gzxC, hP, hC, uP, vP, uC, vC, hdx, ix, g, hm, fx);
+  for (int i = i0; i < i_end; ++i) {
+    const T bp2 = (T)load_b<O>(a, x, i + 2);
+    T hN, huN, hvN, uN, vN;
+    load_q<O>(a, x, i + 1, r);
+    use_q<T>(a, x, i + 1, r, hN, huN, hvN);
+    prims(hN, huN, hvN, hm, uN, vN);
+    const T gzxN = (T(0.5) * (bp2 - b0)) * ix;
+    const T bl = lane_lower(b0), br = lane_upper(b0);
+    const T gzy = (T(0.5) * (br - bl)) * iy;
+    const T hR = lane_upper(hC), uR = lane_upper(uC), vR = lane_upper(vC);
+    const T gzyR = lane_upper(gzy);
+    FaceProd<T> fn, fy;
+    face_prod<T>(b0, bp1, gzxC, gzxN, hC, hN, uC, vC, uN, vN, hdx, ix, g, hm, fn);
+    face_prod<T>(b0, br, gzy, gzyR, hC, hR, vC, uC, vR, uR, hdy, iy, g, hm, fy);
+    const T lFh = lane_lower(fy.Fh), lFN = lane_lower(fy.FN), lFT = lane_lower(fy.FT), lsR = lane_lower(fy.sR);
+    T rh, rhu, rhv, rr0, n;
+    uint8_t fl;
+    sum_faces<T>(fn, fx, fy, lFh, lFN, lFT, lsR, rh, rhu, rhv);
+    cell_inputs<LEAN, T>(a, x, i, rh, rhu, rhv, rr0, n, fl);
+    if (MODE == 0) {
+      if (x.col_ok) {
+        const int64_t idx = (int64_t)i * a.pitch + x.c;
+        a.rhs[0][idx] = rh;
+        a.rhs[1][idx] = rhu;
+        a.rhs[2][idx] = rhv;
+      }
+    } else {
+      S hS = S(0), huS = S(0), hvS = S(0);
+      if (x.col_ok) {
+        T h, hu, hv;
+        update<T>(hC, huC, hvC, rr0, rhu, rhv, dt, n, P, h, hu, hv);
+        if (fl & GS_FLAG_STAGE) {
+          const T hs = x.eta - b0;
+          h = hs > T(0) ? hs : T(0);
+          hu = T(0);
+          hv = T(0);
+        }
+        hS = (S)h;
+        huS = (S)hu;
+        hvS = (S)hv;
+        if (!(fl & GS_FLAG_CFL_SKIP)) {
+          const lam_t<T> key = lam_key<T>((T)hS, (T)huS, (T)hvS, P);
+          lam = key > lam ? key : lam;
+        }
+      }
+      cell_store<LEAN, O>(a, x, i, hS, huS, hvS);
+    }
+    hC = hN; huC = huN; hvC = hvN; uC = uN; vC = vN; gzxC = gzxN;
+    b0 = bp1; bp1 = bp2;
+    fx = fn;
+  }
+}
+
+// MODE 0: residual into a.rhs; MODE 1: fused step. LEAN: see cell_inputs. O: byte offset of a column (row_at).
+template <typename T, int MODE, bool LEAN, typename S, typename O>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(LEAN && sizeof(T) == 4 ? 6 : 1)))
+void k_dense_sweep(DenseK<T, S> a) {
   int par = 0;
-  T dt = T(0), rain_u = T(0), eta = T(0);
+  T dt = T(0);
+  DenseTile<T, S> x;
+  x.rain = T(0);
+  x.eta = T(0);
   int ridx = 0;
   if (MODE == 1) {
     const GsClock* c = a.clock;
@@ -164,24 +510,34 @@ __global__ __launch_bounds__(kBlock) void k_dense_sweep(DenseK<T, S> a) {
     ridx = c->rain_idx;
     if (sizeof(T) == 4) {
       dt = (T)c->dt32;
-      rain_u = (T)c->rain32;
-      eta = (T)c->eta32;
+      x.rain = a.rain_mode == 1 ? (T)c->rain32 : T(0);
+      x.eta = (T)c->eta32;
     } else {
       dt = (T)c->dt;
-      rain_u = a.rain_mode == 1 ? (T)a.plan.rain_rate[ridx] : T(0);
-      eta = (T)c->eta64;
+      x.rain = a.rain_mode == 1 ? (T)a.plan.rain_rate[ridx] : T(0);
+      x.eta = (T)c->eta64;
     }
+  } else {
+    par = a.which;
   }
-  __shared__ T s_ntab[GS_MAX_CLASSES];
-  if (MODE == 1)
+  x.n0 = T(0);
+  x.ntab = nullptr;
+  if (LEAN) {
+    if (a.P.friction) x.n0 = (T)a.ntab[0];
+  } else if (MODE == 1) {
+    __shared__ T s_ntab[GS_MAX_CLASSES];
     for (int k = (int)threadIdx.x; k < a.n_classes; k += (int)blockDim.x) s_ntab[k] = (T)a.ntab[k];
-  __syncthreads();
+    __syncthreads();
+    x.ntab = s_ntab;
+  }
 
-  S* const* qin = MODE == 1 ? a.buf[par] : a.buf[a.which];
-  S* const* qout = a.buf[par ^ 1];
-  const Phys<T>& P = a.P;
-  const T ix = P.inv_dx, iy = P.inv_dy, hdx = P.half_dx, hdy = P.half_dy, g = P.g, hm = P.h_min;
-  const S* frame = (MODE == 1 && a.rain_mode == 2) ? a.rain_frames + (int64_t)ridx * a.frame_stride : nullptr;
+  // the buffers by value: an index into the argument's table at run time would put it in
+  // private memory
+  for (int k = 0; k < 3; ++k) {
+    x.qi[k] = par ? a.buf[1][k] : a.buf[0][k];
+    x.qo[k] = par ? a.buf[0][k] : a.buf[1][k];
+  }
+  x.frame = (MODE == 1 && a.rain_mode == 2) ? a.rain_frames + (int64_t)ridx * a.frame_stride : nullptr;
 
   // XCD-aware order: workgroups are dealt round-robin to the 8 XCDs; give each XCD a
   // contiguous range of tiles so neighbouring strips share that XCD's L2.
@@ -194,131 +550,29 @@ __global__ __launch_bounds__(kBlock) void k_dense_sweep(DenseK<T, S> a) {
   lam_t<T> lam = 0;
 
   if (tile < a.ntiles) {
-    const int rs = tile / a.ncs, cs = tile - rs * a.ncs;
-    const int c = cs * kOut + lane - 2;
-    const int cl = c < -2 ? -2 : (c > a.ny + 1 ? a.ny + 1 : c);   // loads stay within one ghost pair
-    const int i0 = rs * a.tile_rows;
-    const int i_end = min(i0 + a.tile_rows, a.nx);
-    const bool col_ok = (lane >= 2) && (lane < 2 + kOut) && (c < a.ny);
-
-    const ColMap cm = col_map(cl, a.ny, a.bc_y);
-    T bm2 = load_b(a, i0 - 2, cm), bm1 = load_b(a, i0 - 1, cm), b0 = load_b(a, i0, cm),
-      bp1 = load_b(a, i0 + 1, cm);
-    T hP, huP, hvP, uP, vP;
-    load_q(a, qin, i0 - 1, cm, hP, huP, hvP);
-    prims(hP, huP, hvP, hm, uP, vP);
-    const T gzxP = (T(0.5) * (b0 - bm2)) * ix;
-    T hC, huC, hvC, uC, vC;
-    load_q(a, qin, i0, cm, hC, huC, hvC);
-    prims(hC, huC, hvC, hm, uC, vC);
-    T gzxC = (T(0.5) * (bp1 - bm1)) * ix;
-    Face<T> fx;
-    face<T>(bm1, b0, gzxP, gzxC, hP, hC, uP, vP, uC, vC, hdx, g, hm, fx);
-    // the x-face below the current row, as the products the current cell adds (zero when
-    // the face is gated off: see the accumulation below)
-    const bool xg = fx.gate;
-    T xFh = xg ? fx.Fh * ix : T(0), xFN = xg ? fx.FN * ix : T(0), xFT = xg ? fx.FT * ix : T(0),
-      xsR = xg ? fx.srcR * ix : T(0);
-
-    for (int i = i0; i < i_end; ++i) {
-      const T bp2 = load_b(a, i + 2, cm);
-      T hN, huN, hvN, uN, vN;
-      load_q(a, qin, i + 1, cm, hN, huN, hvN);
-      prims(hN, huN, hvN, hm, uN, vN);
-      const T gzxN = (T(0.5) * (bp2 - b0)) * ix;
-      Face<T> fn;
-      face<T>(b0, bp1, gzxC, gzxN, hC, hN, uC, vC, uN, vN, hdx, g, hm, fn);
-      const bool ng = fn.gate;
-      const T nFh = ng ? fn.Fh * ix : T(0), nFN = ng ? fn.FN * ix : T(0), nFT = ng ? fn.FT * ix : T(0);
-      const T nsL = ng ? fn.srcL * ix : T(0), nsR = ng ? fn.srcR * ix : T(0);
-
-      // y faces of row i: lane computes its upper face (c, c+1)
-      const T bl = lane_lower(b0), br = lane_upper(b0);
-      const T gzy = (T(0.5) * (br - bl)) * iy;
-      const T hR = lane_upper(hC), uR = lane_upper(uC), vR = lane_upper(vC);
-      const T gzyR = lane_upper(gzy);
-      Face<T> fy;
-      face<T>(b0, br, gzy, gzyR, hC, hR, vC, uC, vR, uR, hdy, g, hm, fy);
-      const bool yg = fy.gate;
-      const T yFh = yg ? fy.Fh * iy : T(0), yFN = yg ? fy.FN * iy : T(0), yFT = yg ? fy.FT * iy : T(0);
-      const T ysL = yg ? fy.srcL * iy : T(0);
-      const T yFhB = lane_lower(yFh), yFNB = lane_lower(yFN), yFTB = lane_lower(yFT);
-      const T ysRB = lane_lower(yg ? fy.srcR * iy : T(0));
-
-      // The four faces in the reference's order. A face gated off (both cells dry) adds
-      // zeros: the sums start at +0 and IEEE addition yields -0 only from two -0 terms, so
-      // they never hold -0, and x + 0 = x - 0 = x for every other x; the gate costs one
-      // select per face term instead of one per use.
-      T rh = T(0), rhu = T(0), rhv = T(0);
-      rh = rh - nFh;
-      rhu = rhu - nFN;
-      rhv = rhv - nFT;
-      rhu = rhu - nsL;
-      rh = rh + xFh;
-      rhu = rhu + xFN;
-      rhv = rhv + xFT;
-      rhu = rhu + xsR;
-      rh = rh - yFh;
-      rhu = rhu - yFT;
-      rhv = rhv - yFN;
-      rhv = rhv - ysL;
-      rh = rh + yFhB;
-      rhu = rhu + yFTB;
-      rhv = rhv + yFNB;
-      rhv = rhv + ysRB;
-
-      if (col_ok) {
-        const int64_t idx = (int64_t)i * a.pitch + c;
-        const uint8_t fl = a.flags ? a.flags[idx] : (uint8_t)0;
-        const bool inactive = (fl & GS_FLAG_INACTIVE) != 0;
-        if (inactive) { rh = T(0); rhu = T(0); rhv = T(0); }
-        if (MODE == 0) {
-          a.rhs[0][idx] = rh;
-          a.rhs[1][idx] = rhu;
-          a.rhs[2][idx] = rhv;
-        } else {
-          T rr0 = rh;
-          if (!inactive) {
-            if (a.rain_mode == 1) rr0 = rr0 + rain_u;
-            else if (a.rain_mode == 2) rr0 = rr0 + (T)frame[(int64_t)i * a.rain_pitch + c];
-          }
-          T n = T(0);
-          if (P.friction)
-            n = a.n_field ? (T)a.n_field[idx] : s_ntab[a.cls ? a.cls[idx] : (fl & GS_FLAG_CLASS_MASK)];
-          T h, hu, hv;
-          update<T>(hC, huC, hvC, rr0, rhu, rhv, dt, n, P, h, hu, hv);
-          if (fl & GS_FLAG_STAGE) {
-            const T hs = eta - b0;
-            h = hs > T(0) ? hs : T(0);
-            hu = T(0);
-            hv = T(0);
-          }
-          // the stored values (one rounding each when S is narrower than T) are the state the
-          // running max and the next step's wave speed see
-          const S hS = (S)h, huS = (S)hu, hvS = (S)hv;
-          if (a.max_h && hS > a.max_h[idx]) a.max_h[idx] = hS;
-          qout[0][idx] = hS;
-          qout[1][idx] = huS;
-          qout[2][idx] = hvS;
-          if (!(fl & GS_FLAG_CFL_SKIP)) {
-            const lam_t<T> lb_ = lam_key<T>((T)hS, (T)huS, (T)hvS, P);
-            lam = lb_ > lam ? lb_ : lam;
-          }
-        }
-      }
-
-      // slide the window one row down
-      hC = hN; huC = huN; hvC = hvN; uC = uN; vC = vN; gzxC = gzxN;
-      bm1 = b0; b0 = bp1; bp1 = bp2;
-      xFh = nFh; xFN = nFN; xFT = nFT; xsR = nsR;
+    const int rs = __builtin_amdgcn_readfirstlane(tile / a.ncs), cs = tile - rs * a.ncs;
+    x.c = cs * kOut + lane - 2;
+    const int cl = x.c < -2 ? -2 : (x.c > a.ny + 1 ? a.ny + 1 : x.c);   // loads stay within one ghost pair
+    int i = rs * a.tile_rows;
+    const int i_end = min(i + a.tile_rows, a.nx);
+    x.col_ok = (lane >= 2) && (lane < 2 + kOut) && (x.c < a.ny);
+    x.edge = cs == 0 || (cs + 1) * kOut + 2 > a.ny || i < 2 || i_end + 2 > a.nx;
+    x.cm = col_map(cl, a.ny, a.bc_y);
+    if (a.wave & kWaveFast) {
+      const WaveC<T> w = wave_consts<T>(a.P, dt, a.wave);
+      DenseTile<T, S> xv = x;
+      xv.rain = vreg(x.rain);
+      xv.n0 = vreg(x.n0);
+      i = __builtin_amdgcn_readfirstlane(dense_rows<T, MODE, LEAN, S, O>(a, xv, w, i, i_end, lam));
     }
+    if (i < i_end) dense_rows_general<T, MODE, LEAN, S, O>(a, x, dt, i, i_end, lam);
   }
   if (MODE == 1) grid_reduce_and_plan(lam_key_bits64(lam), a.clock, a.plan, true);
 }
 
 // CFL wave speed of the current dense state, then plan dt (no time advance).
 template <typename T, typename S = T>
-__global__ __launch_bounds__(kBlock) void k_dense_cfl(DenseK<T, S> a) {
+__global__ __launch_bounds__(256) void k_dense_cfl(DenseK<T, S> a) {
   const int par = (int)(a.clock->nsteps & 1);
   S* const* q = a.buf[par];
   lam_t<T> lam = 0;
@@ -387,6 +641,7 @@ static int build_dense(const GsDense* d, const GsPhys* p, const GsForcing& f, Gs
   a.cls = d->cls;
   a.max_h = (S*)d->max_h;
   a.P = make_phys<T>(*p, d->dx, d->dy);
+  a.wave = wave_flags<T>(a.P, false);
   a.rain_mode = f.n_rain > 0 ? (f.rain_gridded ? 2 : 1) : 0;
   a.rain_frames = (const S*)f.rain_frames;
   a.frame_stride = f.rain_frame_stride;
@@ -397,13 +652,22 @@ static int build_dense(const GsDense* d, const GsPhys* p, const GsForcing& f, Gs
   return GS_OK;
 }
 
+// Tiles of 2 GiB or more (per plane) take the sweep with 64-bit offsets.
+template <typename T, typename S>
+static bool wide_rows(const DenseK<T, S>& a) {
+  return a.pitch * (int64_t)sizeof(S) >= ((int64_t)1 << 31) / a.tile_rows;
+}
+
 template <typename T, typename S = T>
 static int dense_step_t(const GsDense* d, const GsPhys* p, GsForcing f, GsClock* clk, hipStream_t s) {
   DenseK<T, S> a;
   int rc = build_dense<T, S>(d, p, f, clk, a, true);
   if (rc) return rc;
-  const unsigned blocks = (unsigned)((a.ntiles + 3) / 4);
-  hipLaunchKernelGGL((k_dense_sweep<T, 1, S>), dim3(blocks), dim3(kBlock), 0, s, a);
+  const dim3 grid((unsigned)((a.ntiles + 3) / 4)), block(kBlock);
+  const bool lean = !a.flags && !a.n_field && !a.cls && !a.max_h && a.rain_mode != 2;
+  if (wide_rows(a)) hipLaunchKernelGGL((k_dense_sweep<T, 1, false, S, uint64_t>), grid, block, 0, s, a);
+  else if (lean) hipLaunchKernelGGL((k_dense_sweep<T, 1, true, S, uint32_t>), grid, block, 0, s, a);
+  else hipLaunchKernelGGL((k_dense_sweep<T, 1, false, S, uint32_t>), grid, block, 0, s, a);
   GS_HIP(hipGetLastError(), "k_dense_sweep launch");
   return GS_OK;
 }
@@ -423,8 +687,9 @@ static int dense_residual_t(const GsDense* d, const GsPhys* p, int which, void* 
   a.rhs[1] = (T*)r1;
   a.rhs[2] = (T*)r2;
   // MODE 0 writes qout = buf[which ^ 1] never; buf[par ^ 1] is unused there
-  const unsigned blocks = (unsigned)((a.ntiles + 3) / 4);
-  hipLaunchKernelGGL((k_dense_sweep<T, 0, S>), dim3(blocks), dim3(kBlock), 0, s, a);
+  const dim3 grid((unsigned)((a.ntiles + 3) / 4)), block(kBlock);
+  if (wide_rows(a)) hipLaunchKernelGGL((k_dense_sweep<T, 0, false, S, uint64_t>), grid, block, 0, s, a);
+  else hipLaunchKernelGGL((k_dense_sweep<T, 0, false, S, uint32_t>), grid, block, 0, s, a);
   GS_HIP(hipGetLastError(), "k_dense_sweep(residual) launch");
   return GS_OK;
 }
@@ -435,9 +700,9 @@ static int dense_cfl_t(const GsDense* d, const GsPhys* p, GsForcing f, GsClock* 
   int rc = build_dense<T, S>(d, p, f, clk, a, true);
   if (rc) return rc;
   const int64_t n = (int64_t)a.nx * a.ny;
-  int64_t blocks = (n + kBlock - 1) / kBlock;
+  int64_t blocks = (n + 255) / 256;
   if (blocks > 4096) blocks = 4096;
-  hipLaunchKernelGGL((k_dense_cfl<T, S>), dim3((unsigned)blocks), dim3(kBlock), 0, s, a);
+  hipLaunchKernelGGL((k_dense_cfl<T, S>), dim3((unsigned)blocks), dim3(256), 0, s, a);
   GS_HIP(hipGetLastError(), "k_dense_cfl launch");
   return GS_OK;
 }

@@ -2,6 +2,7 @@
 // fractional-Brownian-motion bed generator used by the synthetic benchmark cases, and a
 // plain streaming copy used to calibrate HBM bandwidth and traffic counters.
 #include "gs_common.h"
+#include "gs_wave.h"
 
 namespace gs {
 
@@ -152,7 +153,8 @@ __global__ __launch_bounds__(256) void k_valu(float* out, int iters, float m, fl
 // CASE 0: 1/b for every b; 1: sqrt(x) for every x (the guarded form), and the short form for
 // every x with |x| outside (0, 2^-96); 2: a/b for 2^32 pairs of seeded bit patterns (every exponent);
 // 3: a/b for every a over four divisors with the hardest significands (all ones, 1 + ulp,
-// 1 - ulp/2, 3). counts[2*k] = mismatches of check k, counts[2*k + 1] = 1 + the largest
+// 1 - ulp/2, 3); 4: the wavefront forms of gs_wave.h: the root for every x >= 2^-96 and 0, and
+// the quotient for 2^32 seeded pairs within its bounds. counts[2*k] = mismatches of check k, counts[2*k + 1] = 1 + the largest
 // offending index (0: none).
 __device__ __forceinline__ bool cr_same(float a, float b) {
   return (a != a && b != b) || __float_as_uint(a) == __float_as_uint(b);
@@ -178,6 +180,17 @@ __global__ __launch_bounds__(256) void k_crmath_check(unsigned long long* counts
       const float a = __uint_as_float(cr_hash(i, 0x2545F491u));
       const float b = __uint_as_float(cr_hash(i, 0x9E3779B9u));
       if (!cr_same(div_cr(a, b), a / b)) { bad0++; last0 = i + 1; }
+    } else if (CASE == 4) {
+      const float x = __uint_as_float((uint32_t)i);
+      if (i == 0 || (x >= 0x1p-96f && x < __builtin_inff()))
+        if (!cr_same(root0_w(x), __builtin_sqrtf(x))) { bad0++; last0 = i + 1; }
+      // numerators 0 or 2^-100 .. 2^28, denominators 2^-21 .. 2^25: the quotient is normal
+      const uint32_t ha = cr_hash(i, 0x2545F491u), hb = cr_hash(i, 0x9E3779B9u);
+      const float a = __uint_as_float((ha & 0x807FFFFFu) | ((27u + ((ha >> 23) & 0xFFu) % 128u) << 23));
+      const uint32_t sign = (i & 0xFFFFu) ? 0x80000000u : 0u;   // zeros over positive denominators
+      const float b = __uint_as_float((hb & (sign | 0x7FFFFFu)) | ((106u + ((hb >> 23) & 63u) % 46u) << 23));
+      const float n = (i & 0xFFFFu) ? a : (ha & 1u ? 0.0f : -0.0f);
+      if (!cr_same(quot_w(n, b, recip_w(b)), n / b)) { bad1++; last1 = i + 1; }
     } else {
       const uint32_t dv[4] = {0x3FFFFFFFu, 0x3F800001u, 0x3F7FFFFFu, 0x40400000u};
       const float a = __uint_as_float((uint32_t)i);
@@ -258,13 +271,14 @@ int gs_bench_valu(float* out, int blocks, int iters, int mode, void* stream) {
 }
 
 int gs_crmath_check(int which, unsigned long long* counts_dev, void* stream) {
-  if (!counts_dev || which < 0 || which > 3) return fail(GS_E_ARG, "gs_crmath_check: counts and which in 0..3 required");
+  if (!counts_dev || which < 0 || which > 4) return fail(GS_E_ARG, "gs_crmath_check: counts and which in 0..4 required");
   hipStream_t s = (hipStream_t)stream;
   const dim3 g(8192), b(256);
   switch (which) {
     case 0: hipLaunchKernelGGL(k_crmath_check<0>, g, b, 0, s, counts_dev); break;
     case 1: hipLaunchKernelGGL(k_crmath_check<1>, g, b, 0, s, counts_dev); break;
     case 2: hipLaunchKernelGGL(k_crmath_check<2>, g, b, 0, s, counts_dev); break;
+    case 4: hipLaunchKernelGGL(k_crmath_check<4>, g, b, 0, s, counts_dev); break;
     default: hipLaunchKernelGGL(k_crmath_check<3>, g, b, 0, s, counts_dev); break;
   }
   GS_HIP(hipGetLastError(), "k_crmath_check launch");
