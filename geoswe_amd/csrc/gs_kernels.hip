@@ -73,7 +73,8 @@ __global__ void k_clock_dt(GsClock* c, Plan p, double dt) {
 // dense layout
 // ---------------------------------------------------------------------------
 constexpr int kOut = 60;      // columns written per strip (lanes 2..61)
-constexpr int kBlock = 256;   // 4 strips per workgroup
+constexpr int kMaxWaves = 8;  // most strips per workgroup
+constexpr int kBlock = 64 * kMaxWaves;
 
 // T is the arithmetic type, S the type of the planes in memory (S = float with T = double:
 // float32 planes stepped with float64 arithmetic, each value rounded once when it is stored).
@@ -546,7 +547,7 @@ void k_dense_sweep(DenseK<T, S> a) {
   const unsigned lb = (xcd < rm) ? xcd * (qd + 1u) + kk : rm * (qd + 1u) + (xcd - rm) * qd + kk;
   const int lane = threadIdx.x & 63;
   // the wavefront index as a scalar: tile, rows and row addresses are then uniform values
-  const int tile = (int)(lb * 4u) + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int tile = (int)(lb * (blockDim.x >> 6)) + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   lam_t<T> lam = 0;
 
   if (tile < a.ntiles) {
@@ -588,18 +589,30 @@ __global__ __launch_bounds__(256) void k_dense_cfl(DenseK<T, S> a) {
   grid_reduce_and_plan(lam_key_bits64(lam), a.clock, a.plan, false);
 }
 
-// Rows per strip: 64 when that still gives 8192 strips, else fewer. On the 640 M-cell grid
-// 64-row strips (167 K wavefronts) ran the step in 7.93 ms against 8.11 ms for 128 rows
-// and 8.30 ms for 256 (the extra halo rows of shorter strips cost less than the better
-// balance of more wavefronts gains); 32 rows took 8.00 ms.
-static int pick_tile_rows(int nx, int ncs, int req) {
+// Rows per tile. A tile costs about 1.3 rows beside its own (the rows above it, the first x-face),
+// so tall tiles do the least work; but a wavefront takes about 1.4 us per row by itself, so a grid
+// that does not fill the GPU several times over wants short ones, and as many wavefronts as there
+// are SIMDs. Measured best heights (float32): 1 row on 128^2 and 256^2, 3 on 500 x 517, 5 on
+// 1024^2, 6-12 on 2000^2, 16 on 4096^2, 24-32 on 8192 x 8000, 32-64 on 640 M cells; float64 within
+// 4 % of its best at the same heights. 1.5 (cells/65536)^0.4 follows them. (With at least 16 rows
+// always, 500 x 517 took 30 us a step against 13.2, 1024^2 33 us against 21.) The bands are then
+// made even.
+static int pick_tile_rows(int nx, int ny, int req) {
   if (req > 0) return req;
-  const int cand[3] = {64, 32, 16};
-  for (int k = 0; k < 3; ++k) {
-    const int64_t nrs = (nx + cand[k] - 1) / cand[k];
-    if ((int64_t)ncs * nrs >= 8192) return cand[k];
-  }
-  return 16;
+  const double cells = (double)nx * (double)ny;
+  int rows = (int)(1.5 * pow(cells / 65536.0, 0.4) + 0.5);
+  rows = rows < 1 ? 1 : (rows > 64 ? 64 : rows);
+  const int bands = (nx + rows - 1) / rows;
+  return (nx + bands - 1) / bands;
+}
+
+// Wavefronts per workgroup: 8 for the short tiles of small float32 grids, else 4. Each workgroup
+// makes two atomics on the clock's line, which the line takes one after the other (5.8 ns each):
+// 1024^2 in 5-row tiles 21.0 us with 8 against 25.1 us with 4. Grids of more tiles hide them, and
+// a workgroup of 4 fills the last free wavefront slots better (8192 x 8000: 577 against 592 us);
+// so do the 12 resident wavefronts of a float64 CU.
+static int tile_waves(int ntiles, size_t arith) {
+  return arith == 4 && ntiles < 16384 ? kMaxWaves : 4;
 }
 
 template <typename T, typename S = T>
@@ -627,7 +640,7 @@ static int build_dense(const GsDense* d, const GsPhys* p, const GsForcing& f, Gs
   a.bc_y = d->bc_y;
   a.pitch = d->pitch;
   a.ncs = (d->ny + kOut - 1) / kOut;
-  a.tile_rows = pick_tile_rows(d->nx, a.ncs, d->tile_rows);
+  a.tile_rows = pick_tile_rows(d->nx, d->ny, d->tile_rows);
   a.nrs = (d->nx + a.tile_rows - 1) / a.tile_rows;
   if ((int64_t)a.ncs * a.nrs > (int64_t)INT32_MAX / 2) return fail(GS_E_RANGE, "too many tiles");
   a.ntiles = a.ncs * a.nrs;
@@ -663,7 +676,8 @@ static int dense_step_t(const GsDense* d, const GsPhys* p, GsForcing f, GsClock*
   DenseK<T, S> a;
   int rc = build_dense<T, S>(d, p, f, clk, a, true);
   if (rc) return rc;
-  const dim3 grid((unsigned)((a.ntiles + 3) / 4)), block(kBlock);
+  const int waves = tile_waves(a.ntiles, sizeof(T));
+  const dim3 grid((unsigned)((a.ntiles + waves - 1) / waves)), block(64 * waves);
   const bool lean = !a.flags && !a.n_field && !a.cls && !a.max_h && a.rain_mode != 2;
   if (wide_rows(a)) hipLaunchKernelGGL((k_dense_sweep<T, 1, false, S, uint64_t>), grid, block, 0, s, a);
   else if (lean) hipLaunchKernelGGL((k_dense_sweep<T, 1, true, S, uint32_t>), grid, block, 0, s, a);
@@ -687,7 +701,8 @@ static int dense_residual_t(const GsDense* d, const GsPhys* p, int which, void* 
   a.rhs[1] = (T*)r1;
   a.rhs[2] = (T*)r2;
   // MODE 0 writes qout = buf[which ^ 1] never; buf[par ^ 1] is unused there
-  const dim3 grid((unsigned)((a.ntiles + 3) / 4)), block(kBlock);
+  const int waves = tile_waves(a.ntiles, sizeof(T));
+  const dim3 grid((unsigned)((a.ntiles + waves - 1) / waves)), block(64 * waves);
   if (wide_rows(a)) hipLaunchKernelGGL((k_dense_sweep<T, 0, false, S, uint64_t>), grid, block, 0, s, a);
   else hipLaunchKernelGGL((k_dense_sweep<T, 0, false, S, uint32_t>), grid, block, 0, s, a);
   GS_HIP(hipGetLastError(), "k_dense_sweep(residual) launch");
