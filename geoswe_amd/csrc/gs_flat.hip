@@ -19,11 +19,20 @@
 #include <vector>
 
 #include "gs_common.h"
+#include "gs_wave.h"
 
 namespace gs {
 
 constexpr int kFOut = 60;     // flat ids written per wavefront (lanes 2..61)
 constexpr int kFBlock = 256;
+// Wavefronts (tiles in flight) per workgroup of a sweep. Each workgroup ends with two atomics on
+// the clock's cache line, which serialize at about 6 ns each: eight wavefronts halve them (2048^2
+// coastal domain, 6-row tiles: 43.1 against 44.5 us per step; 2-row tiles: 57.7 against 81 us). Float64
+// sweeps fit three wavefronts per SIMD, which workgroups of eight would leave at two.
+template <typename T>
+constexpr int kSweepWaves = sizeof(T) == 4 ? 8 : 4;
+template <typename T>
+constexpr int kSBlock = 64 * kSweepWaves<T>;
 
 template <typename T>
 struct FlatK {
@@ -47,6 +56,7 @@ struct FlatK {
   const int32_t* run_d;
   const int32_t* chunk_run;
   Phys<T> P;
+  int wave;         // kWave* flags of P; 0 too where a tile's rows may span 2 GiB
   int rain_mode;
   const T* rain_frames;
   int64_t frame_stride, rain_pitch;
@@ -85,13 +95,30 @@ struct FlatK {
 };
 
 
+// What a wavefront reads whole by scalar loads: the mesh tables (tiles and their rows) and the
+// descriptor itself. No kernel that reads them writes them.
+#define GS_C __attribute__((address_space(4)))
+template <typename P>
+__device__ __forceinline__ const GS_C P* cp(const GS_G P* p) {
+  return (const GS_C P*)(uint64_t)p;
+}
+
+// Read a value that the launch never writes through the constant address space: a
+// uniform address then gives scalar loads. The host pass sees an ordinary read.
+template <typename U>
+__device__ __forceinline__ U const_read(const U* p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return *(const __attribute__((address_space(4))) U*)p;
+#else
+  return *p;
+#endif
+}
+
 // Everything one chunk pass reads, as values: the state buffers picked for this step (a
 // runtime index into the argument's buffer table would put the table in private memory and
 // every state access behind a generic pointer), the mesh arrays, the clock's per-step
 // values and the physics scalars. Filled from the kernel argument (plain step) or from
 // the member table (ensemble).
-#define GS_G __attribute__((address_space(1)))
-
 template <typename T>
 struct FlatCtx {
   const GS_G T* qi0;
@@ -134,8 +161,9 @@ struct FlatCtx {
   const GS_G int32_t* rain_lookup;
   const GS_G T* frame;   // gridded rain frame of this step (rain_mode 2)
   const T* ntab;         // Manning n per class (LDS copy or the member's table)
+  const GS_C FlatK<T>* k;   // the descriptor itself, for cold()
   int64_t n, rain_pitch;
-  int n_runs, ngh, rain_mode;
+  int n_runs, ngh, rain_mode, wave;
   T dt, rain_u, eta;
   Phys<T> P;
 };
@@ -172,16 +200,17 @@ __device__ __forceinline__ FlatClk<T> flat_clock(const FlatK<T>& a) {
       k.live = false;
       return k;
     }
-    k.par = (int)(c->nsteps & 1);
-    const int ridx = c->rain_idx;
+    // uniform values, in scalar registers
+    k.par = __builtin_amdgcn_readfirstlane((int)(c->nsteps & 1));
+    const int ridx = __builtin_amdgcn_readfirstlane(c->rain_idx);
     if (sizeof(T) == 4) {
-      k.dt = (T)c->dt32;
-      k.rain_u = (T)c->rain32;
-      k.eta = (T)c->eta32;
+      k.dt = sreg((T)c->dt32);
+      k.rain_u = sreg((T)c->rain32);
+      k.eta = sreg((T)c->eta32);
     } else {
-      k.dt = (T)c->dt;
-      k.rain_u = a.rain_mode == 1 ? (T)gp(a.plan.rain_rate)[ridx] : T(0);
-      k.eta = (T)c->eta64;
+      k.dt = sreg((T)c->dt);
+      k.rain_u = a.rain_mode == 1 ? sreg((T)gp(a.plan.rain_rate)[ridx]) : T(0);
+      k.eta = sreg((T)c->eta64);
     }
     if (a.rain_mode >= 2) k.frame = gp(a.rain_frames) + (int64_t)ridx * a.frame_stride;
   }
@@ -238,10 +267,56 @@ __device__ __forceinline__ void flat_ctx(const FlatK<T>& a, const FlatClk<T>& k,
   x.n_runs = a.n_runs;
   x.ngh = a.ngh;
   x.rain_mode = a.rain_mode;
+  x.wave = a.wave;
   x.dt = k.dt;
   x.rain_u = k.rain_u;
   x.eta = k.eta;
   x.P = a.P;
+}
+
+// The context with the pointers and physics scalars that a row needs seldom or late read from the
+// descriptor again (scalar loads that hit the scalar cache; a caller pays for what it uses). Held
+// through the row loop they were spilled to vector lanes, 450 lane reads for each two rows of the
+// extended sweep.
+template <typename T>
+__device__ __forceinline__ const GS_C FlatK<T>* cold_ptr(const GS_C FlatK<T>* k) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("" : "+s"(k));
+#endif
+  return k;
+}
+template <typename T>
+__device__ __forceinline__ FlatCtx<T> cold(const FlatCtx<T>& x) {
+  const GS_C FlatK<T>* k = cold_ptr<T>(x.k);
+  FlatCtx<T> y = x;
+  y.n_field = gp((T*)k->n_field);
+  y.cls = gp((uint8_t*)k->cls);
+  y.max_h = gp((T*)k->max_h);
+  y.pre0 = gp((T*)k->pre[0]);
+  y.pre1 = gp((T*)k->pre[1]);
+  y.pre2 = gp((T*)k->pre[2]);
+  y.sponge = gp((T*)k->sponge);
+  y.clamp = gp((T*)k->clamp);
+  y.infil = gp((T*)k->infil);
+  y.drain = gp((T*)k->drain);
+  y.ga_cls = gp((uint8_t*)k->ga_cls);
+  y.ga_ks = gp((T*)k->ga_ks);
+  y.ga_psi = gp((T*)k->ga_psi);
+  y.ga_dth = gp((T*)k->ga_dth);
+  y.ga_F = gp((T*)k->ga_F);
+  y.ga_fmax = gp((T*)k->ga_fmax);
+  y.ga_inv_tau = gp((T*)k->ga_inv_tau);
+  y.rain_lookup = gp((int32_t*)k->rain_lookup);
+  y.P = const_read((const Phys<T>*)(uint64_t)&k->P);
+  return y;
+}
+template <typename T>
+__device__ __forceinline__ const GS_C FlatK<T>* kernel_arg() {   // a kernel whose first argument is a FlatK<T>
+#if defined(__HIP_DEVICE_COMPILE__)
+  return (const GS_C FlatK<T>*)__builtin_amdgcn_kernarg_segment_ptr();
+#else
+  return nullptr;
+#endif
 }
 
 // One wavefront pass over flat ids chunk*60-2 .. chunk*60+61: the residual (MODE 0) or the
@@ -526,7 +601,7 @@ __device__ __forceinline__ void flat_chunk(const FlatCtx<T>& x, int64_t chunk, i
 // is the row's first id (uniform across the wavefront) plus the number of stored lanes below
 // it. The byte offset of that count is returned; accesses add it to the row's start.
 template <typename T>
-__device__ __forceinline__ uint32_t sweep_lane(const GS_G uint64_t* e, int lane, int64_t& base, bool& st) {
+__device__ __forceinline__ uint32_t sweep_lane(const GS_C uint64_t* e, int lane, int64_t& base, bool& st) {
   const uint64_t sm = e[1];
   base = (int64_t)e[0];
   const unsigned below =
@@ -557,31 +632,224 @@ __device__ __forceinline__ T sweep_b(const FlatCtx<T>& x, int64_t base, uint32_t
   return b;
 }
 
-// One row-sweep tile: the fused update of the active lanes of rows i0 .. i0+nr-1 of one
-// 64-column window. As in the dense sweep, every face is evaluated once: the x-face below
-// a row is carried from the row above, the y-face below a lane comes from the lane below
-// by shuffle, and the residual terms are added in the same order as there (and as in
-// flat_chunk), so all three traversals give the same bits. Every lane of the wavefront
-// must call it. PRE: also write the pre-friction state (the adjoint's recomputation); a
-// separate instantiation keeps those pointers out of the plain step's scalar registers.
-// LEAN: the domain has no per-cell Manning field or class plane, no running maximum and no
-// active-cell forcing, so none of their pointers is held (the host checks that they are all
-// null).
-template <typename T, bool PRE, bool EXT, bool LEAN = false>
-__device__ __forceinline__ void flat_tile(const FlatCtx<T>& x, int64_t t, int lane, lam_t<T>& lam) {
+// The cell of an active lane after its update, in the reference's order: the stage, the running
+// max and the forcings (what LEAN leaves out is not there).
+template <typename T, bool EXT, bool LEAN>
+__device__ __forceinline__ void finish_cell(const FlatCtx<T>& x, uint8_t fg, int64_t base, uint32_t off, T b, T& h,
+                                            T& hu, T& hv) {
+  if (fg & GS_FLAG_STAGE) {
+    const T hs = x.eta - b;
+    h = hs > T(0) ? hs : T(0);
+    hu = T(0);
+    hv = T(0);
+  }
+  if (!LEAN) {
+    if (x.max_h && h > gat(x.max_h + base, off)) gat(x.max_h + base, off) = h;
+    active_force<T, EXT>(x, fg, base, off, off / (uint32_t)sizeof(T), h, hu, hv);
+  }
+}
+
+// The tallest tile that flat_rows takes: its rows are addressed with 32-bit offsets.
+constexpr int kWaveRows = 1024;
+
+// One row of a sweep tile.
+struct FlatRow {
+  uint32_t row;        // its first stored id, from the tile's first one (uniform)
+  uint64_t st, act;    // stored and active lanes
+  uint32_t below;      // stored lanes below this one: with `row` the lane's id where it is stored
+};
+__device__ __forceinline__ FlatRow flat_row(const GS_C uint64_t* e, uint32_t g0) {
+  FlatRow r;
+  r.row = (uint32_t)e[0] - g0;
+  r.st = e[1];
+  r.act = e[2];
+  r.below = __builtin_amdgcn_mbcnt_hi((unsigned)(r.st >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)r.st, 0u));
+  return r;
+}
+
+// Rows 0 .. nr-1 of a tile by the wavefront forms (gs_wave.h): every face is evaluated once, the
+// x-face below a row is carried from the row above, the y-face below a lane comes from the lane
+// below by shuffle, and the residual terms are added in the dense sweep's order, so all traversals
+// give the same bits. Returns the first row that it leaves to flat_rows_general (one that holds
+// an operand outside their bounds, before anything of it is written), nr where there is none.
+// A row's state, flags and rain are loaded one row ahead of their use, its bed two rows ahead and
+// its entry before that. Lanes on unstored cells read 0: no face that an active cell uses reads
+// them.
+template <typename T, bool PRE, bool EXT, bool LEAN>
+__device__ __forceinline__ int flat_rows(const FlatCtx<T>& x, const WaveC<T>& w, const GS_C uint64_t* E, int i0, int nr,
+                                         int c0, int lane, lam_t<T>& lam) {
+  constexpr uint32_t es = (uint32_t)sizeof(T);
+  lmask odd = 0;
+  lam_t<T> top = 0;   // the tile's own maximum: what the caller holds need not stay in a register
+  const Lanes ln = lanes_of(lane);
+  const int64_t g0 = (int64_t)E[0];   // ids of a tile's rows ascend
+  const uint32_t g0l = (uint32_t)g0;
+  const RowBuf qi0 = row_buf(x.qi0 + g0), qi1 = row_buf(x.qi1 + g0), qi2 = row_buf(x.qi2 + g0),
+               bed = row_buf(x.bed + g0), qo0 = row_buf(x.qo0 + g0), qo1 = row_buf(x.qo1 + g0),
+               qo2 = row_buf(x.qo2 + g0);
+  // flags and gridded rain are read as 0 where there are none, without a branch
+  const bool gridded = x.rain_mode == 2;
+  const lmask flagged = x.flags ? lm_every() : lm_none(), rained = gridded ? lm_every() : lm_none();
+  const RowBuf flg = row_buf(x.flags + g0);
+  const RowBuf rnb = row_buf(x.frame + (int64_t)(i0 - x.ngh) * x.rain_pitch + (c0 - x.ngh) - 1);   // from lane -1
+  const T rain = vreg(x.rain_mode == 1 ? x.rain_u : T(0));
+  const uint32_t rain_row = (uint32_t)x.rain_pitch * es;
+  auto load_q = [&](const FlatRow& r, T& h, T& hu, T& hv) __attribute__((always_inline)) {
+    const uint32_t off = lm_lane(r.st) ? r.below * es : kNoLane;
+    row_load(qi0, off, r.row * es, h);
+    row_load(qi1, off, r.row * es, hu);
+    row_load(qi2, off, r.row * es, hv);
+  };
+  auto load_b = [&](const FlatRow& r, T& b) __attribute__((always_inline)) {
+    row_load(bed, lm_lane(r.st) ? r.below * es : kNoLane, r.row * es, b);
+  };
+  // a row's flags and rain, on its active lanes
+  auto load_c = [&](const FlatRow& r, int k, uint8_t& fg, T& rn) __attribute__((always_inline)) {
+    row_load(flg, lm_lane(r.act & flagged) ? r.below : kNoLane, r.row, fg);
+    row_load(rnb, lm_lane(r.act & rained) ? (uint32_t)ln.up * (es / 4u) : kNoLane, (uint32_t)k * rain_row, rn);
+  };
+
+  T b0, bp1, hC, huC, hvC, uC, vC, zxC;
+  T sh, shu, shv, sb, srn;   // loaded ahead: the next row's state and rain, the bed of the one after it
+  uint8_t sfl;               // and the next row's flags
+  lmask dryC;
+  FaceProd<T> fx;            // the x-face below the current row
+  FlatRow eC = flat_row(E + 6, g0l), eN = flat_row(E + 9, g0l), eF = flat_row(E + 12, g0l);
+  {
+    const FlatRow e0 = flat_row(E, g0l), e1 = flat_row(E + 3, g0l);
+    T bm2, bm1, hP, huP, hvP, uP, vP;
+    load_b(e0, bm2);
+    load_b(e1, bm1);
+    load_b(eC, b0);
+    load_b(eN, bp1);
+    load_q(e1, hP, huP, hvP);
+    load_q(eC, hC, huC, hvC);
+    load_q(eN, sh, shu, shv);
+    load_b(eF, sb);
+    load_c(eC, 0, sfl, srn);
+    lmask dryP;
+    prims_w<T>(hP, huP, hvP, vabs(bm2) + vabs(bm1), e1.st, w, uP, vP, dryP, odd);
+    prims_w<T>(hC, huC, hvC, vabs(b0) + vabs(bp1), eC.st, w, uC, vC, dryC, odd);
+    const T zxP = w.hdx * ((T(0.5) * (b0 - bm2)) * w.ix);
+    zxC = w.hdx * ((T(0.5) * (bp1 - bm1)) * w.ix);
+    face_w<T>(bm1, b0, zxP, zxC, hP, hC, uP, vP, uC, vC, dryP, dryC, eC.act, w.ix, w, fx, odd);
+    take_loaded(sh, shu, shv, sb);   // nothing is in flight when the rows begin
+  }
+
+  // one row; false if it is left to the general functions
+  auto row = [&](int r) __attribute__((always_inline)) -> bool {
+    T hN = sh, huN = shu, hvN = shv, bp2 = sb;
+    take_loaded(hN, huN, hvN, bp2);
+    const FlatRow e2 = eF;   // row r + 2
+    load_q(e2, sh, shu, shv);
+    eF = flat_row(E + 3 * min(r + 5, nr + 3), g0l);   // row r + 3; the last rows read again what they have
+    T uN, vN;
+    lmask dryN;
+    prims_w<T>(hN, huN, hvN, bp2, eN.st, w, uN, vN, dryN, odd);
+    // y faces of the row: each lane computes its upper face (j, j+1)
+    const T bl = lane_get(ln.dn, b0), br = lane_get(ln.up, b0);
+    const T zy = w.hdy * ((T(0.5) * (br - bl)) * w.iy);
+    const T hR = lane_get(ln.up, hC), uR = lane_get(ln.up, uC), vR = lane_get(ln.up, vC);
+    const T zyR = lane_get(ln.up, zy);
+    const T zxN = w.hdx * ((T(0.5) * (bp2 - b0)) * w.ix);
+    const lmask act = eC.act;
+    FaceProd<T> fn, fy;
+    face_w<T>(b0, br, zy, zyR, hC, hR, vC, uC, vR, uR, dryC, lm_upper(dryC), act | lm_upper(act), w.iy, w, fy, odd);
+    const T lFh = lane_get(ln.dn, fy.Fh), lFN = lane_get(ln.dn, fy.FN), lFT = lane_get(ln.dn, fy.FT),
+            lsR = lane_get(ln.dn, fy.sR);
+    load_b(eF, sb);
+    face_w<T>(b0, bp1, zxC, zxN, hC, hN, uC, vC, uN, vN, dryC, dryN, act | eN.act, w.ix, w, fn, odd);
+    T rh, rhu, rhv;
+    sum_faces<T>(fn, fx, fy, lFh, lFN, lFT, lsR, rh, rhu, rhv);
+
+    const uint8_t fg = sfl;
+    T rr0 = rh + (rain + srn);   // one of them is 0, or both: rh is never -0, and + 0 changes nothing
+    const lmask stage = act & lm_of((fg & GS_FLAG_STAGE) != 0), cfl = act & lm_of(!(fg & GS_FLAG_CFL_SKIP));
+    const int64_t gC = g0 + eC.row;
+    T n = T(0);
+    if (LEAN) {
+      if (x.P.friction) n = x.ntab[fg & GS_FLAG_CLASS_MASK];
+    } else {
+      const FlatCtx<T> y = cold(x);
+      if (EXT && x.rain_mode == 3 && lm_lane(act)) rr0 = rh + x.frame[gat(y.rain_lookup + gC, eC.below * 4u)];
+      if (x.P.friction) {
+        if (y.n_field || y.cls) {
+          if (lm_lane(act)) n = y.n_field ? gat(y.n_field + gC, eC.below * es) : x.ntab[gat(y.cls + gC, eC.below)];
+        } else {
+          n = x.ntab[fg & GS_FLAG_CLASS_MASK];
+        }
+      }
+    }
+    load_c(eN, r + 1, sfl, srn);
+    T h, hu, hv, speed;
+    update_w<T>(hC, huC, hvC, rr0, rhu, rhv, n, act, x.P, w, h, hu, hv, speed, odd);
+    const bool left = lm_any(odd);
+    if (PRE) {   // the first three statements of update(), kept for its reverse
+      const FlatCtx<T> y = cold(x);
+      if (lm_lane(act) && !left) {
+        gat(y.pre0 + gC, eC.below * es) = hC + w.dt * rr0;
+        gat(y.pre1 + gC, eC.below * es) = huC + w.dt * rhu;
+        gat(y.pre2 + gC, eC.below * es) = hvC + w.dt * rhv;
+      }
+    }
+    lam_t<T> key;
+    if (LEAN) {
+      if (lm_any(stage)) {   // |eta| < 2^30 here, and beds are below 2^20
+        h = lm_sel(stage, pos_w(x.eta - b0), h);
+        hu = lm_sel(stage, T(0), hu);
+        hv = lm_sel(stage, T(0), hv);
+        speed = speed_w<T>(h, hu, hv, w);
+      }
+      key = lam_key_w<T>(speed);
+    } else {
+      const FlatCtx<T> y = cold(x);
+      if (lm_lane(act) && !left) finish_cell<T, EXT, LEAN>(y, fg, gC, eC.below * es, b0, h, hu, hv);
+      speed = speed_w<T>(h, hu, hv, w);
+      key = lam_key_w<T>(speed);
+      if (lm_any(act & lm_not(lm_lt(speed, kMaxSpeed<T>)))) key = lam_key<T, true>(h, hu, hv, cold(x).P);
+    }
+    // in a row with an odd lane every lane's store is out of range, so that every way to the next
+    // row's loads holds the same stores
+    const uint32_t so = (lm_lane(act) ? eC.below * es : kNoLane) | (left ? kNoLane : 0u);
+    row_store(qo0, so, eC.row * es, h);
+    row_store(qo1, so, eC.row * es, hu);
+    row_store(qo2, so, eC.row * es, hv);
+    if (left) return false;
+    if (lm_lane(cfl)) top = key > top ? key : top;
+
+    // slide the window one row down
+    hC = hN; huC = huN; hvC = hvN; uC = uN; vC = vN; zxC = zxN; dryC = dryN;
+    b0 = bp1; bp1 = bp2;
+    fx = fn;
+    eC = eN; eN = e2;
+    return true;
+  };
+  int r = 0;   // two rows per trip: half of the window's moves are names instead
+  while (r < nr) {
+    if (!row(r)) break;
+    if (++r == nr) break;
+    if (!row(r)) break;
+    ++r;
+  }
+  lam = top > lam ? top : lam;
+  return r;
+}
+
+// The same rows by the general functions of gs_device.h, for every operand.
+template <typename T, bool PRE, bool EXT, bool LEAN>
+__device__ __forceinline__ void flat_rows_general(const FlatCtx<T>& hot, const GS_C uint64_t* E, int i0, int nr, int c0,
+                                                  int lane, lam_t<T>& lam) {
+  const FlatCtx<T> x = cold(hot);
   const Phys<T>& P = x.P;
   const T ix = P.inv_dx, iy = P.inv_dy, hdx = P.half_dx, hdy = P.half_dy, g = P.g, hm = P.h_min;
-  const GS_G int32_t* irc = x.tile_irc + 3 * t;
-  const int i0 = irc[0], nr = irc[1], c0 = irc[2];
-  const GS_G uint64_t* E = x.ent + 3 * x.tile_e0[t];   // entry of row i0 - 2
   bool sm2, sm1, sC, sN;
   int64_t gm2, gm1, gC, gN;   // first flat id of rows i-2, i-1, i, i+1 (uniform)
   const uint32_t om2 = sweep_lane<T>(E, lane, gm2, sm2);
   const uint32_t om1 = sweep_lane<T>(E + 3, lane, gm1, sm1);
   uint32_t oC = sweep_lane<T>(E + 6, lane, gC, sC);
   uint32_t oN = sweep_lane<T>(E + 9, lane, gN, sN);
-  const T bm2 = sweep_b(x, gm2, om2, sm2);
-  T bm1 = sweep_b(x, gm1, om1, sm1), b0 = sweep_b(x, gC, oC, sC), bp1 = sweep_b(x, gN, oN, sN);
+  const T bm2 = sweep_b(x, gm2, om2, sm2), bm1 = sweep_b(x, gm1, om1, sm1);
+  T b0 = sweep_b(x, gC, oC, sC), bp1 = sweep_b(x, gN, oN, sN);
   T hP, huP, hvP, uP, vP;
   sweep_q(x, gm1, om1, sm1, hP, huP, hvP);
   prims(hP, huP, hvP, hm, uP, vP);
@@ -590,16 +858,11 @@ __device__ __forceinline__ void flat_tile(const FlatCtx<T>& x, int64_t t, int la
   sweep_q(x, gC, oC, sC, hC, huC, hvC);
   prims(hC, huC, hvC, hm, uC, vC);
   T gzxC = (T(0.5) * (bp1 - bm1)) * ix;
-  Face<T> fx;
-  face<T>(bm1, b0, gzxP, gzxC, hP, hC, uP, vP, uC, vC, hdx, g, hm, fx);
-  // the x-face below the current row, as the products the current cell adds (zero when
-  // the face is gated off: see the accumulation below)
-  const bool xg = fx.gate;
-  T xFh = xg ? fx.Fh * ix : T(0), xFN = xg ? fx.FN * ix : T(0), xFT = xg ? fx.FT * ix : T(0),
-    xsR = xg ? fx.srcR * ix : T(0);
+  FaceProd<T> fx;
+  face_prod<T>(bm1, b0, gzxP, gzxC, hP, hC, uP, vP, uC, vC, hdx, ix, g, hm, fx);
 
   for (int r = 0; r < nr; ++r) {
-    const GS_G uint64_t* Er = E + 3 * (r + 2);   // this row's entry
+    const GS_C uint64_t* Er = E + 3 * (r + 2);   // this row's entry
     bool sNN;
     int64_t gNN;
     const uint32_t oNN = sweep_lane<T>(Er + 6, lane, gNN, sNN);
@@ -608,46 +871,16 @@ __device__ __forceinline__ void flat_tile(const FlatCtx<T>& x, int64_t t, int la
     sweep_q(x, gN, oN, sN, hN, huN, hvN);
     prims(hN, huN, hvN, hm, uN, vN);
     const T gzxN = (T(0.5) * (bp2 - b0)) * ix;
-    Face<T> fn;
-    face<T>(b0, bp1, gzxC, gzxN, hC, hN, uC, vC, uN, vN, hdx, g, hm, fn);
-    const bool ng = fn.gate;
-    const T nFh = ng ? fn.Fh * ix : T(0), nFN = ng ? fn.FN * ix : T(0), nFT = ng ? fn.FT * ix : T(0);
-    const T nsL = ng ? fn.srcL * ix : T(0), nsR = ng ? fn.srcR * ix : T(0);
-
-    // y faces of the row: each lane computes its upper face (j, j+1)
+    FaceProd<T> fn, fy;
+    face_prod<T>(b0, bp1, gzxC, gzxN, hC, hN, uC, vC, uN, vN, hdx, ix, g, hm, fn);
     const T bl = lane_lower(b0), br = lane_upper(b0);
     const T gzy = (T(0.5) * (br - bl)) * iy;
     const T hR = lane_upper(hC), uR = lane_upper(uC), vR = lane_upper(vC);
     const T gzyR = lane_upper(gzy);
-    Face<T> fy;
-    face<T>(b0, br, gzy, gzyR, hC, hR, vC, uC, vR, uR, hdy, g, hm, fy);
-    const bool yg = fy.gate;
-    const T yFh = yg ? fy.Fh * iy : T(0), yFN = yg ? fy.FN * iy : T(0), yFT = yg ? fy.FT * iy : T(0);
-    const T ysL = yg ? fy.srcL * iy : T(0);
-    const T yFhB = lane_lower(yFh), yFNB = lane_lower(yFN), yFTB = lane_lower(yFT);
-    const T ysRB = lane_lower(yg ? fy.srcR * iy : T(0));
-
-    // The four faces in the reference's order. A face gated off (both cells dry) adds
-    // zeros: the sums start at +0 and IEEE addition yields -0 only from two -0 terms, so
-    // they never hold -0, and x + 0 = x - 0 = x for every other x; the gate costs one
-    // select per face term instead of one per use.
-    T rh = T(0), rhu = T(0), rhv = T(0);
-    rh = rh - nFh;
-    rhu = rhu - nFN;
-    rhv = rhv - nFT;
-    rhu = rhu - nsL;
-    rh = rh + xFh;
-    rhu = rhu + xFN;
-    rhv = rhv + xFT;
-    rhu = rhu + xsR;
-    rh = rh - yFh;
-    rhu = rhu - yFT;
-    rhv = rhv - yFN;
-    rhv = rhv - ysL;
-    rh = rh + yFhB;
-    rhu = rhu + yFTB;
-    rhv = rhv + yFNB;
-    rhv = rhv + ysRB;
+    face_prod<T>(b0, br, gzy, gzyR, hC, hR, vC, uC, vR, uR, hdy, iy, g, hm, fy);
+    const T lFh = lane_lower(fy.Fh), lFN = lane_lower(fy.FN), lFT = lane_lower(fy.FT), lsR = lane_lower(fy.sR);
+    T rh, rhu, rhv;
+    sum_faces<T>(fn, fx, fy, lFh, lFN, lFT, lsR, rh, rhu, rhv);
 
     if ((Er[2] >> lane) & 1ull) {   // an active cell: lanes 2..61 only
       const uint32_t ob = oC / (uint32_t)sizeof(T);   // byte offset in a 1-byte plane
@@ -660,7 +893,7 @@ __device__ __forceinline__ void flat_tile(const FlatCtx<T>& x, int64_t t, int la
       } else if (EXT && x.rain_mode == 3) {
         rr0 = rr0 + x.frame[gat(x.rain_lookup + gC, (oC / (uint32_t)sizeof(T)) * 4u)];
       }
-      if (PRE) {   // the first three statements of update(), kept for its reverse
+      if (PRE) {
         gat(x.pre0 + gC, oC) = hC + x.dt * rr0;
         gat(x.pre1 + gC, oC) = huC + x.dt * rhu;
         gat(x.pre2 + gC, oC) = hvC + x.dt * rhv;
@@ -671,16 +904,7 @@ __device__ __forceinline__ void flat_tile(const FlatCtx<T>& x, int64_t t, int la
                                  : x.ntab[(!LEAN && x.cls) ? gat(x.cls + gC, ob) : (fg & GS_FLAG_CLASS_MASK)];
       T h, hu, hv;
       update<T>(hC, huC, hvC, rr0, rhu, rhv, x.dt, n, P, h, hu, hv);
-      if (fg & GS_FLAG_STAGE) {
-        const T hs = x.eta - b0;
-        h = hs > T(0) ? hs : T(0);
-        hu = T(0);
-        hv = T(0);
-      }
-      if (!LEAN) {
-        if (x.max_h && h > gat(x.max_h + gC, oC)) gat(x.max_h + gC, oC) = h;
-        active_force<T, EXT>(x, fg, gC, oC, ob, h, hu, hv);
-      }
+      finish_cell<T, EXT, LEAN>(x, fg, gC, oC, b0, h, hu, hv);
       gat(x.qo0 + gC, oC) = h;
       gat(x.qo1 + gC, oC) = hu;
       gat(x.qo2 + gC, oC) = hv;
@@ -692,10 +916,31 @@ __device__ __forceinline__ void flat_tile(const FlatCtx<T>& x, int64_t t, int la
 
     // slide the window one row down
     hC = hN; huC = huN; hvC = hvN; uC = uN; vC = vN; gzxC = gzxN;
-    bm1 = b0; b0 = bp1; bp1 = bp2;
-    xFh = nFh; xFN = nFN; xFT = nFT; xsR = nsR;
+    b0 = bp1; bp1 = bp2;
+    fx = fn;
     gC = gN; oC = oN; gN = gNN; oN = oNN; sN = sNN;
   }
+}
+
+// One row-sweep tile: the fused update of the active lanes of rows i0 .. i0+nr-1 of one
+// 64-column window. Every lane of the wavefront must call it. PRE: also write the pre-friction
+// state (the adjoint's recomputation); a separate instantiation keeps those pointers out of the
+// plain step's scalar registers. LEAN: the domain has no per-cell Manning field or class plane, no
+// running maximum and no active-cell forcing, so none of their pointers is held (the host checks
+// that they are all null).
+template <typename T, bool PRE, bool EXT, bool LEAN = false>
+__device__ __forceinline__ void flat_tile(const FlatCtx<T>& x, int64_t t, int lane, lam_t<T>& lam) {
+  const GS_C FlatK<T>* k = cold_ptr<T>(x.k);
+  const GS_C int32_t* irc = cp(gp((int32_t*)k->tile_irc)) + 3 * t;
+  const int i0 = irc[0], nr = irc[1], c0 = irc[2];
+  const GS_C uint64_t* E = cp(gp((uint64_t*)k->ent)) + 3 * cp(gp((int64_t*)k->tile_e0))[t];   // entry of row i0 - 2
+  int r = 0;
+  constexpr int forms = kWaveFast | kWaveLam;
+  if ((x.wave & forms) == forms && vabs(x.eta) < T(0x1p30) && nr <= kWaveRows) {
+    const WaveC<T> w = wave_consts<T>(x.P, x.dt, x.wave);
+    r = __builtin_amdgcn_readfirstlane(flat_rows<T, PRE, EXT, LEAN>(x, w, E, i0, nr, c0, lane, lam));
+  }
+  if (r < nr) flat_rows_general<T, PRE, EXT, LEAN>(x, E + 3 * r, i0 + r, nr - r, c0, lane, lam);
 }
 
 // Workgroup b's place in an XCD-major order: workgroups are dealt round-robin to the 8
@@ -728,52 +973,54 @@ __global__ __launch_bounds__(kFBlock) void k_flat_step(FlatK<T> a) {
 }
 
 // One step of one flat domain by row-sweep tiles, one wavefront per tile in band-major tile
-// order and XCD-major wavefront order (the loop also serves a grid smaller than that). The float32 plain
-// step is held to 72 VGPRs (7 wavefronts per SIMD instead of 6; a few scalar registers are
-// then reloaded in the row loop), which measured 2-3 % faster. LEAN (a domain with no
-// per-cell Manning field or class plane, running maximum or active-cell forcing) drops those pointers:
-// 34 scalar registers spilled to lanes instead of 75, 4 % faster on the coastal case.
+// order and XCD-major wavefront order. What bounds it is the issue of vector instructions (about
+// 400 per row, 0.8 of the cycles) and, on a domain of one round of tiles, the slowest tile. The
+// float32 steps are held to 80 VGPRs (6 wavefronts per SIMD), where no row reloads a spilled
+// register. LEAN (a domain with no per-cell Manning field or class plane, running maximum or
+// active-cell forcing) drops those paths. us per step, general functions with 4-row tiles before
+// and wavefront forms now: 2048^2 coastal domain (lean) 63 and 40, 1500^2 with the forcing tail
+// (below) 69 and 57.
 template <typename T, bool PRE, bool LEAN = false>
-__global__ __launch_bounds__(kFBlock) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && !PRE ? 7 : 1))) void k_flat_sweep(FlatK<T> a) {
+__global__ __launch_bounds__(kSBlock<T>) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 6 : 1))) void k_flat_sweep(FlatK<T> a) {
   const FlatClk<T> ck = flat_clock<T, 1>(a);
   if (!ck.live) return;   // the whole grid sees the same clock
   FlatCtx<T> x;
   flat_ctx<T, 1>(a, ck, x);
+  x.k = kernel_arg<T>();
   __shared__ T s_ntab[GS_MAX_CLASSES];
   for (int k = (int)threadIdx.x; k < a.n_classes; k += (int)blockDim.x) s_ntab[k] = a.ntab[k];
   __syncthreads();
   x.ntab = s_ntab;
   const int lane = threadIdx.x & 63;
   const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const int64_t nwaves = (int64_t)gridDim.x * (kFBlock / 64);
+  const int64_t nwaves = (int64_t)gridDim.x * kSweepWaves<T>;
   lam_t<T> lam = 0;
   // PRE (the adjoint's recomputation) also compiles the extended forcings in, so that a
   // replay reads rain through the per-cell lookup exactly as the forward run's extended sweep
-  for (int64_t t = (int64_t)xcd_rank(blockIdx.x, gridDim.x) * (kFBlock / 64) + wv; t < a.n_tiles; t += nwaves)
+  for (int64_t t = (int64_t)xcd_rank(blockIdx.x, gridDim.x) * kSweepWaves<T> + wv; t < a.n_tiles; t += nwaves)
     flat_tile<T, PRE, PRE, LEAN>(x, t, lane, lam);
   grid_reduce_and_plan(lam_key_bits64(lam), a.clock, a.plan, true);
 }
 
 // The sweep with the extended forcings compiled in: Green-Ampt infiltration, drain-tau and
 // rain read through a per-cell lookup into a native-grid table (launched only when one of
-// them is set; the plain sweep has no register to spare for them). The float32 build is
-// held to 72 VGPRs (7 wavefronts per SIMD instead of 6, a few registers then spilled):
-// 2.62 against 2.74 ms per step with the coastal forcing tail on the 16384^2 case.
+// them is set).
 template <typename T>
-__global__ __launch_bounds__(kFBlock) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 7 : 1))) void k_flat_sweep_ext(FlatK<T> a) {
+__global__ __launch_bounds__(kSBlock<T>) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 6 : 1))) void k_flat_sweep_ext(FlatK<T> a) {
   const FlatClk<T> ck = flat_clock<T, 1>(a);
   if (!ck.live) return;
   FlatCtx<T> x;
   flat_ctx<T, 1>(a, ck, x);
+  x.k = kernel_arg<T>();
   __shared__ T s_ntab[GS_MAX_CLASSES];
   for (int k = (int)threadIdx.x; k < a.n_classes; k += (int)blockDim.x) s_ntab[k] = a.ntab[k];
   __syncthreads();
   x.ntab = s_ntab;
   const int lane = threadIdx.x & 63;
   const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const int64_t nwaves = (int64_t)gridDim.x * (kFBlock / 64);
+  const int64_t nwaves = (int64_t)gridDim.x * kSweepWaves<T>;
   lam_t<T> lam = 0;
-  for (int64_t t = (int64_t)xcd_rank(blockIdx.x, gridDim.x) * (kFBlock / 64) + wv; t < a.n_tiles; t += nwaves)
+  for (int64_t t = (int64_t)xcd_rank(blockIdx.x, gridDim.x) * kSweepWaves<T> + wv; t < a.n_tiles; t += nwaves)
     flat_tile<T, false, true>(x, t, lane, lam);
   grid_reduce_and_plan(lam_key_bits64(lam), a.clock, a.plan, true);
 }
@@ -979,6 +1226,11 @@ static int build_flat(const GsFlat* f, const GsPhys* p, const GsForcing& fo, GsC
   a.ring_t = f->ring_t;
   a.ring_stage = (const T*)f->ring_stage;
   a.P = make_phys<T>(*p, f->dx, f->dy);
+  // the wavefront forms address a tile's rows and their stencil with 32-bit offsets
+  const int64_t span = (kWaveRows + 4) * (int64_t)sizeof(T);
+  a.wave = (int64_t)f->nyp * span < ((int64_t)1 << 31) && fo.rain_row_pitch * span < ((int64_t)1 << 31)
+               ? wave_flags<T>(a.P, true)
+               : 0;
   a.rain_mode = fo.n_rain > 0 ? (fo.rain_gridded ? (f->rain_lookup ? 3 : 2) : 1) : 0;
   a.rain_lookup = f->rain_lookup;
   a.n_rmode = f->n_ring_mode;
@@ -997,18 +1249,18 @@ static int build_flat(const GsFlat* f, const GsPhys* p, const GsForcing& fo, GsC
 // Workgroups of a one-wavefront-per-item kernel that are resident at once on the current
 // device (cached per device and kernel); the grid never exceeds the work.
 template <typename F>
-static unsigned resident_grid(F kern, std::atomic<int>* cache, int64_t items) {
+static unsigned resident_grid(F kern, std::atomic<int>* cache, int64_t items, int block = kFBlock) {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) dev = -1;
   int per = (dev >= 0 && dev < 64) ? cache[dev].load(std::memory_order_relaxed) : 0;
   if (per <= 0) {
     int occ = 0, cus = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, kern, kFBlock, 0) != hipSuccess) occ = 4;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, kern, block, 0) != hipSuccess) occ = 4;
     if (dev < 0 || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) cus = 256;
     per = (occ > 0 ? occ : 1) * (cus > 0 ? cus : 1);
     if (dev >= 0 && dev < 64) cache[dev].store(per, std::memory_order_relaxed);
   }
-  const int64_t need = (items + kFBlock / 64 - 1) / (kFBlock / 64);
+  const int64_t need = (items + block / 64 - 1) / (block / 64);
   return (unsigned)(need < per ? (need > 0 ? need : 1) : per);
 }
 
@@ -1018,37 +1270,20 @@ static unsigned flat_grid(int64_t nchunks) {
   return resident_grid(k_flat_step<T, MODE>, cache, nchunks);
 }
 
-// The sweeps launch one wavefront per tile (four tiles per workgroup) when the tiles fill
-// the resident grid more than four times: the hardware then keeps every SIMD fed until the
-// last tile, where a resident grid striding over the tiles left a partial last round (and
-// measured 10-14 % slower on the coastal case, 4.9 rounds, and the full 640 M-cell grid,
-// 23). Fewer tiles run on the resident grid: one wavefront per tile from one resident grid
-// up measured 9 % faster on a 2048^2 domain (1.3 rounds) but 4.5 % slower summed over the
-// 64 ensemble members' plain runs (mostly shorter tiles of smaller domains).
-template <typename K>
-static unsigned sweep_grid(K kern, std::atomic<int>* cache, int64_t ntiles) {
-  const unsigned resident = resident_grid(kern, cache, ntiles);
-  const int64_t need = (ntiles + kFBlock / 64 - 1) / (kFBlock / 64);
-  if (need <= 4 * (int64_t)resident) return resident;
-  return (unsigned)need;
-}
-
-template <typename T, bool PRE, bool LEAN = false>
-static unsigned sweep_grid_for(int64_t ntiles) {
-  static std::atomic<int> cache[64];
-  return sweep_grid(k_flat_sweep<T, PRE, LEAN>, cache, ntiles);
+// The sweeps launch one wavefront per tile: the hardware then keeps every SIMD fed until the last
+// tile, where a resident grid striding over the tiles leaves a partial last round and ends all its
+// workgroups at once, whose atomics then queue with nothing beside them (one wavefront per tile
+// against the resident grid: 1536^2 adjoint with its 80 sweeps 10.85 against 11.48 ms, 2048^2 lean
+// 43.1 against 43.5 us per step, 1500^2 with the forcing tail 64.1 against 65.7).
+template <typename T>
+static unsigned sweep_grid(int64_t ntiles) {
+  return (unsigned)((ntiles + kSweepWaves<T> - 1) / kSweepWaves<T>);
 }
 
 // The domain may take the LEAN sweep: nothing it would skip is set.
 template <typename T>
 static bool flat_lean(const FlatK<T>& a) {
   return !a.n_field && !a.cls && !a.max_h && !a.sponge && !a.clamp && !a.infil && !a.drain;
-}
-
-template <typename T>
-static unsigned sweep_ext_grid(int64_t ntiles) {
-  static std::atomic<int> cache[64];
-  return sweep_grid(k_flat_sweep_ext<T>, cache, ntiles);
 }
 
 // The launch gs_flat_step makes for `a` (without the pre-friction state): which kernel, its
@@ -1062,17 +1297,17 @@ static void flat_launch_choice(const FlatK<T>& a, int* kernel, int64_t* blocks, 
     *resident = *blocks;
   } else if (a.ga_ks || a.ga_inv_tau || a.rain_mode == 3) {
     *kernel = 2;
-    *blocks = sweep_ext_grid<T>(a.n_tiles);
-    *resident = resident_grid(k_flat_sweep_ext<T>, c_ext, a.n_tiles);
+    *blocks = sweep_grid<T>(a.n_tiles);
+    *resident = resident_grid(k_flat_sweep_ext<T>, c_ext, a.n_tiles, kSBlock<T>);
   } else if (flat_lean(a)) {
     static std::atomic<int> c_lean[64];
     *kernel = 1;
-    *blocks = sweep_grid_for<T, false, true>(a.n_tiles);
-    *resident = resident_grid(k_flat_sweep<T, false, true>, c_lean, a.n_tiles);
+    *blocks = sweep_grid<T>(a.n_tiles);
+    *resident = resident_grid(k_flat_sweep<T, false, true>, c_lean, a.n_tiles, kSBlock<T>);
   } else {
     *kernel = 1;
-    *blocks = sweep_grid_for<T, false>(a.n_tiles);
-    *resident = resident_grid(k_flat_sweep<T, false>, c_plain, a.n_tiles);
+    *blocks = sweep_grid<T>(a.n_tiles);
+    *resident = resident_grid(k_flat_sweep<T, false>, c_plain, a.n_tiles, kSBlock<T>);
   }
 }
 
@@ -1090,16 +1325,16 @@ static int flat_step_launch(const FlatK<T>& a, hipStream_t s) {
     GS_HIP(hipGetLastError(), "k_flat_ring_force launch");
   }
   if (a.n_tiles > 0 && a.pre[0]) {
-    hipLaunchKernelGGL((k_flat_sweep<T, true>), dim3(sweep_grid_for<T, true>(a.n_tiles)), dim3(kFBlock), 0, s, a);
+    hipLaunchKernelGGL((k_flat_sweep<T, true>), dim3(sweep_grid<T>(a.n_tiles)), dim3(kSBlock<T>), 0, s, a);
     GS_HIP(hipGetLastError(), "k_flat_sweep(pre) launch");
   } else if (a.n_tiles > 0 && (a.ga_ks || a.ga_inv_tau || a.rain_mode == 3)) {
-    hipLaunchKernelGGL((k_flat_sweep_ext<T>), dim3(sweep_ext_grid<T>(a.n_tiles)), dim3(kFBlock), 0, s, a);
+    hipLaunchKernelGGL((k_flat_sweep_ext<T>), dim3(sweep_grid<T>(a.n_tiles)), dim3(kSBlock<T>), 0, s, a);
     GS_HIP(hipGetLastError(), "k_flat_sweep_ext launch");
   } else if (a.n_tiles > 0 && flat_lean(a)) {
-    hipLaunchKernelGGL((k_flat_sweep<T, false, true>), dim3(sweep_grid_for<T, false, true>(a.n_tiles)), dim3(kFBlock), 0, s, a);
+    hipLaunchKernelGGL((k_flat_sweep<T, false, true>), dim3(sweep_grid<T>(a.n_tiles)), dim3(kSBlock<T>), 0, s, a);
     GS_HIP(hipGetLastError(), "k_flat_sweep(lean) launch");
   } else if (a.n_tiles > 0) {
-    hipLaunchKernelGGL((k_flat_sweep<T, false>), dim3(sweep_grid_for<T, false>(a.n_tiles)), dim3(kFBlock), 0, s, a);
+    hipLaunchKernelGGL((k_flat_sweep<T, false>), dim3(sweep_grid<T>(a.n_tiles)), dim3(kSBlock<T>), 0, s, a);
     GS_HIP(hipGetLastError(), "k_flat_sweep launch");
   } else {
     hipLaunchKernelGGL((k_flat_step<T, 1>), dim3(flat_grid<T, 1>(a.nchunks)), dim3(kFBlock), 0, s, a);
@@ -1178,17 +1413,6 @@ struct EnsK {
   unsigned* done;                     // workgroups finished in this launch
 };
 
-// Read a value that the launch never writes through the constant address space: a
-// uniform address then gives scalar loads. The host pass sees an ordinary read.
-template <typename U>
-__device__ __forceinline__ U const_read(const U* p) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  return *(const __attribute__((address_space(4))) U*)p;
-#else
-  return *p;
-#endif
-}
-
 // Fold a wavefront's CFL speed bits of member m into that member's clock (lane 0 waits
 // until its atomic has been performed, as grid_reduce_and_plan's thread 0 does).
 template <typename T>
@@ -1222,19 +1446,22 @@ __device__ __forceinline__ int ens_member_of(const int64_t* tile0, int n, int64_
 // KIND kEnsExt compiles the extended forcings (Green-Ampt, drain-tau, rain through a
 // per-cell lookup) in; kEnsPlain leaves them out; kEnsLean also leaves out the per-cell
 // Manning field, the running maximum and the active-cell forcings (every member has none
-// of them), and its float32 build is held to 72 VGPRs (7 wavefronts per SIMD: 1.81 against
-// 1.93 ms per step on the 64-member case at 82 VGPRs, though 16 VGPRs then spill, a few of
-// them reloaded in the row loop).
+// of them), and its float32 build is held to 96 VGPRs (5 wavefronts per SIMD, nothing spilled; at
+// 80 and 6 the row loop reloads, and 16 members of 256 to 1024 cells a side took 90 us per step at
+// 8 rows a tile against 84).
 enum { kEnsPlain = 0, kEnsExt = 1, kEnsLean = 2 };
 
 template <typename T, int KIND>
-__global__ __launch_bounds__(kFBlock) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && KIND == kEnsLean ? 7 : 1)))
+__global__ __launch_bounds__(kFBlock) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && KIND == kEnsLean ? 5 : 1)))
 void k_ens_step(EnsK<T> e, const FlatK<T>* __restrict__ mem, const int64_t* __restrict__ tile0) {
   const int lane = threadIdx.x & 63;
   const int64_t nwaves = (int64_t)gridDim.x * (kFBlock / 64);
   const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int64_t wave = (int64_t)xcd_rank(blockIdx.x, gridDim.x) * (kFBlock / 64) + wv;
   const int64_t tpp = e.tpp;
+  // the Manning table of the wavefront's member: a lookup beside the row's loads in flight must not
+  // wait for them, as one in global memory would
+  __shared__ T s_ntab[kFBlock / 64][GS_MAX_CLASSES];
   int m = -1;          // the member whose maximum `lam` holds
   lam_t<T> lam = 0;
   for (int64_t base = wave * tpp; base < e.ntiles; base += nwaves * tpp) {
@@ -1247,12 +1474,16 @@ void k_ens_step(EnsK<T> e, const FlatK<T>* __restrict__ mem, const int64_t* __re
         ens_flush(e, m, lam_key_bits64(lam));
         lam = 0;
         m = mt;
+        const T* nt = const_read(&mem[mt].ntab);
+        for (int k = lane; k < const_read(&mem[mt].n_classes); k += 64) s_ntab[wv][k] = gp(nt)[k];
       }
       const FlatK<T> v = const_read(mem + mt);
       const FlatClk<T> ck = flat_clock<T, 1>(v);
       if (!ck.live) continue;
       FlatCtx<T> x;
       flat_ctx<T, 1>(v, ck, x);
+      x.k = cp((const GS_G FlatK<T>*)(mem + mt));
+      x.ntab = s_ntab[wv];
       flat_tile<T, false, KIND == kEnsExt, KIND == kEnsLean>(x, gc - const_read(tile0 + mt), lane, lam);
     }
   }
@@ -1477,6 +1708,10 @@ static int ens_build_views(GsEns* e, const GsFlat* members, const GsPhys* phys, 
   e->ntiles = c0[e->n];
   e->kind = ens_kind<T>(views.data(), e->n);
   e->occ = ens_occupancy<T>(e->kind);
+  // until a launch shape is set: one wavefront per tile, as the plain sweep (16 members of 256 to
+  // 1024 cells a side, tiles of 7 rows: 84 us per step; the resident grid's two rounds: 91)
+  const int64_t per_tile = (e->ntiles + 3) / 4;
+  e->blocks = (int)(per_tile < (1 << 24) ? per_tile : (1 << 24));
   GS_HIP(hipMalloc(&e->mem, sizeof(FlatK<T>) * (size_t)e->n), "ensemble views");
   GS_HIP(hipMalloc((void**)&e->tile0, sizeof(int64_t) * ((size_t)e->n + 1)), "ensemble tile table");
   GS_HIP(hipMalloc((void**)&e->done, 256), "ensemble counter");
@@ -1821,9 +2056,6 @@ static int ens_run_noalloc_t(const GsFlat* members, const GsPhys* phys, const Gs
   // before it is overwritten (a synchronous copy, so the host staging is free on return)
   GS_HIP(hipStreamSynchronize(s), "hipStreamSynchronize");
   GS_HIP(hipMemcpy(base, g_scratch_host, need, hipMemcpyHostToDevice), "scratch h2d");
-  int cus = 256, dev = 0;
-  if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-  if (cus < 1) cus = 256;
   EnsK<T> k;
   k.mem = (const FlatK<T>*)((unsigned char*)base + off_views);
   k.tile0 = (const int64_t*)((unsigned char*)base + off_tile);
@@ -1831,7 +2063,7 @@ static int ens_run_noalloc_t(const GsFlat* members, const GsPhys* phys, const Gs
   k.tpp = 1;
   k.ntiles = c0[n];
   k.done = (unsigned*)base;
-  const int64_t blocks = ens_grid(0, ens_occupancy<T>(kind), cus, k.ntiles, 1);
+  const int64_t blocks = (k.ntiles + 3) / 4 > 0 ? (k.ntiles + 3) / 4 : 1;   // one wavefront per tile
   for (int64_t i = 0; i < nsteps; ++i) {
     ens_launch_kind<T>(kind, blocks, s, k);
     GS_HIP(hipGetLastError(), "k_ens_step launch");

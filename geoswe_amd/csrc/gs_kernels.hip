@@ -202,44 +202,6 @@ __device__ __forceinline__ S load_b(const DenseK<T, S>& a, const DenseTile<T, S>
   return row_at(row_base(a.bed + (int64_t)mi * a.pitch), (O)(uint32_t)x.cm.mjb * (O)sizeof(S));
 }
 
-// The four faces of a cell in the reference's order. A face gated off (both cells dry) adds
-// zeros: the sums start at +0 and IEEE addition yields -0 only from two -0 terms, so they never
-// hold -0, and x + 0 = x - 0 = x for every other x.
-template <typename T>
-__device__ __forceinline__ void sum_faces(const FaceProd<T>& up, const FaceProd<T>& dn, const FaceProd<T>& right,
-                                          T lFh, T lFN, T lFT, T lsR, T& rh, T& rhu, T& rhv) {
-  rh = T(0); rhu = T(0); rhv = T(0);
-  rh = rh - up.Fh;
-  rhu = rhu - up.FN;
-  rhv = rhv - up.FT;
-  rhu = rhu - up.sL;
-  rh = rh + dn.Fh;
-  rhu = rhu + dn.FN;
-  rhv = rhv + dn.FT;
-  rhu = rhu + dn.sR;
-  rh = rh - right.Fh;
-  rhu = rhu - right.FT;
-  rhv = rhv - right.FN;
-  rhv = rhv - right.sL;
-  rh = rh + lFh;
-  rhu = rhu + lFT;
-  rhv = rhv + lFN;
-  rhv = rhv + lsR;
-}
-
-// face() as the products its cells add, zero where it is gated off.
-template <typename T>
-__device__ __forceinline__ void face_prod(T bL, T bR, T gzL, T gzR, T hL, T hR, T uNL, T uTL, T uNR, T uTR, T half,
-                                          T inv, T g, T hm, FaceProd<T>& f) {
-  Face<T> q;
-  face<T>(bL, bR, gzL, gzR, hL, hR, uNL, uTL, uNR, uTR, half, g, hm, q);
-  f.Fh = q.gate ? q.Fh * inv : T(0);
-  f.FN = q.gate ? q.FN * inv : T(0);
-  f.FT = q.gate ? q.FT * inv : T(0);
-  f.sL = q.gate ? q.srcL * inv : T(0);
-  f.sR = q.gate ? q.srcR * inv : T(0);
-}
-
 // What a cell's update reads from its planes. Lanes that write nothing read nothing. LEAN: the
 // domain has no flags, Manning, class and running-max plane and no gridded rain.
 template <bool LEAN, typename T, typename S>
@@ -322,9 +284,9 @@ __device__ __forceinline__ int dense_rows(const DenseK<T, S>& a, const DenseTile
   face_w<T>(bm1, b0, zxP, zxC, hP, hC, uP, vP, uC, vC, dryP, dryC, act, w.ix, w, fx, odd);
 
   // where the written lanes' results go (offsets of 32 bits within the tile)
-  const StoreBase st0 = store_base(x.qo[0] + (int64_t)i0 * a.pitch), st1 = store_base(x.qo[1] + (int64_t)i0 * a.pitch),
-                  st2 = store_base(x.qo[2] + (int64_t)i0 * a.pitch);
-  const uint32_t lane_st = x.col_ok ? (uint32_t)x.c * (uint32_t)sizeof(S) : kNoStore;
+  const RowBuf st0 = row_buf(x.qo[0] + (int64_t)i0 * a.pitch), st1 = row_buf(x.qo[1] + (int64_t)i0 * a.pitch),
+                  st2 = row_buf(x.qo[2] + (int64_t)i0 * a.pitch);
+  const uint32_t lane_st = x.col_ok ? (uint32_t)x.c * (uint32_t)sizeof(S) : kNoLane;
   const uint32_t pitch_st = (uint32_t)a.pitch * (uint32_t)sizeof(S);
   take_loaded(rN.h, rN.hu, rN.hv, sp2);   // nothing is in flight when the rows begin
 
@@ -391,7 +353,7 @@ __device__ __forceinline__ int dense_rows(const DenseK<T, S>& a, const DenseTile
         // a row with an odd lane is left through the same stores, each lane's out of range, so
         // that every way to the next row's loads holds the same stores
         const bool left = lm_any(odd);
-        const uint32_t at = lane_st | (left ? kNoStore : 0u), row_st = (uint32_t)(i - i0) * pitch_st;
+        const uint32_t at = lane_st | (left ? kNoLane : 0u), row_st = (uint32_t)(i - i0) * pitch_st;
         if (!LEAN && a.max_h && x.col_ok && !left) {
           const int64_t idx = (int64_t)i * a.pitch + x.c;
           if (hS > a.max_h[idx]) a.max_h[idx] = hS;

@@ -5,6 +5,7 @@
 // CompressedMesh2D / CompressedSWE numbering, src/geoswe/compressed_mesh.py:108-187 and
 // compressed_rhs.py:241-369), in one pass over the grid with five rolling rows of ids
 // instead of full-grid temporaries.
+#include <algorithm>
 #include <cstdlib>
 #include <cstring>
 #include <vector>
@@ -185,8 +186,13 @@ int gs_flat_mesh_build(const uint8_t* inside, int nxp, int nyp, int ring, int sw
     }
   int64_t rows = sweep_rows;
   if (rows == -1) {
-    rows = 1;
-    while (rows < max_sweep_rows && busy / (2 * rows) >= tile_target) rows *= 2;
+    // about sqrt(busy/1000), kept where it gives tile_target to 2*tile_target tiles
+    const int64_t thousands = busy / 1000;
+    rows = 0;
+    while ((rows + 1) * (rows + 1) <= thousands) ++rows;
+    rows = std::max(rows, busy / (2 * (int64_t)tile_target) + 1);
+    rows = std::min(rows, std::min(busy / (int64_t)tile_target, (int64_t)max_sweep_rows));
+    rows = std::max<int64_t>(rows, 1);
   }
   // row-sweep tiles: in each band of `rows` rows, 64-lane windows placed from the left, each
   // starting two columns before the first active column the previous windows left uncovered

@@ -85,23 +85,33 @@ __device__ __forceinline__ GS_G P* row_base(P* p) {
   __asm__("" : "+s"(q));
   return q;
 }
-// Stores of one row of a tile for the lanes whose offset lies in the buffer (kNoStore does not):
-// without a branch around them, so that the wait for the next row's loads, which are older, need
-// not count on the stores having been made.
-constexpr uint32_t kNoStore = 0xFFFFFFF0u;
-typedef __amdgpu_buffer_rsrc_t StoreBase;
+// One row of a tile through a buffer that starts at the tile: a lane at offset kNoLane stores
+// nothing and loads 0, by the bounds check of the buffer. There is no branch around the access, so
+// that the wait for the next row's loads, which are older than this row's stores, need not count on
+// the stores having been made.
+constexpr uint32_t kNoLane = 0xFFFFFFF0u;
+typedef __amdgpu_buffer_rsrc_t RowBuf;
 template <typename P>
-__device__ __forceinline__ StoreBase store_base(P* p) {
+__device__ __forceinline__ RowBuf row_buf(P* p) {
   const uint64_t a = (uint64_t)p;   // uniform; made so for the compiler too
   const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)a), hi = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32));
   return __builtin_amdgcn_make_buffer_rsrc((void*)(((uint64_t)hi << 32) | lo), 0, 0x80000000, 0x00020000);
 }
-__device__ __forceinline__ void row_store(StoreBase r, uint32_t lane_off, uint32_t row_off, float v) {
+__device__ __forceinline__ void row_store(RowBuf r, uint32_t lane_off, uint32_t row_off, float v) {
   __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), r, lane_off, row_off, 0);
 }
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ void row_store(StoreBase r, uint32_t lane_off, uint32_t row_off, double v) {
+__device__ __forceinline__ void row_store(RowBuf r, uint32_t lane_off, uint32_t row_off, double v) {
   __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), r, lane_off, row_off, 0);
+}
+__device__ __forceinline__ void row_load(RowBuf r, uint32_t lane_off, uint32_t row_off, float& v) {
+  v = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, lane_off, row_off, 0));
+}
+__device__ __forceinline__ void row_load(RowBuf r, uint32_t lane_off, uint32_t row_off, double& v) {
+  v = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, lane_off, row_off, 0));
+}
+__device__ __forceinline__ void row_load(RowBuf r, uint32_t lane_off, uint32_t row_off, uint8_t& v) {
+  v = __builtin_amdgcn_raw_buffer_load_b8(r, lane_off, row_off, 0);
 }
 // Four loaded values moved out of the registers they were loaded into, before the loads of the
 // next row into those registers: the wait that this implies is for loads a row old, where the
@@ -122,6 +132,23 @@ __device__ __forceinline__ void take_loaded(double& a, double& b, double& c, dou
 __device__ __forceinline__ lmask lm_upper(lmask m) { return m >> 1; }
 // a uniform value in a vector register: fast instructions that read a scalar register run at
 // half rate
+// A uniform value in scalar registers.
+__device__ __forceinline__ float sreg(float x) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(x))); }
+__device__ __forceinline__ double sreg(double x) {
+  const uint64_t b = (uint64_t)__double_as_longlong(x);
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)b), hi = __builtin_amdgcn_readfirstlane((uint32_t)(b >> 32));
+  return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+// The value itself, for a rare branch: what is computed from it is not moved out of the row loop,
+// where it would hold a register.
+__device__ __forceinline__ float here(float x) {
+  asm volatile("" : "+v"(x));
+  return x;
+}
+__device__ __forceinline__ double here(double x) {
+  asm volatile("" : "+v"(x));
+  return x;
+}
 __device__ __forceinline__ float vreg(float x) {
   float y;
   __asm__("v_mov_b32 %0, %1" : "=v"(y) : "s"(x));
@@ -211,12 +238,15 @@ struct Lanes {
 GS_HD Lanes lanes_of(int) { return {0, 0}; }
 template <typename T> GS_HD T lane_get(int, T x) { return x; }
 template <typename P> GS_HD GS_G P* row_base(P* p) { return (GS_G P*)p; }
-typedef void* StoreBase;
-constexpr uint32_t kNoStore = 0xFFFFFFF0u;
-template <typename P> GS_HD StoreBase store_base(P* p) { return (void*)p; }
-template <typename T> GS_HD void row_store(StoreBase, uint32_t, uint32_t, T) {}
+typedef void* RowBuf;
+constexpr uint32_t kNoLane = 0xFFFFFFF0u;
+template <typename P> GS_HD RowBuf row_buf(P* p) { return (void*)p; }
+template <typename T> GS_HD void row_store(RowBuf, uint32_t, uint32_t, T) {}
+template <typename T> GS_HD void row_load(RowBuf, uint32_t, uint32_t, T&) {}
 template <typename T> GS_HD void take_loaded(T&, T&, T&, T&) {}
 template <typename T> GS_HD T vreg(T x) { return x; }
+template <typename T> GS_HD T sreg(T x) { return x; }
+template <typename T> GS_HD T here(T x) { return x; }
 template <typename T> GS_HD T min_w(T a, T b) { return vmin(a, b); }
 template <typename T> GS_HD T max_w(T a, T b) { return vmax(a, b); }
 template <typename T> GS_HD T min_abs_w(T a, T b) { return vmin(vabs(a), vabs(b)); }
@@ -301,7 +331,7 @@ GS_HD T root0_w(T x) {
 // ---------------------------------------------------------------------------
 template <typename T>
 struct WaveC {
-  T g, hg, hm, ix, iy, hdx, hdy, dt, dt2, vcap;
+  T g, hg, hm, ix, iy, hdx, hdy, dt, vcap;
   int flags;       // kWave*
   lmask not_wet;   // all lanes unless kWaveWet is set
 };
@@ -342,8 +372,7 @@ GS_HD WaveC<T> wave_consts(const Phys<T>& P, T dt, int flags) {
   w.hdx = vreg(P.half_dx);
   w.hdy = vreg(P.half_dy);
   w.dt = vreg(dt);
-  w.dt2 = vreg(T(2) * dt);
-  w.vcap = P.has_vcap ? P.vcap : T(INFINITY);
+  w.vcap = sreg(P.has_vcap ? P.vcap : T(INFINITY));
   w.flags = flags;
   w.not_wet = (flags & kWaveWet) ? lm_none() : lm_every();
   return w;
@@ -352,9 +381,9 @@ GS_HD WaveC<T> wave_consts(const Phys<T>& P, T dt, int flags) {
 // ---------------------------------------------------------------------------
 // primitive velocities of a row, its wet/dry mask and its sanity
 // ---------------------------------------------------------------------------
-// Lanes whose x is not 0 but too small for the short quotient.
+// Lanes where x or y is not 0 but too small for the short quotient.
 template <typename T>
-GS_HD lmask odd_num(T x, T y, lmask use) {
+GS_HD lmask tiny_num(T x, T y, lmask use) {
   lmask m = (lm_lt(vabs(x), Range<T>::num_tiny()) | lm_lt(vabs(y), Range<T>::num_tiny())) & use;
   if (lm_any(m))   // zeros (still water) are in order
     m = m & lm_of((x != T(0) && vabs(x) < Range<T>::num_tiny()) || (y != T(0) && vabs(y) < Range<T>::num_tiny()));
@@ -368,7 +397,7 @@ template <typename T>
 GS_HD void prims_w(T h, T hu, T hv, T b, lmask use, const WaveC<T>& w, T& u, T& v, lmask& dry, lmask& odd) {
   const lmask wet = lm_gt(h, w.hm);
   dry = lm_none();
-  odd = odd | odd_num<T>(hu, hv, use);
+  const lmask tiny = tiny_num<T>(hu, hv, use);
   if (!lm_any(lm_not(wet) & use)) {
     const T y = recip_w(h);
     u = quot_w(hu, h, y);
@@ -379,6 +408,15 @@ GS_HD void prims_w(T h, T hu, T hv, T b, lmask use, const WaveC<T>& w, T& u, T& 
     const T y = recip_w(hs);
     u = lm_sel(wet, quot_w(hu, hs, y), T(0));
     v = lm_sel(wet, quot_w(hv, hs, y), T(0));
+  }
+  if (lm_any(tiny)) {
+    // Momenta that friction has all but stopped: the division itself. Their rows must not go to the
+    // general functions: a few hundred of 36 000 window rows of a 2048^2 coastal domain hold one
+    // after 200 steps, and with all tiles in one round the slowest tile is the step (50.0 against
+    // 42.5 us).
+    const lmask wet1 = lm_gt(h, w.hm);
+    u = lm_sel(wet1, vdiv(here(hu), max_w(h, w.hm)), T(0));
+    v = lm_sel(wet1, vdiv(here(hv), max_w(h, w.hm)), T(0));
   }
   const T s = (vabs(u) + vabs(v)) + (vabs(b) + vabs(h)) * T(0x1p-10);
   odd = odd | (lm_not(lm_lt(s, T(1024))) & use);
@@ -519,6 +557,47 @@ GS_HD void face_w(T bL, T bR, T zL, T zhR, T hL, T hR, T uNL, T uTL, T uNR, T uT
   f.sR = sR * inv;
 }
 
+// The four faces of a cell in the reference's order. A face gated off (both cells dry) adds
+// zeros: the sums start at +0 and IEEE addition yields -0 only from two -0 terms, so they never
+// hold -0, and x + 0 = x - 0 = x for every other x.
+template <typename T>
+GS_HD void sum_faces(const FaceProd<T>& up, const FaceProd<T>& dn, const FaceProd<T>& right,
+                                          T lFh, T lFN, T lFT, T lsR, T& rh, T& rhu, T& rhv) {
+  rh = T(0); rhu = T(0); rhv = T(0);
+  rh = rh - up.Fh;
+  rhu = rhu - up.FN;
+  rhv = rhv - up.FT;
+  rhu = rhu - up.sL;
+  rh = rh + dn.Fh;
+  rhu = rhu + dn.FN;
+  rhv = rhv + dn.FT;
+  rhu = rhu + dn.sR;
+  rh = rh - right.Fh;
+  rhu = rhu - right.FT;
+  rhv = rhv - right.FN;
+  rhv = rhv - right.sL;
+  rh = rh + lFh;
+  rhu = rhu + lFT;
+  rhv = rhv + lFN;
+  rhv = rhv + lsR;
+}
+
+// face() as the products its cells add, zero where it is gated off.
+template <typename T>
+GS_HD void face_prod(T bL, T bR, T gzL, T gzR, T hL, T hR, T uNL, T uTL, T uNR, T uTR, T half,
+                                          T inv, T g, T hm, FaceProd<T>& f) {
+  Face<T> q;
+  face<T>(bL, bR, gzL, gzR, hL, hR, uNL, uTL, uNR, uTR, half, g, hm, q);
+  f.Fh = q.gate ? q.Fh * inv : T(0);
+  f.FN = q.gate ? q.FN * inv : T(0);
+  f.FT = q.gate ? q.FT * inv : T(0);
+  f.sL = q.gate ? q.srcL * inv : T(0);
+  f.sR = q.gate ? q.srcR * inv : T(0);
+}
+
+template <typename T>
+constexpr T kMaxSpeed = T(0x1p40);
+
 // ---------------------------------------------------------------------------
 // update
 // ---------------------------------------------------------------------------
@@ -548,15 +627,17 @@ GS_HD void update_w(T q0, T q1, T q2, T rr0, T r1, T r2, T n, lmask act, const P
     const T h43 = pow_m43(hs);
     const lmask fastw = lm_gt(modU, w.vcap) & live;
     if (lm_any(fastw)) {
-      const T n_cri = vsqrt(vdiv(T(1), (((T(1.0e-10) + w.dt) * P.g) * h43) * (modU + T(1.0e-30))));
+      const T n_cri = vsqrt(vdiv(T(1), (((T(1.0e-10) + here(w.dt)) * P.g) * h43) * (modU + T(1.0e-30))));
       n = lm_sel(fastw & lm_gt(n_cri, n), n_cri, n);
     }
     const T Cf = ((w.g * n) * n) * h43;
     const lmask creep = lm_lt(m2, Range<T>::root()) & live;
     T alpha, two;
     if (P.quadratic) {
-      two = (w.dt2 * Cf) * modU;
-      alpha = T(2) * recip_w(root_w(vfma(T(2), two, T(1))) + T(1));   // RN(2/d) = 2 RN(1/d)
+      // two = 2*dt*Cf*modU is 2*half, and alpha = 2 / (sqrt(1 + 2*two) + 1), where RN(2/d) = 2 RN(1/d)
+      const T half = (w.dt * Cf) * modU;
+      two = T(2) * half;
+      alpha = T(2) * recip_w(root_w(vfma(T(4), half, T(1))) + T(1));
     } else {
       two = (w.dt * Cf) * modU;
       alpha = recip_w(T(1) + two);
@@ -566,13 +647,22 @@ GS_HD void update_w(T q0, T q1, T q2, T rr0, T r1, T r2, T n, lmask act, const P
     hv = hv * alpha;
   }
   speed = quot_w(max_abs_w(hu, hv), hs, yh) + root_w(w.g * h);
-  odd = odd | (lm_not(lm_lt(speed, T(0x1p40))) & live);
+  odd = odd | (lm_not(lm_lt(speed, kMaxSpeed<T>)) & live);
   if (lm_any(dry & act)) {
     h = lm_sel(dry, P.keep_h ? pos_w(h) : T(0), h);
     hu = lm_sel(dry, T(0), hu);
     hv = lm_sel(dry, T(0), hv);
     speed = lm_sel(dry, T(0), speed);
   }
+}
+
+// The wave speed of a state that the update did not make (a stage, a forcing): the same expression.
+// Not below kMaxSpeed on a wet lane: one that this form does not serve.
+template <typename T>
+GS_HD T speed_w(T h, T hu, T hv, const WaveC<T>& w) {
+  const T hs = max_w(h, w.hm);
+  const T speed = quot_w(max_abs_w(hu, hv), hs, recip_w(hs)) + root_w(w.g * h);
+  return lm_sel(lm_lt(h, w.hm), T(0), speed);
 }
 
 #if defined(__HIPCC__)

@@ -14,6 +14,7 @@ are k+-1 and k+-2 by construction of the dilation.
 """
 from __future__ import annotations
 
+import math
 from dataclasses import dataclass
 
 import numpy as np
@@ -175,7 +176,8 @@ def _build_native(inside_padded: np.ndarray, ngh: int, ring: int, sweep_rows) ->
 
 
 WRITE_LANES = np.uint64(((1 << 62) - 1) & ~3)   # lanes 2..61 of a 64-lane sweep window
-TILE_TARGET = 8192   # tiles a domain should give at least (~1.5 resident wavefronts of an MI355X each)
+TILE_TARGET = 4608   # tiles a domain should give at least where its rows allow: 3/4 of the 6144 wavefronts
+                     # that an MI355X holds of the float32 sweep at once
 MAX_SWEEP_ROWS = 32  # tallest tile: each tile re-reads 4 stencil rows and re-evaluates one x-face row;
                      # on MI355X 32-row tiles run the 16384^2 coastal step 3-4 % faster than 64-row
                      # ones (twice the tiles, a shorter tail of the last round of wavefronts)
@@ -190,12 +192,16 @@ def _window_masks(m: np.ndarray, nwin: int) -> np.ndarray:
 
 
 def sweep_rows_for(busy: int) -> int:
-    """Tile height for `busy` window rows with an active lane: the largest power of two
-    <= MAX_SWEEP_ROWS that still gives about TILE_TARGET tiles."""
-    rows = 1
-    while rows < MAX_SWEEP_ROWS and int(busy) // (2 * rows) >= TILE_TARGET:
-        rows *= 2
-    return rows
+    """Tile height for `busy` window rows with an active lane: about sqrt(busy/1000), kept where it
+    gives TILE_TARGET to 2*TILE_TARGET tiles, at most MAX_SWEEP_ROWS.
+
+    A tile pays for a row and a half of lead-in, few tall tiles leave SIMDs idle. Coastal domains on
+    MI355X, us for 20 lean steps at heights 2/4/6/8/12/16: 21207 busy rows 841/699/661/743/844/1094,
+    36626 rows 1132/1017/865/960/1118/1260, 77431 rows (from 4) 1595/1537/1465/1533/1508; 139562 rows
+    2373 at 12, 2425 at 16, 2532 at 20; 300224 rows within 4 % from 10 to 32."""
+    busy = int(busy)
+    rows = max(math.isqrt(busy // 1000), busy // (2 * TILE_TARGET) + 1)
+    return max(1, min(rows, busy // TILE_TARGET, MAX_SWEEP_ROWS))
 
 
 def mesh_sweep_tiles(fm: "FlatMesh", rows: int):
@@ -225,10 +231,9 @@ def build_sweep_tiles(stored: np.ndarray, active: np.ndarray, rows: int = None):
     side), stored contiguously. Tiles are ordered band-major, so the tiles that run side by
     side read neighbouring columns of the same rows.
 
-    `rows=None` picks the tile height from the domain: the largest power of two <= 32 that
-    still gives about TILE_TARGET tiles of the column grid CHUNK*k, so that a small domain run
-    alone keeps every CU busy (a tile of r rows evaluates 1 + 1/r x-faces per row instead
-    of 2).
+    `rows=None` picks the tile height from the domain (sweep_rows_for, of its windows on the column
+    grid CHUNK*k), so that a small domain run alone keeps every CU busy (a tile of r rows evaluates
+    1 + 1/r x-faces per row instead of 2).
     """
     stored = np.asarray(stored, dtype=bool)
     active = np.asarray(active, dtype=bool)

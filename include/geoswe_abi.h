@@ -434,8 +434,9 @@ int gs_adj_flat_sweep(const GsAdjFlat* a, const GsPhys* phys, int n, const doubl
  * compressed_rhs.py:241-369) that CompressedSolver.from_dense (compressed_solver.py:2903-3124)
  * runs on the host. `inside` is the (nxp, nyp) active mask of the padded grid (row-major,
  * 0/1); the stored set is its `ring`-fold 4-neighbour dilation (ring >= 2), numbered
- * row-major. sweep_rows > 0 fixes the tile height; -1 picks the largest power of two <=
- * max_sweep_rows that still gives ~tile_target tiles. Host memory only, no device call.
+ * row-major. sweep_rows > 0 fixes the tile height; -1 picks it from the number of window rows with
+ * an active cell: about sqrt(rows/1000), kept where it gives tile_target to 2*tile_target tiles, at
+ * most max_sweep_rows. Host memory only, no device call.
  */
 int gs_flat_mesh_build(const uint8_t* inside, int nxp, int nyp, int ring, int sweep_rows, int tile_target,
                        int max_sweep_rows, GsFlatMeshHost* out);
@@ -460,7 +461,8 @@ int gs_ens_create(const GsFlat* members, const GsPhys* phys, const GsForcing* fo
                   GsClock* const* clocks, int n_members, GsEns** out);
 int gs_ens_destroy(GsEns* e);
 /* Launch shape: resident workgroups (0 = one full occupancy wave of the device) and the
- * consecutive row-sweep tiles a wavefront takes per pass (1..64). */
+ * consecutive row-sweep tiles a wavefront takes per pass (1..64). A new ensemble launches one
+ * wavefront per tile. */
 int gs_ens_set_launch(GsEns* e, int blocks, int tiles_per_pass);
 int gs_ens_get_launch(const GsEns* e, int* blocks, int* tiles_per_pass, int64_t* total_tiles);
 /* One step of every member that is not done. */

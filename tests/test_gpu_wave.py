@@ -74,3 +74,41 @@ def test_residual_and_steps_at_tile_edges(gpu, shape, rows, bc, odd):
         ref.step(dt)
     assert np.array_equal(s.q_interior, ref.q_interior)
     assert s._clockv().lam_bits == ref._clockv().lam_bits
+
+
+@pytest.mark.parametrize("odd", [False, True])
+@pytest.mark.parametrize("dtype", ["float32", "float64"])
+@pytest.mark.parametrize("ext,maxh", [(False, False), (False, True), (True, True)])
+@pytest.mark.parametrize("shape,rows", [((6, 5), 1), ((17, 61), 2), ((33, 124), 5), ((40, 130), 2000)])
+def test_flat_sweep_at_tile_edges(gpu, shape, rows, ext, maxh, dtype, odd):
+    """Three steps of the flat sweep (lean, plain and extended) give the chunk traversal's bits, at
+    tiles of one row and more, cut by an irregular mask, and a height (2000) that the wavefront
+    forms leave to the general functions whole; in rows with odd operands too."""
+    from geoswe_amd import CompressedSolver
+    nx, ny = shape
+    q, bed = _state(nx, ny, odd)
+    if odd and dtype == "float64":
+        q, bed = q.astype(np.float64), bed.astype(np.float64)
+        q[1, nx // 2, ny // 2] = 1.0e-300
+    rng = np.random.default_rng(nx + ny)
+    mask = rng.random((nx, ny)) > 0.06
+    mask[nx // 2, ny // 2] = True
+    cls = rng.integers(0, 3, (nx, ny)).astype(np.uint8)
+    out = []
+    for trav in ("tiles", "chunks"):
+        cfg = Config(bc_x="fall", bc_y="fall", dtype=dtype, friction="manning", manning_n=0.03,
+                     rainfall=20.0 / 3.6e6)
+        s = Solver2D(Mesh2D(nx, ny, 2.0, 2.0), cfg, q.astype(dtype), bed.astype(dtype))
+        s.set_inside_mask(mask)
+        c = CompressedSolver.from_dense(s, cfl_linf=True, track_max_depth=maxh, sweep_rows=rows)
+        if ext:
+            g = s.mesh.ngh
+            c.set_ga_drain({"cls_pad": np.pad(cls, g), "Ks_t": [0.0, 1e-5, 4e-5], "psi_t": [0.1, 0.1, 0.2],
+                            "dth_t": [0.3, 0.3, 0.3], "F_pad": None,
+                            "inv_tau_pad": np.full((nx + 2 * g, ny + 2 * g), 1.0 / 600.0), "mode": "fused"})
+        c.traversal = trav
+        c.advance(3)
+        out.append((c.q_flat(), c.t, c.nsteps, c.max_depth() if maxh else None))
+    a, b = out
+    assert a[1:3] == b[1:3] and np.array_equal(a[0], b[0])
+    assert not maxh or np.array_equal(a[3], b[3])

@@ -8,6 +8,7 @@ import shutil
 import subprocess
 from pathlib import Path
 
+import numpy as np
 import pytest
 
 NATIVE = Path(__file__).resolve().parent / "native"
@@ -24,3 +25,20 @@ def test_wave_forms_equal_general(tmp_path):
     print(r.stdout)
     assert r.returncode == 0, r.stdout + r.stderr
     assert "mismatches 0" in r.stdout
+
+
+@pytest.mark.parametrize("target", [1, 3, 7, 500, 4608])
+def test_tile_height_rule_native_equals_python(monkeypatch, target):
+    """The native mesh builder and the Python one pick the same tile height, where the square root
+    decides (4000 to 12000 window rows) and at both clamps."""
+    import geoswe_amd.flatmesh as FM
+    monkeypatch.setattr(FM, "TILE_TARGET", target)
+    for nx, ny in ((3, 61), (40, 121), (700, 400), (1000, 720)):
+        inside = np.zeros((nx + 8, ny + 8), bool)
+        inside[4:-4, 4:-4] = True
+        a = FM.build_flat_mesh(inside, 4, native=True)
+        b = FM.build_flat_mesh(inside, 4, native=False)
+        assert np.array_equal(a.tile_irc, b.tile_irc) and np.array_equal(a.tile_e0, b.tile_e0)
+        rows = FM.sweep_rows_for(nx * ((ny + 1) // 60 + 1))   # windows of the column grid that the rows touch
+        tall = int(a.tile_irc[:, 1].max())
+        assert tall == rows if nx > 2 * rows else tall <= rows    # bands are trimmed to the active rows
