@@ -969,7 +969,7 @@ __global__ __launch_bounds__(kFBlock) void k_flat_step(FlatK<T> a) {
   for (int64_t chunk = (int64_t)xcd_rank(blockIdx.x, gridDim.x) * (kFBlock / 64) + (threadIdx.x >> 6);
        chunk < a.nchunks; chunk += nwaves)
     flat_chunk<T, MODE>(x, chunk, lane, lam);
-  if (MODE == 1) grid_reduce_and_plan(lam_key_bits64(lam), a.clock, a.plan, true);
+  if (MODE == 1) grid_reduce_and_plan(lam, a.clock, a.plan, true);
 }
 
 // One step of one flat domain by row-sweep tiles, one wavefront per tile in band-major tile
@@ -999,7 +999,7 @@ __global__ __launch_bounds__(kSBlock<T>) __attribute__((amdgpu_waves_per_eu(size
   // replay reads rain through the per-cell lookup exactly as the forward run's extended sweep
   for (int64_t t = (int64_t)xcd_rank(blockIdx.x, gridDim.x) * kSweepWaves<T> + wv; t < a.n_tiles; t += nwaves)
     flat_tile<T, PRE, PRE, LEAN>(x, t, lane, lam);
-  grid_reduce_and_plan(lam_key_bits64(lam), a.clock, a.plan, true);
+  grid_reduce_and_plan(lam, a.clock, a.plan, true);
 }
 
 // The sweep with the extended forcings compiled in: Green-Ampt infiltration, drain-tau and
@@ -1022,7 +1022,7 @@ __global__ __launch_bounds__(kSBlock<T>) __attribute__((amdgpu_waves_per_eu(size
   lam_t<T> lam = 0;
   for (int64_t t = (int64_t)xcd_rank(blockIdx.x, gridDim.x) * kSweepWaves<T> + wv; t < a.n_tiles; t += nwaves)
     flat_tile<T, false, true>(x, t, lane, lam);
-  grid_reduce_and_plan(lam_key_bits64(lam), a.clock, a.plan, true);
+  grid_reduce_and_plan(lam, a.clock, a.plan, true);
 }
 
 // The forcings on the ring cells of the band (stored, not active): out = force(in), one
@@ -1144,7 +1144,7 @@ __global__ __launch_bounds__(kFBlock) void k_flat_cfl(FlatK<T> a) {
       lam = l > lam ? l : lam;
     }
   }
-  grid_reduce_and_plan(lam_key_bits64(lam), a.clock, a.plan, false);
+  grid_reduce_and_plan(lam, a.clock, a.plan, false);
 }
 
 template <typename T>
@@ -1416,10 +1416,10 @@ struct EnsK {
 // Fold a wavefront's CFL speed bits of member m into that member's clock (lane 0 waits
 // until its atomic has been performed, as grid_reduce_and_plan's thread 0 does).
 template <typename T>
-__device__ __forceinline__ void ens_flush(const EnsK<T>& e, int m, uint64_t lam) {
-  lam = wave_max_u64(lam);
+__device__ __forceinline__ void ens_flush(const EnsK<T>& e, int m, lam_t<T> lam) {
+  lam = wave_max(lam);
   if (m >= 0 && (threadIdx.x & 63) == 0 && lam)
-    await_atomic(__hip_atomic_fetch_max(&e.mem[m].clock->lam_acc, lam, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    await_atomic(__hip_atomic_fetch_max(&e.mem[m].clock->lam_acc, lam_key_bits64(lam), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
 }
 
 // The member that owns global tile gc (tile0: the members' tile prefix, n + 1 entries).
@@ -1471,7 +1471,7 @@ void k_ens_step(EnsK<T> e, const FlatK<T>* __restrict__ mem, const int64_t* __re
       // them is held across tiles
       const int mt = ens_member_of(tile0, e.n_members, gc);
       if (mt != m) {
-        ens_flush(e, m, lam_key_bits64(lam));
+        ens_flush(e, m, lam);
         lam = 0;
         m = mt;
         const T* nt = const_read(&mem[mt].ntab);
@@ -1490,7 +1490,7 @@ void k_ens_step(EnsK<T> e, const FlatK<T>* __restrict__ mem, const int64_t* __re
   __shared__ int s_m[kFBlock / 64];
   __shared__ uint64_t s_l[kFBlock / 64];
   __shared__ int s_last;
-  const uint64_t lw = wave_max_u64(lam_key_bits64(lam));
+  const uint64_t lw = lam_key_bits64(wave_max(lam));
   if (lane == 0) {
     s_m[wv] = m;
     s_l[wv] = lw;
@@ -1514,9 +1514,9 @@ void k_ens_step(EnsK<T> e, const FlatK<T>* __restrict__ mem, const int64_t* __re
   if (!s_last) return;
   for (int mm = threadIdx.x; mm < e.n_members; mm += blockDim.x) {
     GsClock* c = e.mem[mm].clock;
-    if (c->status & GS_ST_DONE) continue;
-    const uint64_t tot = __hip_atomic_load(&c->lam_acc, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT);
-    plan_finish(c, e.mem[mm].plan, tot, true);
+    const ClockIn k = clock_read(c);
+    if (k.status & GS_ST_DONE) continue;
+    plan_finish(c, e.mem[mm].plan, k, true);
   }
   if (threadIdx.x == 0) __hip_atomic_store(e.done, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }

@@ -55,17 +55,23 @@ __global__ void k_clock_target(GsClock* c, Plan p, double t_end, double dt_max, 
   c->max_steps = max_steps < 0 ? INT64_MAX : c->nsteps + max_steps;
   c->run_mode = run_mode;
   c->status &= ~GS_ST_DONE;
-  plan_dt(c, p);
+  const ClockIn k = clock_read(c);
+  ForcIn f;
+  forcing_read(p, k.t, f);
+  plan_dt(c, p, k, f, c->lam_bits);
 }
 
 __global__ void k_clock_dt(GsClock* c, Plan p, double dt) {
+  const ClockIn k = clock_read(c);
+  ForcIn f;
+  forcing_read(p, k.t, f);
   c->dt = dt;
   c->dt32 = (float)dt;
   c->use_host_dt = 1;
-  c->status &= ~GS_ST_DONE;
-  if (c->status & GS_ST_NONFINITE) c->status |= GS_ST_DONE;
-  if (c->nsteps >= c->max_steps) c->status |= GS_ST_DONE;
-  plan_forcing(c, p);
+  int st = k.status & ~GS_ST_DONE;
+  if ((st & GS_ST_NONFINITE) || k.nsteps >= k.max_steps) st |= GS_ST_DONE;
+  c->status = st;
+  plan_forcing(c, p, f, k.t, dt);
 }
 
 
@@ -530,7 +536,7 @@ void k_dense_sweep(DenseK<T, S> a) {
     }
     if (i < i_end) dense_rows_general<T, MODE, LEAN, S, O>(a, x, dt, i, i_end, lam);
   }
-  if (MODE == 1) grid_reduce_and_plan(lam_key_bits64(lam), a.clock, a.plan, true);
+  if (MODE == 1) grid_reduce_and_plan(lam, a.clock, a.plan, true);
 }
 
 // CFL wave speed of the current dense state, then plan dt (no time advance).
@@ -548,7 +554,7 @@ __global__ __launch_bounds__(256) void k_dense_cfl(DenseK<T, S> a) {
     const lam_t<T> l = lam_key<T>((T)q[0][idx], (T)q[1][idx], (T)q[2][idx], a.P);
     lam = l > lam ? l : lam;
   }
-  grid_reduce_and_plan(lam_key_bits64(lam), a.clock, a.plan, false);
+  grid_reduce_and_plan(lam, a.clock, a.plan, false);
 }
 
 // Rows per tile. A tile costs about 1.3 rows beside its own (the rows above it, the first x-face),
