@@ -138,6 +138,7 @@ _SIGS = {
                                 C.POINTER(_P)]),
     "gs_ens_destroy": (C.c_int, [_P]),
     "gs_ens_set_launch": (C.c_int, [_P, C.c_int, C.c_int]),
+    "gs_ens_status": (C.c_int, [_P, C.POINTER(C.c_int), _P]),
     "gs_ens_get_launch": (C.c_int, [_P, C.POINTER(C.c_int), C.POINTER(C.c_int), C.POINTER(C.c_int64)]),
     "gs_ens_step": (C.c_int, [_P, _P]),
     "gs_ens_run": (C.c_int, [_P, C.c_int64, C.c_int, _P]),
@@ -326,6 +327,14 @@ def read_clock(dev: DeviceArray, stream=None) -> GsClock:
     c = GsClock()
     C.memmove(C.byref(c), raw.ctypes.data, C.sizeof(GsClock))
     return c
+
+
+def run_batch(c: GsClock, batch: int) -> int:
+    """Steps to launch before the next look at a running clock: what its dt makes to t_end, and some
+    for a dt that shrinks, at most ``batch`` (a launch after the end costs the device a few us)."""
+    if c.dt > 0.0 and c.t_end - c.t < c.dt * batch:
+        return max(1, min(batch, int((c.t_end - c.t) / c.dt * 1.125) + 2))
+    return batch
 
 
 def new_clock(t0: float = 0.0, stream=None) -> DeviceArray:

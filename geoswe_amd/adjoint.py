@@ -181,6 +181,11 @@ class GaugeMisfit:
     def gradient(self):
         """(dJ/dn per class (n_classes,), dJ/dbed (N,)) at the parameters of the last
         simulate() (float64 host arrays). Leaves the solver at the initial state and time."""
+        self._reverse()
+        return self._ws["nbar"].download()[:self.n_classes].copy(), self._ws["bbar"].download()
+
+    def _reverse(self) -> None:
+        """The reverse pass: the gradients are left in the workspace (float64 nbar and bbar)."""
         if self.samples is None:
             raise RuntimeError("gradient: call simulate() first")
         s, N, K, S = self.s, self.N, self.K, self.S
@@ -198,11 +203,21 @@ class GaugeMisfit:
                 gz=L.DeviceArray((2, 2, N), dt_),          # double-buffered bed-gradient cotangents
                 bbar=L.DeviceArray((N,), np.float64), nbar=L.DeviceArray((L.MAX_CLASSES,), np.float64),
                 npart=L.DeviceArray((nblk, 32), np.float64))
+            ws = self._ws
+            # what the reverse steps never write: the slots of faces beside no active cell and the
+            # cotangents of inactive cells are zero; the step writes only active cells, and the ring
+            # cells of every state of the segment store are frozen at their initial values
+            for arr in ws["w"] + [ws["xf"], ws["yf"]]:
+                L.call("gs_memset", C.c_void_p(arr.ptr), 0, C.c_size_t(arr.nbytes), None)
+            for st_ in ws["seg_states"]:
+                for m in range(3):
+                    L.call("gs_memcpy_d2d", C.c_void_p(st_[m].ptr), C.c_void_p(self._q0[m].ptr),
+                           C.c_size_t(self._q0[m].nbytes), None)
         ws = self._ws
         seg_states, seg_pre = ws["seg_states"], ws["seg_pre"]
         lam, w, xf, yf, gz = ws["lam"], ws["w"], ws["xf"], ws["yf"], ws["gz"]
         bbar, nbar, npart = ws["bbar"], ws["nbar"], ws["npart"]
-        for arr in lam + w + [xf, yf, gz, bbar, nbar, npart]:   # accumulators and scratch start at zero
+        for arr in lam + [gz, bbar, nbar, npart]:   # accumulators start at zero
             L.call("gs_memset", C.c_void_p(arr.ptr), 0, C.c_size_t(arr.nbytes), None)
         coef = (2.0 * (self.samples - self.h_star)).astype(dt_)          # (S, G): dJ/dh_s at gauges
         d_coef = L.DeviceArray.from_host(coef)
@@ -224,12 +239,6 @@ class GaugeMisfit:
         L.call("gs_adj_add", C.c_void_p(lam[0].ptr), dcode, C.c_void_p(self._d_gauges.ptr),
                C.c_void_p(d_coef.ptr + (S - 1) * G * es), G, None)
         nbytes = self._q0[0].nbytes
-        # every slot of the segment store starts as the initial state: the step writes only
-        # active cells, and the ring cells are frozen at their initial values
-        for st_ in seg_states:
-            for m in range(3):
-                L.call("gs_memcpy_d2d", C.c_void_p(st_[m].ptr), C.c_void_p(self._q0[m].ptr), C.c_size_t(nbytes),
-                       None)
         state_ptrs = (C.c_void_p * (3 * (K + 1)))(*[x[m].ptr for x in seg_states for m in range(3)])
         pre_ptrs = (C.c_void_p * (3 * K))(*[x[m].ptr for x in seg_pre for m in range(3)])
         for seg in range(nseg - 1, -1, -1):
@@ -255,7 +264,6 @@ class GaugeMisfit:
         # leave the solver at the initial state and time (the replay moved its clock)
         self._reset(self._q0, self.t0)
         L.sync(None)
-        return nbar.download()[:self.n_classes].copy(), bbar.download().copy()
 
 
 try:
@@ -267,7 +275,8 @@ try:
 
         @staticmethod
         def forward(ctx, ntab, bed, problem):
-            problem.set_params(ntab.detach().cpu().double().numpy(), bed.detach().cpu().double().numpy())
+            problem.set_params(ntab.detach().cpu().double().numpy(), None)
+            _bed_from_tensor(problem, bed.detach())
             problem.simulate()
             ctx.problem = problem
             ctx.dev = (ntab.device, bed.device)
@@ -275,9 +284,37 @@ try:
 
         @staticmethod
         def backward(ctx, g):
-            gn, gb = ctx.problem.gradient()
+            problem = ctx.problem
+            problem._reverse()
             gs = float(g)
-            return (torch.as_tensor(gn * gs, device=ctx.dev[0]), torch.as_tensor(gb * gs, device=ctx.dev[1]),
-                    None)
+            gn = problem._ws["nbar"].download()[:problem.n_classes]
+            return (torch.as_tensor(gn * gs, device=ctx.dev[0]), _bed_gradient_tensor(problem, ctx.dev[1]) * gs, None)
+
+    def _on_solver_device(device) -> bool:
+        return device.type == "cuda" and device.index == torch.cuda.current_device()
+
+    def _bed_from_tensor(problem, bed) -> None:
+        """set_params(bed=...) of a torch tensor, on the device if it is there already (the host's
+        way took 1.2 M cells through pageable memory in 1.2 ms)."""
+        if not _on_solver_device(bed.device):
+            return problem.set_params(None, bed.cpu().double().numpy())
+        if bed.numel() != problem.N:
+            raise ValueError(f"bed has {bed.numel()} entries, the flat mesh {problem.N}")
+        t = torch.float32 if problem.dtype == np.float32 else torch.float64
+        src = bed.double().to(t).contiguous()
+        dst = problem.s._bed
+        torch.cuda.current_stream().synchronize()     # the copy below is on the solver's stream
+        L.call("gs_memcpy_d2d", C.c_void_p(dst.ptr), C.c_void_p(src.data_ptr()), C.c_size_t(dst.nbytes), None)
+        L.sync(None)                                  # before src may be reused
+
+    def _bed_gradient_tensor(problem, device):
+        bbar = problem._ws["bbar"]
+        if not _on_solver_device(device):
+            return torch.as_tensor(bbar.download(), device=device)
+        out = torch.empty(problem.N, dtype=torch.float64, device=device)
+        torch.cuda.current_stream().synchronize()     # whatever used out's memory before
+        L.call("gs_memcpy_d2d", C.c_void_p(out.data_ptr()), C.c_void_p(bbar.ptr), C.c_size_t(bbar.nbytes), None)
+        L.sync(None)
+        return out
 except ImportError:     # torch is optional for the solver path
     GaugeMisfitFn = None

@@ -756,7 +756,8 @@ class CompressedSolver:
             if c.t >= next_ckpt:
                 self.save_checkpoint(ckpt_dir, fidx, next_frame if frames_on else None)
                 next_ckpt = c.t + checkpoint_every_s
-            for _ in range(batch):
+            # checkpoints are due at looks of every `batch` steps
+            for _ in range(batch if checkpoint_every_s else L.run_batch(c, batch)):
                 L.call("gs_flat_step", d, p, self._fo.s, clk, self.stream)
             self._any_step = True
         c = self._clockv()

@@ -1451,6 +1451,12 @@ __device__ __forceinline__ int ens_member_of(const int64_t* tile0, int n, int64_
 // 8 rows a tile against 84).
 enum { kEnsPlain = 0, kEnsExt = 1, kEnsLean = 2 };
 
+// The members' clock statuses side by side, for one copy to the host.
+template <typename T>
+__global__ void k_ens_status(const FlatK<T>* mem, int n, int* out) {
+  for (int m = blockIdx.x * blockDim.x + threadIdx.x; m < n; m += gridDim.x * blockDim.x) out[m] = mem[m].clock->status;
+}
+
 template <typename T, int KIND>
 __global__ __launch_bounds__(kFBlock) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && KIND == kEnsLean ? 5 : 1)))
 void k_ens_step(EnsK<T> e, const FlatK<T>* __restrict__ mem, const int64_t* __restrict__ tile0) {
@@ -1651,7 +1657,7 @@ struct GsEns {
   int n = 0;
   void* mem = nullptr;          // device FlatK<T>[n]
   int64_t* tile0 = nullptr;     // device [n + 1]
-  unsigned* done = nullptr;     // device counter
+  unsigned* done = nullptr;     // device counter; the members' statuses (gs_ens_status) from byte 256
   int64_t ntiles = 0;
   int blocks = 0;               // 0: one occupancy wave of the device
   int tpp = 1;
@@ -1714,7 +1720,7 @@ static int ens_build_views(GsEns* e, const GsFlat* members, const GsPhys* phys, 
   e->blocks = (int)(per_tile < (1 << 24) ? per_tile : (1 << 24));
   GS_HIP(hipMalloc(&e->mem, sizeof(FlatK<T>) * (size_t)e->n), "ensemble views");
   GS_HIP(hipMalloc((void**)&e->tile0, sizeof(int64_t) * ((size_t)e->n + 1)), "ensemble tile table");
-  GS_HIP(hipMalloc((void**)&e->done, 256), "ensemble counter");
+  GS_HIP(hipMalloc((void**)&e->done, 256 + 4 * (size_t)e->n), "ensemble counter");
   GS_HIP(hipMemcpy(e->mem, views.data(), sizeof(FlatK<T>) * (size_t)e->n, hipMemcpyHostToDevice), "views h2d");
   GS_HIP(hipMemcpy(e->tile0, c0.data(), sizeof(int64_t) * ((size_t)e->n + 1), hipMemcpyHostToDevice),
          "tile table h2d");
@@ -1810,6 +1816,19 @@ int gs_ens_create(const GsFlat* members, const GsPhys* phys, const GsForcing* fo
   return GS_OK;
 }
 
+int gs_ens_status(GsEns* e, int* status, void* stream) {
+  using namespace gs;
+  if (!e || !status) return fail(GS_E_ARG, "gs_ens_status: NULL argument");
+  hipStream_t s = (hipStream_t)stream;
+  int* d = (int*)((char*)e->done + 256);
+  const dim3 grid((unsigned)((e->n + 63) / 64)), block(64);
+  if (e->dtype == GS_F64) hipLaunchKernelGGL(k_ens_status<double>, grid, block, 0, s, (const FlatK<double>*)e->mem, e->n, d);
+  else hipLaunchKernelGGL(k_ens_status<float>, grid, block, 0, s, (const FlatK<float>*)e->mem, e->n, d);
+  GS_HIP(hipGetLastError(), "k_ens_status launch");
+  GS_HIP(hipMemcpyAsync(status, d, sizeof(int) * (size_t)e->n, hipMemcpyDeviceToHost, s), "ensemble status d2h");
+  GS_HIP(hipStreamSynchronize(s), "ensemble status");
+  return GS_OK;
+}
 int gs_ens_destroy(GsEns* e) {
   if (!e) return GS_OK;
   gs::ens_drop_graph(e);

@@ -603,7 +603,7 @@ class Solver2D:
                 self._raise_if_bad(c)
                 if c.status & L.ST_DONE:
                     break
-                for _ in range(batch):
+                for _ in range(L.run_batch(c, batch)):
                     L.call("gs_dense_step", d, p, self._fo.s, clk, self.stream)
                 self._any_step = True
         self._target = None

@@ -465,6 +465,9 @@ int gs_ens_destroy(GsEns* e);
  * wavefront per tile. */
 int gs_ens_set_launch(GsEns* e, int blocks, int tiles_per_pass);
 int gs_ens_get_launch(const GsEns* e, int* blocks, int* tiles_per_pass, int64_t* total_tiles);
+/* Every member's clock status (GS_ST_*) into status[n_members], after the work before it on the
+ * stream; returns when they are there. */
+int gs_ens_status(GsEns* e, int* status, void* stream);
 /* One step of every member that is not done. */
 int gs_ens_step(GsEns* e, void* stream);
 /* nsteps steps; graph_batch > 0 replays a captured hipGraph of graph_batch steps. */
