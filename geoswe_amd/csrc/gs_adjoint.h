@@ -25,6 +25,14 @@ GS_HD T rdiv(T a, T b) {
   return a / b;
 }
 
+// The recomputed forward's correctly rounded operations. Another form of them (same results) is a
+// parameter of the face's reverse; div's `used` says whether the lane needs its quotient.
+template <typename T>
+struct ForwardOps {
+  GS_HD static T sqrt(T x) { return vsqrt(x); }
+  GS_HD static T div(T a, T b, bool) { return vdiv(a, b); }
+};
+
 // Cotangents of the 10 face inputs.
 template <typename T>
 struct FaceGrad {
@@ -33,13 +41,13 @@ struct FaceGrad {
 
 // Reverse of hllc(): given cotangents of (Fh, FN, FT), ACCUMULATES into the six input
 // cotangents.
-template <typename T>
+template <typename T, typename Ops = ForwardOps<T>>
 GS_HD void hllc_vjp(T hL, T uNL, T uTL, T hR, T uNR, T uTR, T g, T h_min, T bFh, T bFN, T bFT, T& ghL,
                     T& guNL, T& guTL, T& ghR, T& guNR, T& guTR) {
   const T z = T(0);
   // ---- forward (as hllc)
-  const T aL = vsqrt(g * (hL > z ? hL : z));
-  const T aR = vsqrt(g * (hR > z ? hR : z));
+  const T aL = Ops::sqrt(g * (hL > z ? hL : z));
+  const T aR = Ops::sqrt(g * (hR > z ? hR : z));
   const T u_st = (T(0.5) * (uNL + uNR) + aL) - aR;
   const T h_rt = T(0.5) * (aL + aR) + T(0.25) * (uNL - uNR);
   const T a_st = (h_rt > z) ? h_rt : z;
@@ -55,7 +63,8 @@ GS_HD void hllc_vjp(T hL, T uNL, T uTL, T hR, T uNR, T uTR, T g, T h_min, T bFh,
   if (both) { SL = z; SR = z; }
   const T denom = hR * (uNR - SR) - hL * (uNL - SL);
   const bool big = vabs(denom) > T(1.0e-14);
-  const T SM = big ? vdiv((SL * hR) * (uNR - SR) - (SR * hL) * (uNL - SL), denom) : T(0.5) * (uNL + uNR);
+  const T SMq = Ops::div((SL * hR) * (uNR - SR) - (SR * hL) * (uNL - SL), denom, big);
+  const T SM = big ? SMq : T(0.5) * (uNL + uNR);
   int br;   // 0 left flux, 1 right flux, 2 left star, 3 right star
   if (SL >= z) br = 0;
   else if (!(SM >= z) && !(SR >= z)) br = 1;
@@ -149,7 +158,7 @@ GS_HD void hllc_vjp(T hL, T uNL, T uTL, T hR, T uNR, T uTR, T g, T h_min, T bFh,
 
 // Reverse of face(): cotangents of (Fh, FN, FT, srcL, srcR) -> cotangents of the 10
 // inputs (overwritten). The gate is not differentiated (a dry face contributes nothing).
-template <typename T>
+template <typename T, typename Ops = ForwardOps<T>>
 GS_HD void face_vjp(T bL, T bR, T gzL, T gzR, T hL, T hR, T uNL, T uTL, T uNR, T uTR, T half_d, T g, T h_min,
                     T bFh, T bFN, T bFT, T bsL, T bsR, FaceGrad<T>& G) {
   const T z = T(0);
@@ -217,7 +226,7 @@ GS_HD void face_vjp(T bL, T bR, T gzL, T gzR, T hL, T hR, T uNL, T uTL, T uNR, T
   gzf0 += gheadL;
   ghL -= gheadL;
   // flux
-  hllc_vjp<T>(hLf, uNL, uTL, hRf, uNR, uTR, g, h_min, bFh, bFN, bFT, ghLf, guNL, guTL, ghRf, guNR, guTR);
+  hllc_vjp<T, Ops>(hLf, uNL, uTL, hRf, uNR, uTR, g, h_min, bFh, bFN, bFT, ghLf, guNL, guTL, ghRf, guNR, guTR);
   // face depths
   const T gR_ = (aRf > z) ? ghRf : z, gL_ = (aLf > z) ? ghLf : z;
   getaR += gR_;
@@ -256,11 +265,11 @@ GS_HD void face_vjp(T bL, T bR, T gzL, T gzR, T hL, T hR, T uNL, T uTL, T uNR, T
   G.uTR = guTR;
 }
 
-// Reverse of prims(): cotangents of (u, v) ACCUMULATED into those of (h, hu, hv).
+// Reverse of prims() with its results u and v: cotangents of (u, v) ACCUMULATED into those of
+// (h, hu, hv).
 template <typename T>
-GS_HD void prims_vjp(T h, T hu, T hv, T h_min, T gu, T gv, T& gh, T& ghu, T& ghv) {
+GS_HD void prims_vjp(T h, T u, T v, T h_min, T gu, T gv, T& gh, T& ghu, T& ghv) {
   if (!(h > h_min)) return;
-  const T u = vdiv(hu, h), v = vdiv(hv, h);
   ghu += rdiv(gu, h);
   ghv += rdiv(gv, h);
   gh -= rdiv(gu * u + gv * v, h);

@@ -8,17 +8,18 @@
 //      pre-friction state -> w = cotangent of (h1, hu1, hv1); residual cotangent is dt*w;
 //      Manning n per class (workgroup sums, one atomic per class and workgroup);
 //      stage cells pass -cot(h) to their bed where eta - b > 0.
-//   B  per face, each face once: reverse of face() + prims() from the residual
-//      cotangents of its two cells; 10 numbers into the face's slot, indexed by its lower
-//      cell (x: (c, i+1), y: (c, j+1)). An active cell owns its upper faces and its lower
-//      faces whose lower cell is not active.
-//   C  per stored cell: cotangent of q_s = w + the four face slots touching the cell; bed
+//   B  per stored cell c, its upper faces along x and y (each face once): reverse of face() +
+//      prims() from the residual cotangents of the two cells. What the faces give to c itself is
+//      summed with w at once; what they give to the upper cells (5 numbers each) goes into slots
+//      indexed by c.
+//   C  per stored cell: cotangent of q_s = the sum of B + the slots of its two lower faces; bed
 //      cotangent from the faces' direct terms; the cell's bed-gradient cotangents.
 //   D  per stored cell: bed cotangent through the central bed gradients of its four
 //      neighbours, gz_X = 0.5*(b_{X+1} - b_{X-1})*inv_d.
 // The arithmetic is gs_adjoint.h's (checked against finite differences on the CPU).
 #include "gs_common.h"
 #include "gs_adjoint.h"
+#include "gs_wave.h"
 
 namespace gs {
 
@@ -39,8 +40,9 @@ struct AdjK {
   const T* pre[3];
   T* lam[3];
   T* w[3];
-  T* xf;                  // [10][n]
-  T* yf;                  // [10][n]
+  T* xf;                  // [10][n]: 0-2 w + own parts (h, hu, hv), 3 own bed, 4 own gz_x, 5-9 the upper
+                          // cell's parts of the x-face (h, hu, hv, bed, gz)
+  T* yf;                  // [10][n]: 4 own gz_y, 5-9 the upper cell's parts of the y-face
   T* gz;                  // [2][n]
   const T* gz_prev;       // [2][n] of the previous reverse step, or NULL
   double* bbar;
@@ -122,115 +124,163 @@ __global__ __launch_bounds__(64) void k_adj_nsum(const double* npart, int nblock
   if (threadIdx.x == 0 && k < n_classes) nbar[k] += v;
 }
 
-// Reverse of one face (L, R) along x (axis 0) or y (axis 1) into slot L of `slots`.
+// The forward's operations in the wavefront forms (gs_wave.h), the same bits: a wavefront with an
+// operand outside their bounds divides or takes the root itself.
 template <typename T>
-__device__ __forceinline__ void face_slot(const AdjK<T>& a, int axis, int64_t L, int64_t R, T* slots) {
-  const T hm = a.P.h_min, g = a.P.g;
-  const T inv = axis == 0 ? a.P.inv_dx : a.P.inv_dy;
-  const T half = axis == 0 ? a.P.half_dx : a.P.half_dy;
-  const int up = axis == 0 ? 0 : 2, dn = axis == 0 ? 1 : 3;
-  const int64_t n = a.n;
-  const T hL = a.q[0][L], huL = a.q[1][L], hvL = a.q[2][L];
-  const T hR = a.q[0][R], huR = a.q[1][R], hvR = a.q[2][R];
-  T* s = slots + L;
-  if (hL < hm && hR < hm) {   // dry face: no contribution either way
-    for (int k = 0; k < 10; ++k) s[k * n] = T(0);
-    return;
+struct WaveOps {
+  __device__ __forceinline__ static T sqrt(T x) {   // x >= 0 or NaN
+    T r = root0_w(x);
+    if (lm_any(lm_of((x > T(0) && x < Range<T>::root()) || !(x < Range<T>::hi())))) r = vsqrt(here(x));
+    return r;
   }
-  const T bL = a.bed[L], bR = a.bed[R];
-  // the cells either side of L and R along the axis are stored for every face of an
-  // active cell (ring-2 set, checked when the table is built); clamp all the same
-  const int32_t* nl = a.nbr + 4 * L;
-  const int32_t* nr = a.nbr + 4 * R;
-  const int64_t lu = nl[up] >= 0 ? nl[up] : L, ld = nl[dn] >= 0 ? nl[dn] : L;
-  const int64_t ru = nr[up] >= 0 ? nr[up] : R, rd = nr[dn] >= 0 ? nr[dn] : R;
-  const T gzL = (T(0.5) * (a.bed[lu] - a.bed[ld])) * inv;
-  const T gzR = (T(0.5) * (a.bed[ru] - a.bed[rd])) * inv;
-  T uL, vL, uR, vR;
-  prims(hL, huL, hvL, hm, uL, vL);
-  prims(hR, huR, hvR, hm, uR, vR);
-  // residual cotangents dt*w of both cells (zero outside active non-stage cells)
-  const T dt = a.dt;
-  const T rhL = dt * a.w[0][L], ruL = dt * a.w[1][L], rvL = dt * a.w[2][L];
-  const T rhR = dt * a.w[0][R], ruR = dt * a.w[1][R], rvR = dt * a.w[2][R];
-  FaceGrad<T> G;
-  if (axis == 0) {
-    face_vjp<T>(bL, bR, gzL, gzR, hL, hR, uL, vL, uR, vR, half, g, hm, inv * (rhR - rhL), inv * (ruR - ruL),
-                inv * (rvR - rvL), -(inv * ruL), inv * ruR, G);
-  } else {
-    face_vjp<T>(bL, bR, gzL, gzR, hL, hR, vL, uL, vR, uR, half, g, hm, inv * (rhR - rhL), inv * (rvR - rvL),
-                inv * (ruR - ruL), -(inv * rvL), inv * rvR, G);
+  __device__ __forceinline__ static bool sane(T a, T b) {
+    const T m = vabs(a), d = vabs(b);
+    return (a == T(0) || (m >= Range<T>::num_tiny() && m < Range<T>::hi())) && d > small() && d < T(1) / small();
   }
-  T ghL = G.hL, ghuL = T(0), ghvL = T(0), ghR = G.hR, ghuR = T(0), ghvR = T(0);
-  if (axis == 0) {
-    prims_vjp<T>(hL, huL, hvL, hm, G.uNL, G.uTL, ghL, ghuL, ghvL);
-    prims_vjp<T>(hR, huR, hvR, hm, G.uNR, G.uTR, ghR, ghuR, ghvR);
-  } else {
-    prims_vjp<T>(hL, huL, hvL, hm, G.uTL, G.uNL, ghL, ghuL, ghvL);
-    prims_vjp<T>(hR, huR, hvR, hm, G.uTR, G.uNR, ghR, ghuR, ghvR);
+  __device__ __forceinline__ static T div(T a, T b, bool used) {
+    T q = quot_w(a, b, recip_w(b));
+    if (lm_any(lm_of(used && !sane(a, b)))) q = vdiv(here(a), b);
+    return q;
   }
-  s[0] = ghL;
-  s[n] = ghuL;
-  s[2 * n] = ghvL;
-  s[3 * n] = G.bL;
-  s[4 * n] = G.gzL;
-  s[5 * n] = ghR;
-  s[6 * n] = ghuR;
-  s[7 * n] = ghvR;
-  s[8 * n] = G.bR;
-  s[9 * n] = G.gzR;
+  // a quotient of sane operands is a normal number (2^-80 / 2^40)
+  __device__ __forceinline__ static T small() { return T(0x1p-40); }
+};
+
+// prims() of gs_device.h: both quotients by one reciprocal.
+template <typename T>
+__device__ __forceinline__ void adj_prims(T h, T hu, T hv, T hm, T& u, T& v) {
+  const bool wet = h > hm;
+  const T hs = wet ? h : hm;
+  const T y = recip_w(hs);
+  u = quot_w(hu, hs, y);
+  v = quot_w(hv, hs, y);
+  if (lm_any(lm_of(wet && !(WaveOps<T>::sane(hu, hs) && WaveOps<T>::sane(hv, hs))))) {
+    u = vdiv(here(hu), hs);
+    v = vdiv(here(hv), hs);
+  }
+  u = wet ? u : T(0);
+  v = wet ? v : T(0);
 }
 
-// Every face with an active cell on either side, computed by its lower cell (the slots are
-// indexed by it): each stored cell, active or ring, takes its upper face along each axis
-// when it or the cell above is active. A wavefront then runs at most two face reverses (a
-// scheme in which an active cell also took its lower face beside a ring cell ran up to
-// four, the extra two for the few lanes on the active set's lower edges). One face per
-// trip of a loop that is not unrolled, so the reverse of a face is compiled once.
-template <typename T>
+// Element c of plane k of [planes][n], c given as its byte offset in a plane of T.
+template <typename T, typename O>
+__device__ __forceinline__ GS_G T& adj_at(T* plane, int k, int64_t n, O off) {
+  return row_at((GS_G T*)plane + k * n, off);
+}
+
+// Every face with an active cell on either side, computed by its lower cell: each stored cell,
+// active or ring, takes its upper face along each axis when it or the cell above is active. A
+// wavefront then runs at most two face reverses (a scheme in which an active cell also took its
+// lower face beside a ring cell ran up to four, the extra two for the few lanes on the active set's
+// lower edges). One face per trip of a loop that is not unrolled, so the reverse of a face is
+// compiled once. The pass is bound by vector instructions (a face is some 600) beside 130 bytes a
+// cell: the forward's quotients and roots take the short forms, a cell's velocities are computed
+// once for both its faces and their reverses, its upper neighbour's gradient is two loads (that
+// neighbour is one of its own ends), and planes are addressed by 32-bit offsets where they fit
+// (1.15 M stored cells: 44.5 us against 50.7; the gather after it, which reads 16 numbers of the
+// slots instead of 20 and no w, 26.4 against 31).
+template <typename T, typename O>
 __global__ __launch_bounds__(kABlock) void k_adj_faces(AdjK<T> a) {
-  for (int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; c < a.n; c += (int64_t)gridDim.x * blockDim.x) {
+  const T hm = a.P.h_min, g = a.P.g, dt = a.dt;
+  const int64_t n = a.n;
+  for (int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; c < n; c += (int64_t)gridDim.x * blockDim.x) {
+    const O L = (O)c * (O)sizeof(T);
     const int32_t* nb = a.nbr + 4 * c;
     const bool act = a.active[c] != 0;
+    const T hL = adj_at<const T>(a.q[0], 0, n, L), huL = adj_at<const T>(a.q[1], 0, n, L),
+            hvL = adj_at<const T>(a.q[2], 0, n, L), bL = adj_at<const T>(a.bed, 0, n, L);
+    const T wL = adj_at<T>(a.w[0], 0, n, L), wuL = adj_at<T>(a.w[1], 0, n, L), wvL = adj_at<T>(a.w[2], 0, n, L);
+    T uL, vL;
+    adj_prims(hL, huL, hvL, hm, uL, vL);
+    T sh = wL, shu = wuL, shv = wvL, sb = T(0);   // what the cell's faces and w give to it
 #pragma unroll 1
     for (int axis = 0; axis < 2; ++axis) {   // nb[0]: upper x, nb[2]: upper y
+      T* slots = axis == 0 ? a.xf : a.yf;
       const int64_t u = nb[2 * axis];
-      if (u < 0 || !(act || a.active[u])) continue;
-      face_slot<T>(a, axis, c, u, axis == 0 ? a.xf : a.yf);
+      T gzl = T(0);
+      if (u >= 0 && (act || a.active[u])) {
+        const O R = (O)u * (O)sizeof(T);
+        const T hR = adj_at<const T>(a.q[0], 0, n, R);
+        T r0 = T(0), r1 = T(0), r2 = T(0), r3 = T(0), r4 = T(0);   // the upper cell's parts
+        if (!(hL < hm && hR < hm)) {   // a dry face contributes nothing either way
+          const T huR = adj_at<const T>(a.q[1], 0, n, R), hvR = adj_at<const T>(a.q[2], 0, n, R),
+                  bR = adj_at<const T>(a.bed, 0, n, R);
+          const T inv = axis == 0 ? a.P.inv_dx : a.P.inv_dy;
+          const T half = axis == 0 ? a.P.half_dx : a.P.half_dy;
+          // the cells either side of L and R along the axis are stored for every face of an
+          // active cell (ring-2 set, checked when the table is built); clamp all the same
+          const int64_t dn = nb[2 * axis + 1], up = a.nbr[4 * u + 2 * axis];
+          const T bLd = dn >= 0 ? adj_at<const T>(a.bed, 0, n, (O)dn * (O)sizeof(T)) : bL;
+          const T bRu = up >= 0 ? adj_at<const T>(a.bed, 0, n, (O)up * (O)sizeof(T)) : bR;
+          const T gzL = (T(0.5) * (bR - bLd)) * inv;
+          const T gzR = (T(0.5) * (bRu - bL)) * inv;
+          T uR, vR;
+          adj_prims(hR, huR, hvR, hm, uR, vR);
+          // residual cotangents dt*w of both cells (zero outside active non-stage cells)
+          const T rhL = dt * wL, ruL = dt * wuL, rvL = dt * wvL;
+          const T rhR = dt * adj_at<T>(a.w[0], 0, n, R), ruR = dt * adj_at<T>(a.w[1], 0, n, R),
+                  rvR = dt * adj_at<T>(a.w[2], 0, n, R);
+          // along x the normal velocity is u, along y it is v
+          const bool x = axis == 0;
+          const T rnL = x ? ruL : rvL, rtL = x ? rvL : ruL, rnR = x ? ruR : rvR, rtR = x ? rvR : ruR;
+          FaceGrad<T> G;
+          face_vjp<T, WaveOps<T>>(bL, bR, gzL, gzR, hL, hR, x ? uL : vL, x ? vL : uL, x ? uR : vR, x ? vR : uR, half,
+                                  g, hm, inv * (rhR - rhL), inv * (rnR - rnL), inv * (rtR - rtL), -(inv * rnL),
+                                  inv * rnR, G);
+          T ghL = G.hL, ghuL = T(0), ghvL = T(0);
+          prims_vjp<T>(hL, uL, vL, hm, x ? G.uNL : G.uTL, x ? G.uTL : G.uNL, ghL, ghuL, ghvL);
+          r0 = G.hR;
+          prims_vjp<T>(hR, uR, vR, hm, x ? G.uNR : G.uTR, x ? G.uTR : G.uNR, r0, r1, r2);
+          r3 = G.bR;
+          r4 = G.gzR;
+          sh += ghL;
+          shu += ghuL;
+          shv += ghvL;
+          sb += G.bL;
+          gzl = G.gzL;
+        }
+        adj_at(slots, 5, n, L) = r0;
+        adj_at(slots, 6, n, L) = r1;
+        adj_at(slots, 7, n, L) = r2;
+        adj_at(slots, 8, n, L) = r3;
+        adj_at(slots, 9, n, L) = r4;
+      }
+      adj_at(slots, 4, n, L) = gzl;
     }
+    adj_at(a.xf, 0, n, L) = sh;
+    adj_at(a.xf, 1, n, L) = shu;
+    adj_at(a.xf, 2, n, L) = shv;
+    adj_at(a.xf, 3, n, L) = sb;
   }
 }
 
-template <typename T>
+template <typename T, typename O>
 __global__ __launch_bounds__(kABlock) void k_adj_gather(AdjK<T> a) {
   const int64_t n = a.n;
   for (int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; c < n; c += (int64_t)gridDim.x * blockDim.x) {
     const int32_t* nb = a.nbr + 4 * c;
-    const int64_t W = nb[1], S = nb[3];
-    const T* x = a.xf;
-    const T* y = a.yf;
-    T gzx = x[4 * n + c], gzy = y[4 * n + c];
-    T bb = x[3 * n + c] + y[3 * n + c];
-    if (W >= 0) { gzx += x[9 * n + W]; bb += x[8 * n + W]; }
-    if (S >= 0) { gzy += y[9 * n + S]; bb += y[8 * n + S]; }
-    a.gz[c] = gzx;
-    a.gz[n + c] = gzy;
+    const int32_t W = nb[1], S = nb[3];
+    const O o = (O)c * (O)sizeof(T), oW = (O)W * (O)sizeof(T), oS = (O)S * (O)sizeof(T);
+    T gzx = adj_at(a.xf, 4, n, o), gzy = adj_at(a.yf, 4, n, o), bb = adj_at(a.xf, 3, n, o);
+    if (W >= 0) { gzx += adj_at(a.xf, 9, n, oW); bb += adj_at(a.xf, 8, n, oW); }
+    if (S >= 0) { gzy += adj_at(a.yf, 9, n, oS); bb += adj_at(a.yf, 8, n, oS); }
+    adj_at(a.gz, 0, n, o) = gzx;
+    adj_at(a.gz, 1, n, o) = gzy;
     if (a.gz_prev) {   // the bed-gradient term of the previous reverse step (its gz is complete)
       const T hx = T(0.5) * a.P.inv_dx, hy = T(0.5) * a.P.inv_dy;
-      const int64_t E = nb[0], Nn = nb[2];
-      const T* gp_ = a.gz_prev;
-      if (W >= 0) bb += hx * gp_[W];
-      if (E >= 0) bb -= hx * gp_[E];
-      if (S >= 0) bb += hy * gp_[n + S];
-      if (Nn >= 0) bb -= hy * gp_[n + Nn];
+      const int32_t E = nb[0], Nn = nb[2];
+      if (W >= 0) bb += hx * adj_at<const T>(a.gz_prev, 0, n, oW);
+      if (E >= 0) bb -= hx * adj_at<const T>(a.gz_prev, 0, n, (O)E * (O)sizeof(T));
+      if (S >= 0) bb += hy * adj_at<const T>(a.gz_prev, 1, n, oS);
+      if (Nn >= 0) bb -= hy * adj_at<const T>(a.gz_prev, 1, n, (O)Nn * (O)sizeof(T));
     }
     a.bbar[c] += (double)bb;
     if (a.active[c]) {
       for (int k = 0; k < 3; ++k) {
-        T l = a.w[k][c] + x[k * n + c] + y[k * n + c];
-        if (W >= 0) l += x[(5 + k) * n + W];
-        if (S >= 0) l += y[(5 + k) * n + S];
-        a.lam[k][c] = l;
+        T l = adj_at(a.xf, k, n, o);
+        if (W >= 0) l += adj_at(a.xf, 5 + k, n, oW);
+        if (S >= 0) l += adj_at(a.yf, 5 + k, n, oS);
+        adj_at(a.lam[k], 0, n, o) = l;
       }
     }
   }
@@ -294,8 +344,13 @@ static int adj_step_t(const GsAdjFlat* f, const GsPhys* p, double dt, hipStream_
   const int64_t blocks = adj_blocks(a.n);
   const dim3 gr((unsigned)blocks), bl(kABlock);
   hipLaunchKernelGGL(k_adj_update<T>, gr, bl, 0, s, a);
-  hipLaunchKernelGGL(k_adj_faces<T>, gr, bl, 0, s, a);
-  hipLaunchKernelGGL(k_adj_gather<T>, gr, bl, 0, s, a);
+  if (a.n < ((int64_t)1 << 32) / (int64_t)sizeof(T)) {   // byte offsets in a plane fit 32 bits
+    hipLaunchKernelGGL((k_adj_faces<T, uint32_t>), gr, bl, 0, s, a);
+    hipLaunchKernelGGL((k_adj_gather<T, uint32_t>), gr, bl, 0, s, a);
+  } else {
+    hipLaunchKernelGGL((k_adj_faces<T, uint64_t>), gr, bl, 0, s, a);
+    hipLaunchKernelGGL((k_adj_gather<T, uint64_t>), gr, bl, 0, s, a);
+  }
   // with gz_prev the caller folds this step's bed-gradient term into the next reverse step's
   // gather (double-buffered gz) and flushes the last one with gs_adj_flat_bedgrad
   if (!a.gz_prev) hipLaunchKernelGGL(k_adj_bedgrad<T>, gr, bl, 0, s, a);

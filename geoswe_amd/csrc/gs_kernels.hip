@@ -140,18 +140,6 @@ __device__ __forceinline__ ColMap col_map(int c, int ny, int bc) {
   return m;
 }
 
-// Element at byte offset `off` of a row that starts at `row` (uniform): the row's address stays
-// in scalar registers and the lane adds a 32-bit offset, so an access costs no vector address
-// arithmetic. O is uint32_t unless a row spans 4 GiB or more.
-template <typename P, typename O>
-__device__ __forceinline__ GS_G P& row_at(GS_G P* row, O off) {
-  // a value of its own, widened beside the access: a widening hoisted out of the row loop would
-  // make the lane's address a 64-bit vector add
-  if (sizeof(O) == 4) __asm__("" : "+v"(off));
-  typedef typename std::conditional<std::is_const<P>::value, const char, char>::type B;
-  return *(GS_G P*)((GS_G B*)row + off);
-}
-
 // What a tile's rows read besides the kernel argument.
 template <typename T, typename S>
 struct DenseTile {

@@ -28,6 +28,8 @@
 // The host build (one lane, masks are bools) serves the CPU comparison with gs_device.h.
 #pragma once
 
+#include <type_traits>
+
 #include "gs_device.h"
 
 // device buffers are global memory: an explicit address space gives global (not generic) accesses
@@ -325,6 +327,20 @@ template <typename T>
 GS_HD T root0_w(T x) {
   return root_from_rsq(x, rsq_approx(max_w(x, Range<T>::root())));
 }
+
+#if defined(__HIPCC__)
+// Element at byte offset `off` of a row that starts at `row` (uniform): the row's address stays
+// in scalar registers and the lane adds a 32-bit offset, so an access costs no vector address
+// arithmetic. O is uint32_t unless a row spans 4 GiB or more.
+template <typename P, typename O>
+__device__ __forceinline__ GS_G P& row_at(GS_G P* row, O off) {
+  // a value of its own, widened beside the access: a widening hoisted out of the row loop would
+  // make the lane's address a 64-bit vector add
+  if (sizeof(O) == 4) __asm__("" : "+v"(off));
+  typedef typename std::conditional<std::is_const<P>::value, const char, char>::type B;
+  return *(GS_G P*)((GS_G B*)row + off);
+}
+#endif
 
 // ---------------------------------------------------------------------------
 // the uniform scalars of a row
