@@ -373,6 +373,10 @@ static int adj_bedgrad_t(const GsAdjFlat* f, const GsPhys* p, hipStream_t s) {
   return GS_OK;
 }
 
+// The dt that a step's plan may set for the step after it: a positive one (0, which gs_clock_set_dt
+// takes, and what it refuses go through it). A launch less per step: 5.2 us.
+static double given_dt(double dt) { return dt > 0.0 && !isinf(dt) ? dt : 0.0; }
+
 }  // namespace gs
 
 extern "C" {
@@ -444,14 +448,17 @@ int gs_flat_run_frozen(const GsFlat* f, const GsPhys* phys, GsForcing forc, GsCl
   const size_t es = f->dtype == GS_F64 ? 8 : 4;
   const size_t bytes = (size_t)f->n_stored * es;
   hipStream_t s = (hipStream_t)stream;
+  bool planned = false;   // the step before set this one's dt
   for (int j = 0; j < n; ++j) {
     if (ckpt && j % ckpt_every == 0) {   // the clock counts from 0: the state is q[j & 1]
       const int c = j / ckpt_every;
       for (int k = 0; k < 3; ++k)
         GS_HIP(hipMemcpyAsync(ckpt[3 * c + k], f->q[j & 1][k], bytes, hipMemcpyDeviceToDevice, s), "checkpoint");
     }
-    int rc = gs_clock_set_dt(clock_dev, dts[j], phys, forc, stream);
-    if (!rc) rc = gs_flat_step(f, phys, forc, clock_dev, stream);
+    const double next = j + 1 < n ? given_dt(dts[j + 1]) : 0.0;
+    int rc = planned ? GS_OK : gs_clock_set_dt(clock_dev, dts[j], phys, forc, stream);
+    if (!rc) rc = flat_step_next(f, phys, forc, clock_dev, nullptr, next, stream);
+    planned = next > 0.0;
     if (!rc && n_gauges > 0)
       rc = gs_flat_sample(f, clock_dev, gauge_ids, n_gauges, (char*)samples + (size_t)j * n_gauges * es, stream);
     if (rc) return rc;
@@ -465,14 +472,17 @@ int gs_flat_replay_pre(const GsFlat* f, const GsPhys* phys, GsForcing forc, GsCl
   if (!f || !phys || !clock_dev || (n > 0 && (!dts || !states || !pre))) return fail(GS_E_ARG, "NULL argument");
   if (n < 0) return fail(GS_E_ARG, "n < 0");
   GsFlat d = *f;
+  bool planned = false;   // the step before set this one's dt
   for (int j = 0; j < n; ++j) {
     const int par = j & 1;   // the clock counts the replayed steps from 0
     for (int k = 0; k < 3; ++k) {
       d.q[par][k] = states[3 * j + k];
       d.q[par ^ 1][k] = states[3 * (j + 1) + k];
     }
-    int rc = gs_clock_set_dt(clock_dev, dts[j], phys, forc, stream);
-    if (!rc) rc = gs_flat_step_pre(&d, phys, forc, clock_dev, pre[3 * j], pre[3 * j + 1], pre[3 * j + 2], stream);
+    const double next = j + 1 < n ? given_dt(dts[j + 1]) : 0.0;
+    int rc = planned ? GS_OK : gs_clock_set_dt(clock_dev, dts[j], phys, forc, stream);
+    if (!rc) rc = flat_step_next(&d, phys, forc, clock_dev, &pre[3 * j], next, stream);
+    planned = next > 0.0;
     if (rc) return rc;
   }
   return GS_OK;

@@ -50,6 +50,7 @@ struct Plan {
   const double* rain_cap;
   const double* stage_t;
   const double* stage_v;
+  double next_dt;   // > 0: the next step's dt, given by the host (as gs_clock_set_dt would after the step)
 };
 
 static inline Plan make_plan(const GsPhys& p, const GsForcing& f) {
@@ -64,6 +65,7 @@ static inline Plan make_plan(const GsPhys& p, const GsForcing& f) {
   pl.rain_cap = f.rain_cap;
   pl.stage_t = f.stage_t;
   pl.stage_v = f.stage_v;
+  pl.next_dt = 0.0;
   return pl;
 }
 
@@ -193,6 +195,17 @@ __device__ __forceinline__ void plan_dt(GsClock* c, const Plan& p, const ClockIn
   plan_forcing(c, p, f, k.t, dt);
 }
 
+// A dt that the host gives (gs_clock_set_dt, or Plan::next_dt from the step before).
+__device__ __forceinline__ void plan_host_dt(GsClock* c, const Plan& p, const ClockIn& k, const ForcIn& f, double dt) {
+  c->dt = dt;
+  c->dt32 = (float)dt;
+  c->use_host_dt = 1;
+  int st = k.status & ~GS_ST_DONE;
+  if ((st & GS_ST_NONFINITE) || k.nsteps >= k.max_steps) st |= GS_ST_DONE;
+  c->status = st;
+  plan_forcing(c, p, f, k.t, dt);
+}
+
 // Called by the last workgroup of a step (advance) or of a CFL pass. k: the clock before it; the
 // forcing tables are searched while the grid's maximum is on its way.
 __device__ __forceinline__ void plan_finish(GsClock* c, const Plan& p, ClockIn k, bool advance) {
@@ -210,7 +223,13 @@ __device__ __forceinline__ void plan_finish(GsClock* c, const Plan& p, ClockIn k
   c->lam_bits = lam;
   c->lam_acc = 0ull;
   c->blocks_done = 0u;
-  plan_dt(c, p, k, f, lam);
+  if (p.next_dt > 0.0) {
+    const double l = __longlong_as_double((long long)lam);
+    if (!(l == l) || isinf(l)) k.status |= GS_ST_NONFINITE;
+    plan_host_dt(c, p, k, f, p.next_dt);
+  } else {
+    plan_dt(c, p, k, f, lam);
+  }
 }
 
 // Neighbour-lane values for the y-faces: lane l receives lane l+1's value (lane_upper)
@@ -303,6 +322,11 @@ static inline Phys<T> make_phys(const GsPhys& p, double dx, double dy) {
   P.cfl_l2 = p.cfl_l2;
   return P;
 }
+
+// gs_flat_step (pre: NULL, or the three planes of gs_flat_step_pre) whose plan takes `next_dt` for the
+// step after it if that is positive.
+int flat_step_next(const GsFlat* f, const GsPhys* phys, const GsForcing& forc, GsClock* clock_dev, void* const* pre,
+                   double next_dt, void* stream);
 
 static inline int check_phys(const GsPhys* p) {
   if (!p) return fail(GS_E_ARG, "phys is NULL");

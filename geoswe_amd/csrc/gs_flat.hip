@@ -1362,10 +1362,11 @@ static int flat_step_launch(const FlatK<T>& a, hipStream_t s) {
 
 template <typename T>
 static int flat_step_t(const GsFlat* f, const GsPhys* p, GsForcing fo, GsClock* clk, hipStream_t s,
-                       void* pre0 = nullptr, void* pre1 = nullptr, void* pre2 = nullptr) {
+                       void* pre0 = nullptr, void* pre1 = nullptr, void* pre2 = nullptr, double next_dt = 0.0) {
   FlatK<T> a;
   int rc = build_flat<T>(f, p, fo, clk, a, true);
   if (rc) return rc;
+  a.plan.next_dt = next_dt;
   if ((pre0 || pre1 || pre2) && !(pre0 && pre1 && pre2)) return fail(GS_E_ARG, "pre: all three planes or none");
   if (pre0 && a.n_tiles == 0)
     return fail(GS_E_ARG, "the pre-friction state is written by the row-sweep traversal only (n_tiles > 0)");
@@ -1575,6 +1576,17 @@ static void ens_launch_kind(int kind, int64_t blocks, hipStream_t s, const EnsK<
     hipLaunchKernelGGL((k_ens_step<T, kEnsLean>), dim3((unsigned)blocks), dim3(kFBlock), 0, s, k, k.mem, k.tile0);
   else
     hipLaunchKernelGGL((k_ens_step<T, kEnsPlain>), dim3((unsigned)blocks), dim3(kFBlock), 0, s, k, k.mem, k.tile0);
+}
+
+int flat_step_next(const GsFlat* f, const GsPhys* phys, const GsForcing& forc, GsClock* clock_dev, void* const* pre,
+                   double next_dt, void* stream) {
+  if (!f) return fail(GS_E_ARG, "flat descriptor is NULL");
+  void *p0 = pre ? pre[0] : nullptr, *p1 = pre ? pre[1] : nullptr, *p2 = pre ? pre[2] : nullptr;
+  if (pre && (!p0 || !p1 || !p2)) return fail(GS_E_ARG, "pre arrays are NULL");
+  const hipStream_t s = (hipStream_t)stream;
+  if (f->dtype == GS_F64) return flat_step_t<double>(f, phys, forc, clock_dev, s, p0, p1, p2, next_dt);
+  if (f->dtype == GS_F32) return flat_step_t<float>(f, phys, forc, clock_dev, s, p0, p1, p2, next_dt);
+  return fail(GS_E_DTYPE, "unsupported dtype %d", f->dtype);
 }
 
 }  // namespace gs

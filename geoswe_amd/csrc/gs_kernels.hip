@@ -65,13 +65,7 @@ __global__ void k_clock_dt(GsClock* c, Plan p, double dt) {
   const ClockIn k = clock_read(c);
   ForcIn f;
   forcing_read(p, k.t, f);
-  c->dt = dt;
-  c->dt32 = (float)dt;
-  c->use_host_dt = 1;
-  int st = k.status & ~GS_ST_DONE;
-  if ((st & GS_ST_NONFINITE) || k.nsteps >= k.max_steps) st |= GS_ST_DONE;
-  c->status = st;
-  plan_forcing(c, p, f, k.t, dt);
+  plan_host_dt(c, p, k, f, dt);
 }
 
 

@@ -46,3 +46,41 @@ def test_rain_and_stage_of_a_plan_equal_the_host(gpu, n, kind):
             seg = min(max(bisect.bisect_right(ts.tolist(), float(t)) - 1, 0), n - 1)
             assert c.rain_idx == seg and c.rain32 == np.float32(sv[seg] + 1.0)
             assert c.eta64 == sb.stage_at_time(float(t) + dt), (t, dt)
+
+
+@pytest.mark.parametrize("dtype", ["float32", "float64"])
+@pytest.mark.parametrize("trav", ["tiles", "chunks"])
+def test_frozen_steps_plan_the_next_dt(gpu, dtype, trav):
+    """Steps whose plan takes the next frozen dt end in the state and the clock, byte for byte, of
+    steps that are each given theirs; a dt of 0 among them (which a plan does not take) too."""
+    from geoswe_amd import CompressedSolver, RainfallForcing, _lib as L
+    rng = np.random.default_rng(11)
+    nx, ny = 24, 70
+    bed = rng.random((nx, ny))
+    q = np.stack([np.maximum(1.0 - bed, 0), np.zeros((nx, ny)), np.zeros((nx, ny))])
+    dts = np.array([0.01, 0.02, 0.015, 0.0, 0.03, 0.01])
+    out = []
+    for frozen in (True, False):
+        mesh = Mesh2D(nx, ny, 2.0, 2.0)
+        sea = np.zeros((nx, ny), bool)
+        sea[0] = True
+        sb = StageBoundary.from_mask(sea, mesh, bed, np.array([0.0, 0.02, 0.05, 1.0]), np.array([1.0, 1.3, 0.9, 1.1]))
+        cfg = Config(bc_x="fall", bc_y="fall", dtype=dtype, friction="manning", manning_n=0.03, stage_boundary=sb,
+                     rainfall_forcing=RainfallForcing(np.array([0.0, 0.03, 0.06]), np.array([10.0, 50.0, 0.0])))
+        c = CompressedSolver.from_dense(Solver2D(mesh, cfg, q.astype(dtype), bed.astype(dtype)), cfl_linf=True,
+                                        track_max_depth=False)
+        c.traversal = trav
+        if frozen:
+            c._ensure_lam()
+            L.call("gs_flat_run_frozen", C.byref(c._desc()), C.byref(c._phys()), c._fo.s, C.c_void_p(c._clock.ptr),
+                   len(dts), C.c_void_p(dts.ctypes.data), None, 0, None, 1, None, None)
+            L.sync(None)
+        else:
+            c._ensure_lam()
+            for dt in dts:
+                L.call("gs_clock_set_dt", C.c_void_p(c._clock.ptr), C.c_double(dt), C.byref(c._phys()), c._fo.s, None)
+                L.call("gs_flat_step", C.byref(c._desc()), C.byref(c._phys()), c._fo.s, C.c_void_p(c._clock.ptr), None)
+            L.sync(None)
+        out.append((c.q_flat(), c._clock.download().tobytes(), c.nsteps))
+    assert out[0][2] == out[1][2] == len(dts)
+    assert np.array_equal(out[0][0], out[1][0]) and out[0][1] == out[1][1]
