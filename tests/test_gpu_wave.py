@@ -112,3 +112,44 @@ def test_flat_sweep_at_tile_edges(gpu, shape, rows, ext, maxh, dtype, odd):
     a, b = out
     assert a[1:3] == b[1:3] and np.array_equal(a[0], b[0])
     assert not maxh or np.array_equal(a[3], b[3])
+
+
+@pytest.mark.parametrize("dtype,compute", [("float32", None), ("float64", None), ("float32", "float64")])
+@pytest.mark.parametrize("manning", ["flags", "plane", "field"])
+@pytest.mark.parametrize("gridded,masked", [(False, False), (True, False), (False, True), (True, True)])
+@pytest.mark.parametrize("shape,rows", [((5, 61), 1), ((23, 130), 4)])
+def test_dense_planes_loaded_ahead(gpu, shape, rows, gridded, masked, manning, dtype, compute):
+    """The cells' flags, classes, Manning field, rain frame and running maximum loaded a row ahead give
+    the bits of the sweep with 64-bit offsets (tile height 1 << 20), which loads them at their use."""
+    from geoswe_amd import RainfallForcing, StageBoundary
+    nx, ny = shape
+    rng = np.random.default_rng(nx + ny)
+    q, bed = _state(nx, ny, False)
+    mask = rng.random((nx, ny)) > 0.1
+    frames = rng.random((2, nx, ny)) * 4.0e4
+    cls = rng.integers(0, 40 if manning == "plane" else 5, (nx, ny)).astype(np.uint8)
+    n_of = np.linspace(0.02, 0.09, 40 if manning == "plane" else 5)
+    mesh = Mesh2D(nx, ny, 2.0, 2.0, ngh=4)
+    sea = np.zeros((nx, ny), bool)
+    sea[:, 0] = True
+    out = []
+    for tile_rows in (rows, 1 << 20):
+        kw = dict(rainfall_forcing=RainfallForcing(np.array([0.0, 2e-3]), frames)) if gridded else \
+            dict(rainfall=20.0 / 3.6e6)
+        if masked:
+            kw["stage_boundary"] = StageBoundary.from_mask(sea, mesh, bed, np.array([0.0, 1.0]), np.array([0.9, 1.4]))
+        cfg = Config(bc_x="fall", bc_y="wall", dtype=dtype, compute_dtype=compute, friction="manning",
+                     manning_n=0.03, **kw)
+        s = Solver2D(mesh, cfg, q.astype(dtype), bed.astype(dtype), tile_rows=tile_rows)
+        if manning == "field":
+            s.set_manning(n_of[cls] + 1e-3 * np.arange(ny))
+        else:
+            s.set_manning_table(np.pad(cls, 4, mode="edge"), n_of)
+        if masked:
+            s.set_inside_mask(mask)
+            s.set_cfl_ghost_mask(~mask)
+        for dt in (1e-3, 2e-3, 1e-3):
+            s.step(dt)
+        out.append((s.q_interior, s.max_depth(), s._clockv().lam_bits))
+    a, b = out
+    assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1]) and a[2] == b[2]
