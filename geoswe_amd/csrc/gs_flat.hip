@@ -88,6 +88,7 @@ struct FlatK {
   const int64_t* fring;
   const int32_t* fring_row;  // nullable: gauge-ring row of each entry, -1 for none
   int ring_ng, ring_nt;
+  unsigned ring_blocks;  // first workgroups of a sweep that take the ring cells (a multiple of 8, 0: none)
   const T* ring_bed;
   const T* ring_w;
   const double* ring_t;
@@ -978,80 +979,11 @@ __global__ __launch_bounds__(kFBlock) void k_flat_step(FlatK<T> a) {
   if (MODE == 1) grid_reduce_and_plan(lam, a.clock, a.plan, true);
 }
 
-// One step of one flat domain by row-sweep tiles, one wavefront per tile in band-major tile
-// order and XCD-major wavefront order. What bounds it is the issue of vector instructions (about
-// 400 per row, 0.8 of the cycles) and, on a domain of one round of tiles, the slowest tile. The
-// float32 steps are held to 80 VGPRs (6 wavefronts per SIMD), where no row reloads a spilled
-// register. LEAN (a domain with no per-cell Manning field or class plane, running maximum or
-// active-cell forcing) drops those paths. us per step, general functions with 4-row tiles before
-// and wavefront forms now: 2048^2 coastal domain (lean) 63 and 40, 1500^2 with the forcing tail
-// (below) 69 and 57.
-template <typename T, bool PRE, bool LEAN = false>
-__global__ __launch_bounds__(kSBlock<T>) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 6 : 1))) void k_flat_sweep(FlatK<T> a) {
-  // What waits on nothing but the argument is asked for first: the tile's place, the Manning table
-  // and the clock. Each wavefront keeps its own copy of the table, so that none waits for another
-  // (2048^2 coastal step: 38.4 us against 39.5; the extended sweep, with fewer registers to spare,
-  // gained nothing from it and keeps the shorter form).
-  const GS_C FlatK<T>* k = kernel_arg<T>();
-  const int lane = threadIdx.x & 63;
-  const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const int64_t nwaves = (int64_t)gridDim.x * kSweepWaves<T>;
-  int64_t t = (int64_t)xcd_rank(blockIdx.x, gridDim.x) * kSweepWaves<T> + wv;
-  TileHead h = tile_head<T>(k, t < a.n_tiles ? t : a.n_tiles - 1);
-  __shared__ T s_ntab[kSweepWaves<T>][GS_MAX_CLASSES];
-  const T n_mine = lane < a.n_classes ? gp(a.ntab)[lane] : T(0);
-  const FlatClk<T> ck = flat_clock<T, 1>(a);
-  if (!ck.live) return;   // the whole grid sees the same clock
-  FlatCtx<T> x;
-  flat_ctx<T, 1>(a, ck, x);
-  x.k = k;
-  s_ntab[wv][lane] = n_mine;
-  for (int c = lane + 64; c < a.n_classes; c += 64) s_ntab[wv][c] = gp(a.ntab)[c];
-  x.ntab = s_ntab[wv];
-  lam_t<T> lam = 0;
-  // PRE (the adjoint's recomputation) also compiles the extended forcings in, so that a
-  // replay reads rain through the per-cell lookup exactly as the forward run's extended sweep
-  while (t < a.n_tiles) {
-    flat_tile<T, PRE, PRE, LEAN>(x, h, lane, lam);
-    t += nwaves;
-    if (t < a.n_tiles) h = tile_head<T>(cold_ptr<T>(k), t);
-  }
-  grid_reduce_and_plan(lam, a.clock, a.plan, true);
-}
-
-// The sweep with the extended forcings compiled in: Green-Ampt infiltration, drain-tau and
-// rain read through a per-cell lookup into a native-grid table (launched only when one of
-// them is set).
+// The forcings on the ring cells of the band (stored, not active): out = force(in), one thread per
+// listed id, by `blocks` workgroups. The step itself only reads these cells, from the input buffer,
+// so the two never touch the same word.
 template <typename T>
-__global__ __launch_bounds__(kSBlock<T>) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 6 : 1))) void k_flat_sweep_ext(FlatK<T> a) {
-  const FlatClk<T> ck = flat_clock<T, 1>(a);
-  if (!ck.live) return;
-  FlatCtx<T> x;
-  flat_ctx<T, 1>(a, ck, x);
-  x.k = kernel_arg<T>();
-  __shared__ T s_ntab[GS_MAX_CLASSES];
-  for (int k = (int)threadIdx.x; k < a.n_classes; k += (int)blockDim.x) s_ntab[k] = a.ntab[k];
-  __syncthreads();
-  x.ntab = s_ntab;
-  const int lane = threadIdx.x & 63;
-  const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const int64_t nwaves = (int64_t)gridDim.x * kSweepWaves<T>;
-  lam_t<T> lam = 0;
-  for (int64_t t = (int64_t)xcd_rank(blockIdx.x, gridDim.x) * kSweepWaves<T> + wv; t < a.n_tiles; t += nwaves)
-    flat_tile<T, false, true>(x, tile_head<T>(cold_ptr<T>(x.k), t), lane, lam);
-  grid_reduce_and_plan(lam, a.clock, a.plan, true);
-}
-
-// The forcings on the ring cells of the band (stored, not active): out = force(in), one
-// thread per listed id. Launched just before the step kernel on the same stream, it reads
-// the clock the step will read (its input buffer, its done state); the step kernel only
-// reads these cells, from the input buffer, so the two never touch the same word.
-template <typename T>
-__global__ __launch_bounds__(kFBlock) void k_flat_ring_force(FlatK<T> a) {
-  const FlatClk<T> ck = flat_clock<T, 1>(a);
-  if (!ck.live) return;
-  FlatCtx<T> x;
-  flat_ctx<T, 1>(a, ck, x);
+__device__ __forceinline__ void ring_cells(const FlatK<T>& a, const FlatCtx<T>& x, unsigned block, unsigned blocks) {
   const bool sp = x.sponge != nullptr, cl = x.clamp != nullptr;
   const GS_G int64_t* ids = gp(a.fring);
   const GS_G int32_t* rows = gp(a.fring_row);
@@ -1059,14 +991,10 @@ __global__ __launch_bounds__(kFBlock) void k_flat_ring_force(FlatK<T> a) {
   T wa = T(0), wb = T(0);
   int ti = 0;
   if (rows) {
-    const GS_G double* tc = gp(a.ring_t);
+    const double* tc = a.ring_t;
     const double t = gp(a.clock)->t;
-    int lo = 0, hi = a.ring_nt;   // bisect_left: the number of samples below t
-    while (lo < hi) {
-      const int mid = (lo + hi) >> 1;
-      if (tc[mid] < t) lo = mid + 1; else hi = mid;
-    }
-    ti = lo - 1;
+    // bisect_left: the number of samples below t
+    ti = table_count(tc, 0, a.ring_nt, [t](double v) { return v < t; }) - 1;
     if (ti > a.ring_nt - 2) ti = a.ring_nt - 2;
     if (ti < 0) ti = 0;
     double wt = (t - tc[ti]) / (tc[ti + 1] - tc[ti] + 1.0e-12);
@@ -1075,7 +1003,7 @@ __global__ __launch_bounds__(kFBlock) void k_flat_ring_force(FlatK<T> a) {
     wa = (T)(1.0 - wt);
     wb = (T)wt;
   }
-  for (int64_t i = (int64_t)blockIdx.x * kFBlock + threadIdx.x; i < a.n_fring; i += (int64_t)gridDim.x * kFBlock) {
+  for (int64_t i = (int64_t)block * blockDim.x + threadIdx.x; i < a.n_fring; i += (int64_t)blocks * blockDim.x) {
     const int64_t k = ids[i];
     T h = x.qi0[k], hu = x.qi1[k], hv = x.qi2[k];
     const bool fc = x.flags != nullptr && (x.flags[k] & GS_FLAG_FORCE);
@@ -1100,6 +1028,87 @@ __global__ __launch_bounds__(kFBlock) void k_flat_ring_force(FlatK<T> a) {
     x.qo1[k] = hu;
     x.qo2[k] = hv;
   }
+}
+
+// Launched just before the chunk traversal on the same stream: it reads the clock the step will read.
+template <typename T>
+__global__ __launch_bounds__(kFBlock) void k_flat_ring_force(FlatK<T> a) {
+  const FlatClk<T> ck = flat_clock<T, 1>(a);
+  if (!ck.live) return;
+  FlatCtx<T> x;
+  flat_ctx<T, 1>(a, ck, x);
+  ring_cells<T>(a, x, blockIdx.x, gridDim.x);
+}
+
+// One step of one flat domain by row-sweep tiles, one wavefront per tile in band-major tile
+// order and XCD-major wavefront order. What bounds it is the issue of vector instructions (about
+// 400 per row, 0.8 of the cycles) and, on a domain of one round of tiles, the slowest tile. The
+// float32 steps are held to 80 VGPRs (6 wavefronts per SIMD), where no row reloads a spilled
+// register. LEAN (a domain with no per-cell Manning field or class plane, running maximum or
+// active-cell forcing) drops those paths. us per step, general functions with 4-row tiles before
+// and wavefront forms now: 2048^2 coastal domain (lean) 63 and 40, 1500^2 with the forcing tail
+// (below) 69 and 57.
+template <typename T, bool PRE, bool LEAN = false>
+__global__ __launch_bounds__(kSBlock<T>) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 6 : 1))) void k_flat_sweep(FlatK<T> a) {
+  // What waits on nothing but the argument is asked for first: the tile's place, the Manning table
+  // and the clock. Each wavefront keeps its own copy of the table, so that none waits for another
+  // (2048^2 coastal step: 38.4 us against 39.5; the extended sweep, with fewer registers to spare,
+  // gained nothing from it and keeps the shorter form).
+  const GS_C FlatK<T>* k = kernel_arg<T>();
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const unsigned rb = LEAN || PRE ? 0u : a.ring_blocks;
+  const bool ring = blockIdx.x < rb;
+  const int64_t nwaves = (int64_t)(gridDim.x - rb) * kSweepWaves<T>;
+  int64_t t = (int64_t)xcd_rank(blockIdx.x - rb, gridDim.x - rb) * kSweepWaves<T> + wv;
+  TileHead h = tile_head<T>(k, !ring && t < a.n_tiles ? t : a.n_tiles - 1);   // (a ring workgroup's is not used)
+  __shared__ T s_ntab[kSweepWaves<T>][GS_MAX_CLASSES];
+  const T n_mine = lane < a.n_classes ? gp(a.ntab)[lane] : T(0);
+  const FlatClk<T> ck = flat_clock<T, 1>(a);
+  if (!ck.live) return;   // the whole grid sees the same clock
+  FlatCtx<T> x;
+  flat_ctx<T, 1>(a, ck, x);
+  x.k = k;
+  s_ntab[wv][lane] = n_mine;
+  for (int c = lane + 64; c < a.n_classes; c += 64) s_ntab[wv][c] = gp(a.ntab)[c];
+  x.ntab = s_ntab[wv];
+  lam_t<T> lam = 0;
+  // PRE (the adjoint's recomputation) also compiles the extended forcings in, so that a
+  // replay reads rain through the per-cell lookup exactly as the forward run's extended sweep
+  if (ring) ring_cells<T>(a, x, blockIdx.x, rb);
+  while (!ring && t < a.n_tiles) {
+    flat_tile<T, PRE, PRE, LEAN>(x, h, lane, lam);
+    t += nwaves;
+    if (t < a.n_tiles) h = tile_head<T>(cold_ptr<T>(k), t);
+  }
+  grid_reduce_and_plan(lam, a.clock, a.plan, true);
+}
+
+// The sweep with the extended forcings compiled in: Green-Ampt infiltration, drain-tau and
+// rain read through a per-cell lookup into a native-grid table (launched only when one of
+// them is set).
+template <typename T>
+__global__ __launch_bounds__(kSBlock<T>) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 6 : 1))) void k_flat_sweep_ext(FlatK<T> a) {
+  const FlatClk<T> ck = flat_clock<T, 1>(a);
+  if (!ck.live) return;
+  FlatCtx<T> x;
+  flat_ctx<T, 1>(a, ck, x);
+  x.k = kernel_arg<T>();
+  __shared__ T s_ntab[GS_MAX_CLASSES];
+  for (int k = (int)threadIdx.x; k < a.n_classes; k += (int)blockDim.x) s_ntab[k] = a.ntab[k];
+  __syncthreads();
+  x.ntab = s_ntab;
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const unsigned rb = a.ring_blocks;
+  const bool ring = blockIdx.x < rb;
+  const int64_t nwaves = (int64_t)(gridDim.x - rb) * kSweepWaves<T>;
+  lam_t<T> lam = 0;
+  if (ring) ring_cells<T>(a, x, blockIdx.x, rb);
+  for (int64_t t = (int64_t)xcd_rank(blockIdx.x - rb, gridDim.x - rb) * kSweepWaves<T> + wv; !ring && t < a.n_tiles;
+       t += nwaves)
+    flat_tile<T, false, true>(x, tile_head<T>(cold_ptr<T>(x.k), t), lane, lam);
+  grid_reduce_and_plan(lam, a.clock, a.plan, true);
 }
 
 // The ring modes of the cached replay on the step's input state, before the step reads
@@ -1330,13 +1339,20 @@ static void flat_launch_choice(const FlatK<T>& a, int* kernel, int64_t* blocks, 
 
 // The fused step: row-sweep tiles when the descriptor has them, else chunks of the run table.
 template <typename T>
-static int flat_step_launch(const FlatK<T>& a, hipStream_t s) {
+static int flat_step_launch(FlatK<T>& a, hipStream_t s) {
   if (a.n_rmode > 0) {
     const int64_t nb = (a.n_rmode + kFBlock - 1) / kFBlock;
     hipLaunchKernelGGL((k_flat_ring_mode<T>), dim3((unsigned)(nb < 1024 ? nb : 1024)), dim3(kFBlock), 0, s, a);
     GS_HIP(hipGetLastError(), "k_flat_ring_mode launch");
   }
-  if (a.n_fring > 0) {
+  const bool ext = a.ga_ks || a.ga_inv_tau || a.rain_mode == 3;
+  if (a.n_fring > 0 && a.n_tiles > 0 && !a.pre[0] && (ext || !flat_lean(a))) {
+    // the ring cells by workgroups of the sweep itself, ahead of its tiles (a launch of their own took
+    // 8 us beside a 46 us sweep: 1500^2 with the forcing tail 547 -> 484 us for 10 steps); the lean
+    // sweep, which only a gauge ring by itself would bring here, has no register for them
+    const int64_t nb = (a.n_fring + kSBlock<T> - 1) / kSBlock<T>;
+    a.ring_blocks = (unsigned)(((nb < 1024 ? nb : 1024) + 7) / 8 * 8);
+  } else if (a.n_fring > 0) {
     const int64_t nb = (a.n_fring + kFBlock - 1) / kFBlock;
     hipLaunchKernelGGL((k_flat_ring_force<T>), dim3((unsigned)(nb < 1024 ? nb : 1024)), dim3(kFBlock), 0, s, a);
     GS_HIP(hipGetLastError(), "k_flat_ring_force launch");
@@ -1344,14 +1360,14 @@ static int flat_step_launch(const FlatK<T>& a, hipStream_t s) {
   if (a.n_tiles > 0 && a.pre[0]) {
     hipLaunchKernelGGL((k_flat_sweep<T, true>), dim3(sweep_grid<T>(a.n_tiles)), dim3(kSBlock<T>), 0, s, a);
     GS_HIP(hipGetLastError(), "k_flat_sweep(pre) launch");
-  } else if (a.n_tiles > 0 && (a.ga_ks || a.ga_inv_tau || a.rain_mode == 3)) {
-    hipLaunchKernelGGL((k_flat_sweep_ext<T>), dim3(sweep_grid<T>(a.n_tiles)), dim3(kSBlock<T>), 0, s, a);
+  } else if (a.n_tiles > 0 && ext) {
+    hipLaunchKernelGGL((k_flat_sweep_ext<T>), dim3(sweep_grid<T>(a.n_tiles) + a.ring_blocks), dim3(kSBlock<T>), 0, s, a);
     GS_HIP(hipGetLastError(), "k_flat_sweep_ext launch");
   } else if (a.n_tiles > 0 && flat_lean(a)) {
     hipLaunchKernelGGL((k_flat_sweep<T, false, true>), dim3(sweep_grid<T>(a.n_tiles)), dim3(kSBlock<T>), 0, s, a);
     GS_HIP(hipGetLastError(), "k_flat_sweep(lean) launch");
   } else if (a.n_tiles > 0) {
-    hipLaunchKernelGGL((k_flat_sweep<T, false>), dim3(sweep_grid<T>(a.n_tiles)), dim3(kSBlock<T>), 0, s, a);
+    hipLaunchKernelGGL((k_flat_sweep<T, false>), dim3(sweep_grid<T>(a.n_tiles) + a.ring_blocks), dim3(kSBlock<T>), 0, s, a);
     GS_HIP(hipGetLastError(), "k_flat_sweep launch");
   } else {
     hipLaunchKernelGGL((k_flat_step<T, 1>), dim3(flat_grid<T, 1>(a.nchunks)), dim3(kFBlock), 0, s, a);
