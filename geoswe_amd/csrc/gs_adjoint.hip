@@ -457,9 +457,12 @@ int gs_flat_run_frozen(const GsFlat* f, const GsPhys* phys, GsForcing forc, GsCl
     }
     const double next = j + 1 < n ? given_dt(dts[j + 1]) : 0.0;
     int rc = planned ? GS_OK : gs_clock_set_dt(clock_dev, dts[j], phys, forc, stream);
-    if (!rc) rc = flat_step_next(f, phys, forc, clock_dev, nullptr, next, stream);
+    // the state after step j - 1 is this step's input, which its sweep samples on its way (a launch
+    // per step less: 5 us)
+    const FlatSample smp = {gauge_ids, n_gauges, (char*)samples + (size_t)(j - 1) * n_gauges * es};
+    if (!rc) rc = flat_step_next(f, phys, forc, clock_dev, nullptr, next, j > 0 && n_gauges > 0 ? &smp : nullptr, stream);
     planned = next > 0.0;
-    if (!rc && n_gauges > 0)
+    if (!rc && n_gauges > 0 && j + 1 == n)
       rc = gs_flat_sample(f, clock_dev, gauge_ids, n_gauges, (char*)samples + (size_t)j * n_gauges * es, stream);
     if (rc) return rc;
   }
@@ -481,7 +484,7 @@ int gs_flat_replay_pre(const GsFlat* f, const GsPhys* phys, GsForcing forc, GsCl
     }
     const double next = j + 1 < n ? given_dt(dts[j + 1]) : 0.0;
     int rc = planned ? GS_OK : gs_clock_set_dt(clock_dev, dts[j], phys, forc, stream);
-    if (!rc) rc = flat_step_next(&d, phys, forc, clock_dev, &pre[3 * j], next, stream);
+    if (!rc) rc = flat_step_next(&d, phys, forc, clock_dev, &pre[3 * j], next, nullptr, stream);
     planned = next > 0.0;
     if (rc) return rc;
   }

@@ -324,9 +324,14 @@ static inline Phys<T> make_phys(const GsPhys& p, double dx, double dy) {
 }
 
 // gs_flat_step (pre: NULL, or the three planes of gs_flat_step_pre) whose plan takes `next_dt` for the
-// step after it if that is positive.
+// step after it if that is positive. smp: NULL, or depths of the step's input state to sample.
+struct FlatSample {
+  const int64_t* ids;
+  int n;
+  void* out;
+};
 int flat_step_next(const GsFlat* f, const GsPhys* phys, const GsForcing& forc, GsClock* clock_dev, void* const* pre,
-                   double next_dt, void* stream);
+                   double next_dt, const FlatSample* smp, void* stream);
 
 static inline int check_phys(const GsPhys* p) {
   if (!p) return fail(GS_E_ARG, "phys is NULL");

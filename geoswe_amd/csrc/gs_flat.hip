@@ -88,6 +88,9 @@ struct FlatK {
   const int64_t* fring;
   const int32_t* fring_row;  // nullable: gauge-ring row of each entry, -1 for none
   int ring_ng, ring_nt;
+  const int64_t* smp_ids;  // lean sweep: depths of the step's input state at smp_n ids into smp_out
+  int smp_n;
+  T* smp_out;
   unsigned ring_blocks;  // first workgroups of a sweep that take the ring cells (a multiple of 8, 0: none)
   const T* ring_bed;
   const T* ring_w;
@@ -202,11 +205,11 @@ __device__ __forceinline__ FlatClk<T> flat_clock(const FlatK<T>& a) {
     const int64_t ns = c->nsteps;
     const T dt = sizeof(T) == 4 ? (T)c->dt32 : (T)c->dt, eta = sizeof(T) == 4 ? (T)c->eta32 : (T)c->eta64;
     const T rain = sizeof(T) == 4 ? (T)c->rain32 : T(0);
+    k.par = __builtin_amdgcn_readfirstlane((int)(ns & 1));
     if (st & GS_ST_DONE) {
       k.live = false;
       return k;
     }
-    k.par = __builtin_amdgcn_readfirstlane((int)(ns & 1));
     k.dt = sreg(dt);
     k.rain_u = sizeof(T) == 4 ? sreg(rain) : a.rain_mode == 1 ? sreg((T)gp(a.plan.rain_rate)[ridx]) : T(0);
     k.eta = sreg(eta);
@@ -1065,6 +1068,10 @@ __global__ __launch_bounds__(kSBlock<T>) __attribute__((amdgpu_waves_per_eu(size
   __shared__ T s_ntab[kSweepWaves<T>][GS_MAX_CLASSES];
   const T n_mine = lane < a.n_classes ? gp(a.ntab)[lane] : T(0);
   const FlatClk<T> ck = flat_clock<T, 1>(a);
+  if (LEAN && a.smp_n > 0 && blockIdx.x == gridDim.x - 1 && wv == 0) {
+    const GS_G T* h0 = gp(ck.par ? a.buf[1][0] : a.buf[0][0]);
+    for (int i = lane; i < a.smp_n; i += 64) gp(a.smp_out)[i] = h0[gp(a.smp_ids)[i]];
+  }
   if (!ck.live) return;   // the whole grid sees the same clock
   FlatCtx<T> x;
   flat_ctx<T, 1>(a, ck, x);
@@ -1073,11 +1080,11 @@ __global__ __launch_bounds__(kSBlock<T>) __attribute__((amdgpu_waves_per_eu(size
   for (int c = lane + 64; c < a.n_classes; c += 64) s_ntab[wv][c] = gp(a.ntab)[c];
   x.ntab = s_ntab[wv];
   lam_t<T> lam = 0;
-  // PRE (the adjoint's recomputation) also compiles the extended forcings in, so that a
-  // replay reads rain through the per-cell lookup exactly as the forward run's extended sweep
+  // PRE (the adjoint's recomputation) also compiles the extended forcings in unless it is LEAN, so
+  // that a replay reads rain through the per-cell lookup exactly as the forward run's extended sweep
   if (ring) ring_cells<T>(a, x, blockIdx.x, rb);
   while (!ring && t < a.n_tiles) {
-    flat_tile<T, PRE, PRE, LEAN>(x, h, lane, lam);
+    flat_tile<T, PRE, PRE && !LEAN, LEAN>(x, h, lane, lam);
     t += nwaves;
     if (t < a.n_tiles) h = tile_head<T>(cold_ptr<T>(k), t);
   }
@@ -1357,7 +1364,11 @@ static int flat_step_launch(FlatK<T>& a, hipStream_t s) {
     hipLaunchKernelGGL((k_flat_ring_force<T>), dim3((unsigned)(nb < 1024 ? nb : 1024)), dim3(kFBlock), 0, s, a);
     GS_HIP(hipGetLastError(), "k_flat_ring_force launch");
   }
-  if (a.n_tiles > 0 && a.pre[0]) {
+  if (a.n_tiles > 0 && a.pre[0] && !ext && flat_lean(a)) {
+    // 1536^2 adjoint: 33.5 us against the general pre-friction sweep's 36
+    hipLaunchKernelGGL((k_flat_sweep<T, true, true>), dim3(sweep_grid<T>(a.n_tiles)), dim3(kSBlock<T>), 0, s, a);
+    GS_HIP(hipGetLastError(), "k_flat_sweep(pre, lean) launch");
+  } else if (a.n_tiles > 0 && a.pre[0]) {
     hipLaunchKernelGGL((k_flat_sweep<T, true>), dim3(sweep_grid<T>(a.n_tiles)), dim3(kSBlock<T>), 0, s, a);
     GS_HIP(hipGetLastError(), "k_flat_sweep(pre) launch");
   } else if (a.n_tiles > 0 && ext) {
@@ -1376,9 +1387,19 @@ static int flat_step_launch(FlatK<T>& a, hipStream_t s) {
   return GS_OK;
 }
 
+// Depth of the current state at listed flat ids (gauges), read after a step.
+template <typename T>
+__global__ void k_flat_sample(FlatK<T> a, const int64_t* ids, int n, T* out) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= n) return;
+  const int par = (int)(a.clock->nsteps & 1);
+  out[t] = a.buf[par][0][ids[t]];
+}
+
 template <typename T>
 static int flat_step_t(const GsFlat* f, const GsPhys* p, GsForcing fo, GsClock* clk, hipStream_t s,
-                       void* pre0 = nullptr, void* pre1 = nullptr, void* pre2 = nullptr, double next_dt = 0.0) {
+                       void* pre0 = nullptr, void* pre1 = nullptr, void* pre2 = nullptr, double next_dt = 0.0,
+                       const FlatSample* smp = nullptr) {
   FlatK<T> a;
   int rc = build_flat<T>(f, p, fo, clk, a, true);
   if (rc) return rc;
@@ -1389,6 +1410,15 @@ static int flat_step_t(const GsFlat* f, const GsPhys* p, GsForcing fo, GsClock* 
   a.pre[0] = (T*)pre0;
   a.pre[1] = (T*)pre1;
   a.pre[2] = (T*)pre2;
+  if (smp && a.n_tiles > 0 && !pre0 && !(a.ga_ks || a.ga_inv_tau || a.rain_mode == 3) && flat_lean(a)) {
+    a.smp_ids = smp->ids;   // by a wavefront of the sweep, on its way
+    a.smp_n = smp->n;
+    a.smp_out = (T*)smp->out;
+  } else if (smp) {
+    hipLaunchKernelGGL(k_flat_sample<T>, dim3((unsigned)((smp->n + 255) / 256)), dim3(256), 0, s, a, smp->ids, smp->n,
+                       (T*)smp->out);
+    GS_HIP(hipGetLastError(), "k_flat_sample launch");
+  }
   return flat_step_launch<T>(a, s);
 }
 
@@ -1424,15 +1454,6 @@ static int flat_cfl_t(const GsFlat* f, const GsPhys* p, GsForcing fo, GsClock* c
   return GS_OK;
 }
 
-
-// Depth of the current state at listed flat ids (gauges), read after a step.
-template <typename T>
-__global__ void k_flat_sample(FlatK<T> a, const int64_t* ids, int n, T* out) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
-  const int par = (int)(a.clock->nsteps & 1);
-  out[t] = a.buf[par][0][ids[t]];
-}
 
 // ---------------------------------------------------------------------------
 // batched ensemble: every member's sweep tiles in one launch, per-member clocks
@@ -1595,13 +1616,13 @@ static void ens_launch_kind(int kind, int64_t blocks, hipStream_t s, const EnsK<
 }
 
 int flat_step_next(const GsFlat* f, const GsPhys* phys, const GsForcing& forc, GsClock* clock_dev, void* const* pre,
-                   double next_dt, void* stream) {
+                   double next_dt, const FlatSample* smp, void* stream) {
   if (!f) return fail(GS_E_ARG, "flat descriptor is NULL");
   void *p0 = pre ? pre[0] : nullptr, *p1 = pre ? pre[1] : nullptr, *p2 = pre ? pre[2] : nullptr;
   if (pre && (!p0 || !p1 || !p2)) return fail(GS_E_ARG, "pre arrays are NULL");
   const hipStream_t s = (hipStream_t)stream;
-  if (f->dtype == GS_F64) return flat_step_t<double>(f, phys, forc, clock_dev, s, p0, p1, p2, next_dt);
-  if (f->dtype == GS_F32) return flat_step_t<float>(f, phys, forc, clock_dev, s, p0, p1, p2, next_dt);
+  if (f->dtype == GS_F64) return flat_step_t<double>(f, phys, forc, clock_dev, s, p0, p1, p2, next_dt, smp);
+  if (f->dtype == GS_F32) return flat_step_t<float>(f, phys, forc, clock_dev, s, p0, p1, p2, next_dt, smp);
   return fail(GS_E_DTYPE, "unsupported dtype %d", f->dtype);
 }
 

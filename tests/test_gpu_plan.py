@@ -84,3 +84,38 @@ def test_frozen_steps_plan_the_next_dt(gpu, dtype, trav):
         out.append((c.q_flat(), c._clock.download().tobytes(), c.nsteps))
     assert out[0][2] == out[1][2] == len(dts)
     assert np.array_equal(out[0][0], out[1][0]) and out[0][1] == out[1][1]
+
+
+@pytest.mark.parametrize("trav,ga", [("tiles", False), ("chunks", False), ("tiles", True)])
+@pytest.mark.parametrize("n", [1, 2, 5])
+def test_frozen_steps_sample_the_gauges(gpu, trav, ga, n):
+    """The depths after every frozen step at 1, 64 and 130 gauges (repeated ids among them), whether
+    the next step's sweep samples them or a launch does, are the depths of steps taken one by one."""
+    from geoswe_amd import CompressedSolver, _lib as L
+    rng = np.random.default_rng(3)
+    nx, ny = 20, 66
+    bed = rng.random((nx, ny))
+    q = np.stack([np.maximum(1.2 - bed, 0), np.zeros((nx, ny)), np.zeros((nx, ny))]).astype(np.float32)
+    dts = np.full(n, 0.01)
+
+    def solver():
+        cfg = Config(bc_x="fall", bc_y="fall", dtype="float32", friction="manning", manning_n=0.03)
+        c = CompressedSolver.from_dense(Solver2D(Mesh2D(nx, ny, 2.0, 2.0), cfg, q, bed.astype(np.float32)),
+                                        cfl_linf=True, track_max_depth=ga)     # the maximum: not the lean sweep
+        c.traversal = trav
+        c._ensure_lam()
+        return c
+
+    ref = solver()
+    want = []
+    for dt in dts:
+        ref.step(dt)
+        want.append(ref.q_flat()[0])
+    for g in (1, 64, 130):
+        c = solver()
+        ids = rng.choice(np.flatnonzero(c.fm.active), size=g)
+        d_ids, out = L.DeviceArray.from_host(ids.astype(np.int64)), L.DeviceArray((n, g), np.float32, zero=True)
+        L.call("gs_flat_run_frozen", C.byref(c._desc()), C.byref(c._phys()), c._fo.s, C.c_void_p(c._clock.ptr), n,
+               C.c_void_p(dts.ctypes.data), C.c_void_p(d_ids.ptr), g, C.c_void_p(out.ptr), 1, None, None)
+        L.sync(None)
+        assert np.array_equal(out.download(), np.stack([w[ids] for w in want]))
