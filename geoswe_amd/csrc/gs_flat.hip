@@ -420,47 +420,64 @@ __device__ __forceinline__ float exp_ieee_f(float x) {
   return ldexpf(p, (int)kf);
 }
 
-// Green-Ampt infiltration then drain-tau of one active cell (ga_drain_flat); `ob` is the
-// cell's offset in a one-byte plane.
+// What the forcings of every active cell read: its infiltration rate, and with GA its Green-Ampt and
+// drain-tau values (0 where there are none). Loaded ahead of the update, all at once: at their use,
+// behind the branches on the rate, K and h, seven loads waited for one another, and the whole forcing
+// tail on 121 M cells took 2.44 ms per step against 2.01 (10 steps on 1500^2: 484 us against 451).
 template <typename T>
-__device__ __forceinline__ void ga_cell(const FlatCtx<T>& x, int64_t base, uint32_t off, uint32_t ob, T& h, T& hu,
-                                        T& hv) {
+struct ForceIn {
+  T rate, K, psi, dth, F0, fmax, inv_tau;
+};
+template <typename T, bool GA>
+__device__ __forceinline__ ForceIn<T> force_load(const FlatCtx<T>& x, uint8_t fg, int64_t base, uint32_t off,
+                                                 uint32_t ob) {
+  ForceIn<T> v = {T(0), T(0), T(0), T(0), T(0), T(0), T(0)};
+  if (GA && x.ga_ks) {
+    const int c = gat(x.ga_cls + base, ob);
+    v.F0 = gat(x.ga_F + base, off);
+    if (x.ga_fmax) v.fmax = gat(x.ga_fmax + base, off);
+    if (x.ga_inv_tau) v.inv_tau = gat(x.ga_inv_tau + base, off);
+    v.K = x.ga_ks[c];
+    v.psi = x.ga_psi[c];
+    v.dth = x.ga_dth[c];
+  } else if (GA && x.ga_inv_tau) {
+    v.inv_tau = gat(x.ga_inv_tau + base, off);
+  }
+  if (x.infil) v.rate = x.infil[x.cls ? gat(x.cls + base, ob) : (fg & GS_FLAG_CLASS_MASK)];
+  return v;
+}
+
+// Green-Ampt infiltration then drain-tau of one active cell (ga_drain_flat).
+template <typename T>
+__device__ __forceinline__ void ga_cell(const FlatCtx<T>& x, const ForceIn<T>& v, int64_t base, uint32_t off, T& h,
+                                        T& hu, T& hv) {
   if (h <= T(0)) return;
   T scale = T(1);
-  if (x.ga_ks) {
-    const int c = gat(x.ga_cls + base, ob);
-    const T K = x.ga_ks[c];
-    if (K > T(0)) {
-      const T KsDt = K * x.dt;
-      const T head = x.ga_psi[c] + h;
-      GS_G T& Fr = gat(x.ga_F + base, off);
-      const T F0 = Fr;
-      const T a = F0 + KsDt;
-      const T disc = a * a + ((T(4) * KsDt) * head) * x.ga_dth[c];
-      const T F1 = T(0.5) * (a + sqrt(disc > T(0) ? disc : T(0)));   // fmax(disc, 0): NaN gives 0
-      T dF = F1 - F0;
-      dF = dF > T(0) ? dF : T(0);
-      if (dF > h) dF = h;
-      if (x.ga_fmax) {
-        const T room = gat(x.ga_fmax + base, off) - F0;
-        if (dF > room) dF = room > T(0) ? room : T(0);
-      }
-      const T hn = h - dF;
-      scale = scale * (hn / h);
-      h = hn;
-      Fr = F0 + dF;
+  if (v.K > T(0)) {
+    const T KsDt = v.K * x.dt;
+    const T head = v.psi + h;
+    const T a = v.F0 + KsDt;
+    const T disc = a * a + ((T(4) * KsDt) * head) * v.dth;
+    const T F1 = T(0.5) * (a + sqrt(disc > T(0) ? disc : T(0)));   // fmax(disc, 0): NaN gives 0
+    T dF = F1 - v.F0;
+    dF = dF > T(0) ? dF : T(0);
+    if (dF > h) dF = h;
+    if (x.ga_fmax) {
+      const T room = v.fmax - v.F0;
+      if (dF > room) dF = room > T(0) ? room : T(0);
     }
+    const T hn = h - dF;
+    scale = scale * (hn / h);
+    h = hn;
+    gat(x.ga_F + base, off) = v.F0 + dF;
   }
-  if (x.ga_inv_tau) {
-    const T it = gat(x.ga_inv_tau + base, off);
-    if (it > T(0) && h > T(0)) {
-      const T arg = (-x.dt) * it;
-      T decay;
-      if constexpr (sizeof(T) == 4) decay = exp_ieee_f(arg);
-      else decay = exp_ieee(arg);
-      scale = scale * decay;
-      h = h * decay;
-    }
+  if (v.inv_tau > T(0) && h > T(0)) {
+    const T arg = (-x.dt) * v.inv_tau;
+    T decay;
+    if constexpr (sizeof(T) == 4) decay = exp_ieee_f(arg);
+    else decay = exp_ieee(arg);
+    scale = scale * decay;
+    h = h * decay;
   }
   hu = hu * scale;
   hv = hv * scale;
@@ -472,14 +489,13 @@ __device__ __forceinline__ void ga_cell(const FlatCtx<T>& x, int64_t base, uint3
 // the karst drain of a GS_FLAG_FORCE cell. GA = false leaves Green-Ampt out of the code (the
 // plain sweep's instantiation, which has no register to spare for it).
 template <typename T, bool GA>
-__device__ __forceinline__ void active_force(const FlatCtx<T>& x, uint8_t fg, int64_t base, uint32_t off,
-                                             uint32_t ob, T& h, T& hu, T& hv) {
-  if (x.infil)
-    infil_cell<T>(x.infil[x.cls ? gat(x.cls + base, ob) : (fg & GS_FLAG_CLASS_MASK)], x.dt, x.P.h_min, h, hu, hv);
+__device__ __forceinline__ void active_force(const FlatCtx<T>& x, const ForceIn<T>& v, uint8_t fg, int64_t base,
+                                             uint32_t off, T& h, T& hu, T& hv) {
+  if (x.infil) infil_cell<T>(v.rate, x.dt, x.P.h_min, h, hu, hv);
   const bool fc = (fg & GS_FLAG_FORCE) != 0;
   if (fc && x.sponge)
     sponge_cell<T>(gat(x.sponge + 2 * base, 2 * off), gat(x.sponge + 2 * base + 1, 2 * off), h, hu, hv);
-  if (GA && (x.ga_ks || x.ga_inv_tau)) ga_cell<T>(x, base, off, ob, h, hu, hv);
+  if (GA && (x.ga_ks || x.ga_inv_tau)) ga_cell<T>(x, v, base, off, h, hu, hv);
   if (fc && x.clamp) clamp_cell<T>(gat(x.clamp + base, off), h, hu, hv);
   if (fc && x.drain) drain_cell<T>(gat(x.drain + base, off), h, hu, hv);
 }
@@ -587,7 +603,7 @@ __device__ __forceinline__ void flat_chunk(const FlatCtx<T>& x, int64_t chunk, i
     hv = T(0);
   }
   if (a.max_h && h > a.max_h[k]) a.max_h[k] = h;
-  active_force<T, true>(x, fg, k, 0u, 0u, h, hu, hv);
+  active_force<T, true>(x, force_load<T, true>(x, fg, k, 0u, 0u), fg, k, 0u, h, hu, hv);
   x.qo0[k] = h;
   x.qo1[k] = hu;
   x.qo2[k] = hv;
@@ -636,8 +652,8 @@ __device__ __forceinline__ T sweep_b(const FlatCtx<T>& x, int64_t base, uint32_t
 // The cell of an active lane after its update, in the reference's order: the stage, the running
 // max and the forcings (what LEAN leaves out is not there).
 template <typename T, bool EXT, bool LEAN>
-__device__ __forceinline__ void finish_cell(const FlatCtx<T>& x, uint8_t fg, int64_t base, uint32_t off, T b, T& h,
-                                            T& hu, T& hv) {
+__device__ __forceinline__ void finish_cell(const FlatCtx<T>& x, const ForceIn<T>& v, uint8_t fg, int64_t base,
+                                            uint32_t off, T b, T& h, T& hu, T& hv) {
   if (fg & GS_FLAG_STAGE) {
     const T hs = x.eta - b;
     h = hs > T(0) ? hs : T(0);
@@ -646,7 +662,7 @@ __device__ __forceinline__ void finish_cell(const FlatCtx<T>& x, uint8_t fg, int
   }
   if (!LEAN) {
     if (x.max_h && h > gat(x.max_h + base, off)) gat(x.max_h + base, off) = h;
-    active_force<T, EXT>(x, fg, base, off, off / (uint32_t)sizeof(T), h, hu, hv);
+    active_force<T, EXT>(x, v, fg, base, off, h, hu, hv);
   }
 }
 
@@ -782,6 +798,11 @@ __device__ __forceinline__ int flat_rows(const FlatCtx<T>& x, const WaveC<T>& w,
       }
     }
     load_c(eN, r + 1, sfl, srn);
+    ForceIn<T> fin;
+    if (!LEAN) {
+      const FlatCtx<T> y = cold(x);
+      if (lm_lane(act)) fin = force_load<T, EXT>(y, fg, gC, eC.below * es, eC.below);
+    }
     T h, hu, hv, speed;
     update_w<T>(hC, huC, hvC, rr0, rhu, rhv, n, act, x.P, w, h, hu, hv, speed, odd);
     const bool left = lm_any(odd);
@@ -804,7 +825,7 @@ __device__ __forceinline__ int flat_rows(const FlatCtx<T>& x, const WaveC<T>& w,
       key = lam_key_w<T>(speed);
     } else {
       const FlatCtx<T> y = cold(x);
-      if (lm_lane(act) && !left) finish_cell<T, EXT, LEAN>(y, fg, gC, eC.below * es, b0, h, hu, hv);
+      if (lm_lane(act) && !left) finish_cell<T, EXT, LEAN>(y, fin, fg, gC, eC.below * es, b0, h, hu, hv);
       speed = speed_w<T>(h, hu, hv, w);
       key = lam_key_w<T>(speed);
       if (lm_any(act & lm_not(lm_lt(speed, kMaxSpeed<T>)))) key = lam_key<T, true>(h, hu, hv, cold(x).P);
@@ -905,7 +926,9 @@ __device__ __forceinline__ void flat_rows_general(const FlatCtx<T>& hot, const G
                                  : x.ntab[(!LEAN && x.cls) ? gat(x.cls + gC, ob) : (fg & GS_FLAG_CLASS_MASK)];
       T h, hu, hv;
       update<T>(hC, huC, hvC, rr0, rhu, rhv, x.dt, n, P, h, hu, hv);
-      finish_cell<T, EXT, LEAN>(x, fg, gC, oC, b0, h, hu, hv);
+      ForceIn<T> fin;
+      if (!LEAN) fin = force_load<T, EXT>(x, fg, gC, oC, ob);
+      finish_cell<T, EXT, LEAN>(x, fin, fg, gC, oC, b0, h, hu, hv);
       gat(x.qo0 + gC, oC) = h;
       gat(x.qo1 + gC, oC) = hu;
       gat(x.qo2 + gC, oC) = hv;
