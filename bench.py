@@ -114,7 +114,7 @@ def mixed_timing(nx, ny, bed, steps, warmup):
     wall, ev_ms = timed_steps(s, steps)
     cells = nx * ny
     out = {"value": cells * steps / wall, "unit": "cell-updates/s", "steps": steps, "ms_per_step": 1e3 * wall / steps,
-           "kernel_ms": ev_ms / steps, "kernel": "gs::k_dense_sweep<double, 1, float>",
+           "kernel_ms": ev_ms / steps, "kernel": "gs::k_dense_sweep<double, 1, true, float, unsigned int>",
            "hbm_frac": BYTES_PER_CELL["dense"] * cells / (ev_ms / steps * 1e-3) / 1e9 / HBM_PEAK_GBS}
     log(f"float32 planes, float64 arithmetic: {out['ms_per_step']:.3f} ms/step, {out['value'] / 1e9:.2f} G "
         f"cell-updates/s")
@@ -341,7 +341,7 @@ def coastal_forcing_tail(case, steps, sweep_rows, plain_ms):
     log(f"with the forcing tail: {ms:.3f} ms/step against {plain_ms:.3f} ms/step plain "
         f"({(ms / plain_ms - 1) * 100:+.1f} %)")
     return {"ms_per_step": ms, "plain_ms_per_step": plain_ms, "overhead": ms / plain_ms - 1.0, "cells": cells,
-            "kernels": ["gs::k_flat_ring_force<float>", "gs::k_flat_sweep_ext<float>"]}
+            "kernels": ["gs::k_flat_sweep_ext<float>"]}
 
 
 def ensemble(args):
@@ -815,8 +815,9 @@ def main():
             valu = {"insts_per_cell": v["valu_insts_per_cell"], "wave_insts_per_launch": v["valu_wave_insts_per_launch"],
                     "wave_insts_per_s": v["valu_wave_insts_per_launch"] / (kern_ms * 1e-3), "source": v["source"]}
             # the device's measured float32 multiply/add issue rate (gs_bench_valu) and the
-            # step's VALU rate against it: at or above 1 the step is bound by instruction issue
-            # (its compares, selects and moves issue faster than float32 arithmetic)
+            # step's VALU rate against it: near or above 1 the step is bound by instruction issue
+            # (the calibration's operations each have a scalar operand; on vector registers alone
+            # they issue up to 1.7 times as fast, compares and selects at the calibration's rate)
             cal = valu_calibration()
             valu.update({"fp32_peak_wave_insts_per_s": cal["simple_wave_insts_per_s"],
                          "rate_over_fp32_peak": valu["wave_insts_per_s"] / cal["simple_wave_insts_per_s"],
@@ -862,7 +863,7 @@ def main():
         # against the device's measured float32 issue rate; achieved/peak/frac are the HBM figures
         "roofline": {"bound": "valu" if valu else "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
-                     "kernel": "gs::k_dense_sweep<float, 1, float>" if args.layout == "dense" else "gs::k_flat_sweep<float, false, true>",
+                     "kernel": "gs::k_dense_sweep<float, 1, true, float, unsigned int>" if args.layout == "dense" else "gs::k_flat_sweep<float, false, true>",
                      "kernel_ms": kern_ms, "bytes_per_cell": BYTES_PER_CELL[args.layout], "valu": valu,
                      "copy_GBps": copy["GBps_read_plus_write"],
                      "frac_of_copy": achieved / copy["GBps_read_plus_write"]},

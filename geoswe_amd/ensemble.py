@@ -3,9 +3,10 @@
 The reference advances independent scenarios one after another, each through
 ``CompressedSolver.run`` (src/geoswe/compressed_solver.py:3359-3450) with one host-driven
 launch sequence per step. ``Ensemble`` advances all members together: one launch of
-``k_ens_step`` per step walks every member's sweep tiles on a resident grid, each member keeps
-its own device clock (its own CFL dt, rain frame and tide level), the last workgroup plans
-every member's next dt, and the steps are replayed from a captured hipGraph. The cell
+``k_ens_step`` per step walks every member's sweep tiles (one wavefront per tile unless a
+launch shape is set), each member keeps its own device clock (its own CFL dt, rain frame and
+tide level), the last workgroup plans every member's next dt, and the steps are replayed from
+a captured hipGraph. The cell
 arithmetic is the flat step's own device code, so member k's state is bit for bit the one
 its plain ``CompressedSolver`` run produces in the same number of steps.
 """
