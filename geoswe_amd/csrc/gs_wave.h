@@ -47,7 +47,7 @@ namespace gs {
 #if defined(__HIP_DEVICE_COMPILE__)
 typedef uint64_t lmask;
 // predicates of the compare builtins (ordered unless noted)
-enum { kGT = 2, kGE = 3, kLT = 4, kLE = 5 };
+enum { kGT = 2, kGE = 3, kLT = 4, kLE = 5, kORD = 7 };
 __device__ __forceinline__ lmask lm_gt(float a, float b) { return __builtin_amdgcn_fcmpf(a, b, kGT); }
 __device__ __forceinline__ lmask lm_ge(float a, float b) { return __builtin_amdgcn_fcmpf(a, b, kGE); }
 __device__ __forceinline__ lmask lm_lt(float a, float b) { return __builtin_amdgcn_fcmpf(a, b, kLT); }
@@ -56,6 +56,9 @@ __device__ __forceinline__ lmask lm_gt(double a, double b) { return __builtin_am
 __device__ __forceinline__ lmask lm_ge(double a, double b) { return __builtin_amdgcn_fcmp(a, b, kGE); }
 __device__ __forceinline__ lmask lm_lt(double a, double b) { return __builtin_amdgcn_fcmp(a, b, kLT); }
 __device__ __forceinline__ lmask lm_le(double a, double b) { return __builtin_amdgcn_fcmp(a, b, kLE); }
+// neither is NaN
+__device__ __forceinline__ lmask lm_ord(float a, float b) { return __builtin_amdgcn_fcmpf(a, b, kORD); }
+__device__ __forceinline__ lmask lm_ord(double a, double b) { return __builtin_amdgcn_fcmp(a, b, kORD); }
 __device__ __forceinline__ lmask lm_of(bool c) { return __ballot(c); }
 __device__ __forceinline__ lmask lm_none() { return 0ull; }
 __device__ __forceinline__ lmask lm_every() { return ~0ull; }
@@ -228,6 +231,7 @@ template <typename T> GS_HD lmask lm_gt(T a, T b) { return a > b; }
 template <typename T> GS_HD lmask lm_ge(T a, T b) { return a >= b; }
 template <typename T> GS_HD lmask lm_lt(T a, T b) { return a < b; }
 template <typename T> GS_HD lmask lm_le(T a, T b) { return a <= b; }
+template <typename T> GS_HD lmask lm_ord(T a, T b) { return a == a && b == b; }
 GS_HD lmask lm_none() { return false; }
 GS_HD lmask lm_every() { return true; }
 GS_HD lmask lm_not(lmask m) { return !m; }
@@ -622,7 +626,8 @@ constexpr T kMaxSpeed = T(0x1p40);
 //
 // One test of the final speed stands for the operands: where a depth, a momentum or an
 // intermediate is not finite, or too large for a quotient, the speed is not below 2^40 (NaN
-// included). Small momenta need no test: below 2^-100 their square vanishes beside any square
+// included: the maximum drops one NaN of two, but with friction both momenta are then NaN, by the
+// speed that scales them, and without it they are tested). Small momenta need no test: below 2^-100 their square vanishes beside any square
 // that matters, and velocities below 2^-48, whose root may be an ulp off, must vanish beside the
 // 1 of alpha's denominator (`creep`).
 template <typename T>
@@ -661,6 +666,8 @@ GS_HD void update_w(T q0, T q1, T q2, T rr0, T r1, T r2, T n, lmask act, const P
     if (lm_any(creep)) odd = odd | (creep & lm_ge(two, Range<T>::vanish()));
     hu = hu * alpha;
     hv = hv * alpha;
+  } else {
+    odd = odd | (lm_not(lm_ord(hu, hv)) & live);
   }
   speed = quot_w(max_abs_w(hu, hv), hs, yh) + root_w(w.g * h);
   odd = odd | (lm_not(lm_lt(speed, kMaxSpeed<T>)) & live);
@@ -673,12 +680,13 @@ GS_HD void update_w(T q0, T q1, T q2, T rr0, T r1, T r2, T n, lmask act, const P
 }
 
 // The wave speed of a state that the update did not make (a stage, a forcing): the same expression.
-// Not below kMaxSpeed on a wet lane: one that this form does not serve.
+// Not below kMaxSpeed on a wet lane: one that this form does not serve (a NaN momentum beside a
+// finite one among them, which the maximum alone would drop).
 template <typename T>
 GS_HD T speed_w(T h, T hu, T hv, const WaveC<T>& w) {
   const T hs = max_w(h, w.hm);
   const T speed = quot_w(max_abs_w(hu, hv), hs, recip_w(hs)) + root_w(w.g * h);
-  return lm_sel(lm_lt(h, w.hm), T(0), speed);
+  return lm_sel(lm_lt(h, w.hm), T(0), lm_sel(lm_ord(hu, hv), speed, T(INFINITY)));
 }
 
 #if defined(__HIPCC__)
