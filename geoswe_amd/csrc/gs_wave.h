@@ -309,22 +309,19 @@ GS_HD double root_from_rsq(double x, double y) {
 }
 template <typename T> GS_HD T root_w(T x) { return root_from_rsq(x, rsq_approx(x)); }
 // x below `root` takes the general root (0 excepted); numerators below `num_tiny` the general
-// quotient, where a remainder could be inexact; quotients of operands in [lo, hi] are safe;
-// 1 + 2x = 1 for x below `vanish`
+// quotient, where a remainder could be inexact; quotients of operands in [lo, hi] are safe
 template <typename T> struct Range;
 template <> struct Range<float> {
   GS_HD static float root() { return 0x1p-96f; }
   GS_HD static float num_tiny() { return 0x1p-80f; }
   GS_HD static float lo() { return 0x1p-60f; }
   GS_HD static float hi() { return 0x1p60f; }
-  GS_HD static float vanish() { return 0x1p-27f; }
 };
 template <> struct Range<double> {
   GS_HD static double root() { return 0x1p-700; }
   GS_HD static double num_tiny() { return 0x1p-700; }
   GS_HD static double lo() { return 0x1p-400; }
   GS_HD static double hi() { return 0x1p400; }
-  GS_HD static double vanish() { return 0x1p-56; }
 };
 // RN(sqrt(x)) with sqrt(0) = 0 (x >= 0, not in (0, root()))
 template <typename T>
@@ -627,9 +624,8 @@ constexpr T kMaxSpeed = T(0x1p40);
 // One test of the final speed stands for the operands: where a depth, a momentum or an
 // intermediate is not finite, or too large for a quotient, the speed is not below 2^40 (NaN
 // included: the maximum drops one NaN of two, but with friction both momenta are then NaN, by the
-// speed that scales them, and without it they are tested). Small momenta need no test: below 2^-100 their square vanishes beside any square
-// that matters, and velocities below 2^-48, whose root may be an ulp off, must vanish beside the
-// 1 of alpha's denominator (`creep`).
+// speed that scales them, and without it they are tested). Small momenta need no test: below 2^-100
+// their square vanishes beside any square that matters.
 template <typename T>
 GS_HD void update_w(T q0, T q1, T q2, T rr0, T r1, T r2, T n, lmask act, const Phys<T>& P, const WaveC<T>& w, T& h,
                     T& hu, T& hv, T& speed, lmask& odd) {
@@ -644,7 +640,12 @@ GS_HD void update_w(T q0, T q1, T q2, T rr0, T r1, T r2, T n, lmask act, const P
     const T u = quot_w(hu, hs, yh);
     const T v = quot_w(hv, hs, yh);
     const T m2 = u * u + v * v;
-    const T modU = root0_w(m2);
+    T modU = root0_w(m2);
+    lmask creep = lm_lt(m2, Range<T>::root()) & live;
+    if (lm_any(creep)) {   // still water is in order; velocities below 2^-48 take the general root
+      creep = creep & lm_gt(m2, T(0));
+      if (lm_any(creep)) modU = lm_sel(creep, vsqrt(here(m2)), modU);
+    }
     const T h43 = pow_m43(hs);
     const lmask fastw = lm_gt(modU, w.vcap) & live;
     if (lm_any(fastw)) {
@@ -652,18 +653,14 @@ GS_HD void update_w(T q0, T q1, T q2, T rr0, T r1, T r2, T n, lmask act, const P
       n = lm_sel(fastw & lm_gt(n_cri, n), n_cri, n);
     }
     const T Cf = ((w.g * n) * n) * h43;
-    const lmask creep = lm_lt(m2, Range<T>::root()) & live;
-    T alpha, two;
+    T alpha;
     if (P.quadratic) {
       // two = 2*dt*Cf*modU is 2*half, and alpha = 2 / (sqrt(1 + 2*two) + 1), where RN(2/d) = 2 RN(1/d)
       const T half = (w.dt * Cf) * modU;
-      two = T(2) * half;
       alpha = T(2) * recip_w(root_w(vfma(T(4), half, T(1))) + T(1));
     } else {
-      two = (w.dt * Cf) * modU;
-      alpha = recip_w(T(1) + two);
+      alpha = recip_w(T(1) + (w.dt * Cf) * modU);
     }
-    if (lm_any(creep)) odd = odd | (creep & lm_ge(two, Range<T>::vanish()));
     hu = hu * alpha;
     hv = hv * alpha;
   } else {

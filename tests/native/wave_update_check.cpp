@@ -1,7 +1,8 @@
 // CPU comparison of update_w and speed_w (gs_wave.h, built for one lane) with the general functions
-// (gs_device.h), over the physics that wave_check.cpp holds fixed: friction on and off, with and
-// without the velocity cap and the kept film, and values that are not finite in the momenta of dry
-// cells as of wet ones. Test infrastructure only.
+// (gs_device.h), over the physics that wave_check.cpp holds fixed: friction on and off, both
+// friction formulas, with and without the velocity cap and the kept film, steps of 1 ms to 3 h,
+// Manning numbers and momenta of every size, and values that are not finite in the momenta of
+// dry cells as of wet ones. Test infrastructure only.
 #define main wave_check_main
 #include "wave_check.cpp"
 #undef main
@@ -9,19 +10,21 @@
 template <typename T>
 static double log_uni(double lo, double hi) { return pow(10.0, uni(lo, hi)); }
 
-// kind: 0 flood, 2 special values in the momenta, 3 special values anywhere
+// kind: 0 flood, 1 creeping films, 2 special values in the momenta, 3 special values anywhere
 template <typename T>
 static void updates(int kind, long n, Count& c) {
   for (long k = 0; k < n; ++k) {
-    Phys<T> P = phys<T>(rnd() % 4 == 0 ? T(1e-3) : T(1e-6), 1);
+    Phys<T> P = phys<T>(rnd() % 4 == 0 ? T(1e-3) : T(1e-6), (int)(rnd() & 1));
     P.friction = (int)(rnd() % 3 != 0);
     P.keep_h = (int)(rnd() & 1);
     P.has_vcap = (int)(rnd() & 1);
-    const T dt = (T)uni(1e-3, 2.0);
+    if (rnd() % 4 == 0) P.vcap = (T)log_uni<T>(-25, 2);
+    const T dt = (T)log_uni<T>(-3, 4);
     const WaveC<T> w = wave_consts<T>(P, dt, wave_flags<T>(P, false));
     T h = rnd() % 4 == 0 ? T(0) : (T)log_uni<T>(-8, 1), hu, hv;
     switch (kind) {
       case 0: hu = (T)(h * uni(-3, 3)); hv = (T)(h * uni(-3, 3)); break;
+      case 1: hu = (T)(h * uni(-1, 1) * log_uni<T>(-25, -8)); hv = rnd() & 1 ? T(0) : (T)(h * uni(-1, 1) * log_uni<T>(-25, -8)); break;
       default: hu = rnd() & 1 ? special<T>() : (T)uni(-2, 2); hv = rnd() & 1 ? special<T>() : (T)uni(-2, 2); break;
     }
     T r0 = (T)(uni(-0.2, 1.0) * log_uni<T>(-8, -3)), r1 = T(0), r2 = T(0);
@@ -31,7 +34,7 @@ static void updates(int kind, long n, Count& c) {
       if (rnd() % 4 == 0) r0 = special<T>();
       if (rnd() % 4 == 0) r1 = special<T>();
     }
-    const T nn = (T)uni(0.0, 0.12);
+    T nn = kind == 3 && rnd() % 4 == 0 ? vabs(special<T>()) : (T)(rnd() % 8 == 0 ? 0.0 : log_uni<T>(-3, 0));
     T oh, ohu, ohv, speed, eh, ehu, ehv;
     lmask odd = false;
     update_w<T>(h, hu, hv, r0, r1, r2, nn, true, P, w, oh, ohu, ohv, speed, odd);
@@ -60,10 +63,9 @@ static void updates(int kind, long n, Count& c) {
 }
 
 int main() {
-  const char* names[] = {"flood", "", "special momenta", "special values"};
+  const char* names[] = {"flood", "creeping films", "special momenta", "special values"};
   int rc = 0;
   for (int k = 0; k < 4; ++k) {
-    if (k == 1) continue;
     Count f, d;
     updates<float>(k, 2000000, f);
     updates<double>(k, 1000000, d);
