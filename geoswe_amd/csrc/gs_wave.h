@@ -655,11 +655,15 @@ GS_HD void update_w(T q0, T q1, T q2, T rr0, T r1, T r2, T n, lmask act, const P
     const T Cf = ((w.g * n) * n) * h43;
     T alpha;
     if (P.quadratic) {
-      // two = 2*dt*Cf*modU is 2*half, and alpha = 2 / (sqrt(1 + 2*two) + 1), where RN(2/d) = 2 RN(1/d)
-      const T half = (w.dt * Cf) * modU;
-      alpha = T(2) * recip_w(root_w(vfma(T(4), half, T(1))) + T(1));
+      // alpha = 2 / (sqrt(1 + 2*two) + 1), where RN(2/d) = 2 RN(1/d); doubled where (2*dt)*Cf would
+      // overflow, so that it does here too
+      const T dtCf = w.dt * Cf;
+      const T two = (dtCf + dtCf) * modU;
+      alpha = T(2) * recip_w(root_w(vfma(T(2), two, T(1))) + T(1));
     } else {
-      alpha = recip_w(T(1) + (w.dt * Cf) * modU);
+      const T d = T(1) + (w.dt * Cf) * modU;
+      alpha = recip_w(d);
+      odd = odd | (lm_gt(d, Range<T>::hi()) & live);   // alpha may be subnormal
     }
     hu = hu * alpha;
     hv = hv * alpha;

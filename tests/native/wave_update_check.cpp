@@ -35,6 +35,7 @@ static void updates(int kind, long n, Count& c) {
       if (rnd() % 4 == 0) r1 = special<T>();
     }
     T nn = kind == 3 && rnd() % 4 == 0 ? vabs(special<T>()) : (T)(rnd() % 8 == 0 ? 0.0 : log_uni<T>(-3, 0));
+    if (kind > 1 && rnd() % 4 == 0) nn = (T)log_uni<T>(3, sizeof(T) == 4 ? 19 : 154);   // n^2 up to the largest number
     T oh, ohu, ohv, speed, eh, ehu, ehv;
     lmask odd = false;
     update_w<T>(h, hu, hv, r0, r1, r2, nn, true, P, w, oh, ohu, ohv, speed, odd);
