@@ -154,10 +154,15 @@ __global__ __launch_bounds__(256) void k_valu(float* out, int iters, float m, fl
 // every x with |x| outside (0, 2^-96); 2: a/b for 2^32 pairs of seeded bit patterns (every exponent);
 // 3: a/b for every a over four divisors with the hardest significands (all ones, 1 + ulp,
 // 1 - ulp/2, 3); 4: the wavefront forms of gs_wave.h: the root for every x >= 2^-96 and 0, and
-// the quotient for 2^32 seeded pairs within its bounds. counts[2*k] = mismatches of check k, counts[2*k + 1] = 1 + the largest
-// offending index (0: none).
+// the quotient for 2^32 seeded pairs within its bounds; 5: their float64 forms for 2^30 seeded operands
+// within their bounds, every other one of the hardest significands (next below 2, next above 1):
+// root; quotients, of 1 and 2 too. counts[2*k] = mismatches of check k, counts[2*k + 1] = 1 + the
+// largest offending index (0: none).
 __device__ __forceinline__ bool cr_same(float a, float b) {
   return (a != a && b != b) || __float_as_uint(a) == __float_as_uint(b);
+}
+__device__ __forceinline__ bool cr_same(double a, double b) {
+  return (a != a && b != b) || __double_as_longlong(a) == __double_as_longlong(b);
 }
 __device__ __forceinline__ uint32_t cr_hash(uint64_t i, uint32_t k) {
   return philox2x32((uint32_t)i, (uint32_t)(i >> 32), k);
@@ -165,7 +170,7 @@ __device__ __forceinline__ uint32_t cr_hash(uint64_t i, uint32_t k) {
 
 template <int CASE>
 __global__ __launch_bounds__(256) void k_crmath_check(unsigned long long* counts) {
-  const uint64_t n = CASE == 3 ? (4ull << 32) : (1ull << 32);
+  const uint64_t n = CASE == 3 ? (4ull << 32) : CASE == 5 ? (1ull << 30) : (1ull << 32);
   unsigned long long bad0 = 0, bad1 = 0, last0 = 0, last1 = 0;
   for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (uint64_t)gridDim.x * 256) {
     if (CASE == 0) {
@@ -191,6 +196,20 @@ __global__ __launch_bounds__(256) void k_crmath_check(unsigned long long* counts
       const float b = __uint_as_float((hb & (sign | 0x7FFFFFu)) | ((106u + ((hb >> 23) & 63u) % 46u) << 23));
       const float n = (i & 0xFFFFu) ? a : (ha & 1u ? 0.0f : -0.0f);
       if (!cr_same(quot_w(n, b, recip_w(b)), n / b)) { bad1++; last1 = i + 1; }
+    } else if (CASE == 5) {
+      const uint64_t ha = cr_hash(i, 0x2545F491u), hb = cr_hash(i, 0x9E3779B9u), hc = cr_hash(i, 0x85EBCA6Bu);
+      const uint64_t ones = 0xFFFFFFFFFFFFFull;
+      const uint64_t ma = (ha << 20 | (hc & 0xFFFFFu)) & ones, mb = (hb << 20 | hc >> 12) & ones;
+      // exponents: x 2^-700 .. 2^899, a 2^-690 .. 2^359, b 2^-36 .. 2^63, d 1 .. 2^399
+      const uint64_t ex = 1023 - 700 + hc % 1600, ea = 1023 - 690 + (hc >> 3) % 1050, eb = 1023 - 36 + (hc >> 5) % 100,
+                     ed = 1023 + (hc >> 7) % 400;
+      const uint64_t mx = i & 1 ? ma & 0xFFF : ma, md = i & 1 ? ones - (mb & 0xFFF) : mb;
+      const double x = i < 2 ? 0.0 : __longlong_as_double((long long)(ex << 52 | mx));
+      const double a = __longlong_as_double((long long)((ha >> 31) << 63 | ea << 52 | ma));
+      const double b = __longlong_as_double((long long)(eb << 52 | md)), d = __longlong_as_double((long long)(ed << 52 | md));
+      if (!cr_same(root0_w(x), __builtin_sqrt(x))) { bad0++; last0 = i + 1; }
+      if (!cr_same(quot_w(a, b, recip_w(b)), a / b) || !cr_same(unit_quot_w(1.0, d), 1.0 / d) ||
+          !cr_same(unit_quot_w(2.0, d), 2.0 / d)) { bad1++; last1 = i + 1; }
     } else {
       const uint32_t dv[4] = {0x3FFFFFFFu, 0x3F800001u, 0x3F7FFFFFu, 0x40400000u};
       const float a = __uint_as_float((uint32_t)i);
@@ -271,7 +290,7 @@ int gs_bench_valu(float* out, int blocks, int iters, int mode, void* stream) {
 }
 
 int gs_crmath_check(int which, unsigned long long* counts_dev, void* stream) {
-  if (!counts_dev || which < 0 || which > 4) return fail(GS_E_ARG, "gs_crmath_check: counts and which in 0..4 required");
+  if (!counts_dev || which < 0 || which > 5) return fail(GS_E_ARG, "gs_crmath_check: counts and which in 0..5 required");
   hipStream_t s = (hipStream_t)stream;
   const dim3 g(8192), b(256);
   switch (which) {
@@ -279,6 +298,7 @@ int gs_crmath_check(int which, unsigned long long* counts_dev, void* stream) {
     case 1: hipLaunchKernelGGL(k_crmath_check<1>, g, b, 0, s, counts_dev); break;
     case 2: hipLaunchKernelGGL(k_crmath_check<2>, g, b, 0, s, counts_dev); break;
     case 4: hipLaunchKernelGGL(k_crmath_check<4>, g, b, 0, s, counts_dev); break;
+    case 5: hipLaunchKernelGGL(k_crmath_check<5>, g, b, 0, s, counts_dev); break;
     default: hipLaunchKernelGGL(k_crmath_check<3>, g, b, 0, s, counts_dev); break;
   }
   GS_HIP(hipGetLastError(), "k_crmath_check launch");

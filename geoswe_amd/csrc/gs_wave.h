@@ -276,8 +276,8 @@ GS_HD double vfma(double a, double b, double c) { return fma(a, b, c); }
 // ---------------------------------------------------------------------------
 // quotients and roots away from the ends of the exponent range
 // ---------------------------------------------------------------------------
-// RN(1/b). float32: one Newton step on v_rcp_f32, correctly rounded (gs_crmath.h). float64: the
-// two steps of the compiler's own division.
+// 1/b. float32: one Newton step on v_rcp_f32, correctly rounded (gs_crmath.h). float64: the two
+// steps of the compiler's own division, RN(1/b) but for a few b beside a midpoint.
 GS_HD float recip_w(float b) { return cr_recip_refine(b, rcp_approx(b)); }
 GS_HD double recip_w(double b) {
   double y = rcp_approx(b);
@@ -292,6 +292,11 @@ GS_HD T quot_w(T a, T b, T y) {
   const T q = a * y;
   return vfma(-vfma(b, q, -a), y, q);
 }
+// RN(a/d) for a = 1 or 2 and d >= 1. The float64 reciprocal is not RN(1/d) for every d (not, on the
+// device, for 0.15 % of the significands within 2^12 ulps below 2), so it takes the quotient's
+// correction, as the division of the general functions does.
+GS_HD float unit_quot_w(float a, float d) { return a * recip_w(d); }
+GS_HD double unit_quot_w(double a, double d) { return quot_w(a, d, recip_w(d)); }
 // RN(sqrt(x)) from y = v_rsq_f32(x): s = x*y, then one correction by the exact remainder
 // (x - s*s)*(y/2). Over every float32 x >= 2^-96 the device result equals the general root's
 // (the crmath check's third test). float64: the compiler's own sequence without its scaling.
@@ -655,14 +660,14 @@ GS_HD void update_w(T q0, T q1, T q2, T rr0, T r1, T r2, T n, lmask act, const P
     const T Cf = ((w.g * n) * n) * h43;
     T alpha;
     if (P.quadratic) {
-      // alpha = 2 / (sqrt(1 + 2*two) + 1), where RN(2/d) = 2 RN(1/d); doubled where (2*dt)*Cf would
-      // overflow, so that it does here too
+      // alpha = 2 / (sqrt(1 + 2*two) + 1); doubled where (2*dt)*Cf would overflow, so that it does
+      // here too
       const T dtCf = w.dt * Cf;
       const T two = (dtCf + dtCf) * modU;
-      alpha = T(2) * recip_w(root_w(vfma(T(2), two, T(1))) + T(1));
+      alpha = unit_quot_w(T(2), root_w(vfma(T(2), two, T(1))) + T(1));
     } else {
       const T d = T(1) + (w.dt * Cf) * modU;
-      alpha = recip_w(d);
+      alpha = unit_quot_w(T(1), d);
       odd = odd | (lm_gt(d, Range<T>::hi()) & live);   // alpha may be subnormal
     }
     hu = hu * alpha;

@@ -545,7 +545,8 @@ int gs_bench_valu(float* out, int blocks, int iters, int mode, void* stream);
  * float32 b; 1: sqrt(x) for every x (the guarded form; the short form where |x| is outside (0, 2^-96));
  * 2: a/b for 2^32 seeded bit-pattern pairs; 3: a/b for every a over four divisors of hard
  * significands; 4: the sweeps' shorter root for every x >= 2^-96 and 0, and their shorter
- * quotient for 2^32 seeded pairs within its bounds. counts_dev (4 x uint64, zeroed by the caller) receives, per check, the
+ * quotient for 2^32 seeded pairs within its bounds; 5: the float64 forms of both for 2^30 seeded
+ * operands. counts_dev (4 x uint64, zeroed by the caller) receives, per check, the
  * mismatch count and 1 + the largest offending index. No reference counterpart. */
 int gs_crmath_check(int which, unsigned long long* counts_dev, void* stream);
 
