@@ -1433,8 +1433,11 @@ static int flat_step_t(const GsFlat* f, const GsPhys* p, GsForcing fo, GsClock* 
   a.pre[0] = (T*)pre0;
   a.pre[1] = (T*)pre1;
   a.pre[2] = (T*)pre2;
-  if (smp && a.n_tiles > 0 && !pre0 && !(a.ga_ks || a.ga_inv_tau || a.rain_mode == 3) && flat_lean(a)) {
-    a.smp_ids = smp->ids;   // by a wavefront of the sweep, on its way
+  if (smp && a.n_tiles > 0 && a.n_rmode == 0 && !pre0 && !(a.ga_ks || a.ga_inv_tau || a.rain_mode == 3) &&
+      flat_lean(a)) {
+    // by a wavefront of the sweep, on its way (not where a ring mode overwrites cells of the sweep's
+    // input ahead of it)
+    a.smp_ids = smp->ids;
     a.smp_n = smp->n;
     a.smp_out = (T*)smp->out;
   } else if (smp) {
