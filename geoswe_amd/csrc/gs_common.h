@@ -50,7 +50,6 @@ struct Plan {
   const double* rain_cap;
   const double* stage_t;
   const double* stage_v;
-  double next_dt;   // > 0: the next step's dt, given by the host (as gs_clock_set_dt would after the step)
 };
 
 static inline Plan make_plan(const GsPhys& p, const GsForcing& f) {
@@ -65,7 +64,6 @@ static inline Plan make_plan(const GsPhys& p, const GsForcing& f) {
   pl.rain_cap = f.rain_cap;
   pl.stage_t = f.stage_t;
   pl.stage_v = f.stage_v;
-  pl.next_dt = 0.0;
   return pl;
 }
 
@@ -195,7 +193,7 @@ __device__ __forceinline__ void plan_dt(GsClock* c, const Plan& p, const ClockIn
   plan_forcing(c, p, f, k.t, dt);
 }
 
-// A dt that the host gives (gs_clock_set_dt, or Plan::next_dt from the step before).
+// A dt that the host gives (gs_clock_set_dt, or next_dt of the step before).
 __device__ __forceinline__ void plan_host_dt(GsClock* c, const Plan& p, const ClockIn& k, const ForcIn& f, double dt) {
   c->dt = dt;
   c->dt32 = (float)dt;
@@ -207,8 +205,9 @@ __device__ __forceinline__ void plan_host_dt(GsClock* c, const Plan& p, const Cl
 }
 
 // Called by the last workgroup of a step (advance) or of a CFL pass. k: the clock before it; the
-// forcing tables are searched while the grid's maximum is on its way.
-__device__ __forceinline__ void plan_finish(GsClock* c, const Plan& p, ClockIn k, bool advance) {
+// forcing tables are searched while the grid's maximum is on its way. next_dt > 0: the next step's dt,
+// given by the host (as gs_clock_set_dt would after the step).
+__device__ __forceinline__ void plan_finish(GsClock* c, const Plan& p, ClockIn k, bool advance, double next_dt = 0.0) {
   const uint64_t lam = __hip_atomic_load(&c->lam_acc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   if (advance) {
     k.t = k.t + k.dt;
@@ -223,10 +222,10 @@ __device__ __forceinline__ void plan_finish(GsClock* c, const Plan& p, ClockIn k
   c->lam_bits = lam;
   c->lam_acc = 0ull;
   c->blocks_done = 0u;
-  if (p.next_dt > 0.0) {
+  if (next_dt > 0.0) {
     const double l = __longlong_as_double((long long)lam);
     if (!(l == l) || isinf(l)) k.status |= GS_ST_NONFINITE;
-    plan_host_dt(c, p, k, f, p.next_dt);
+    plan_host_dt(c, p, k, f, next_dt);
   } else {
     plan_dt(c, p, k, f, lam);
   }
@@ -282,7 +281,8 @@ __device__ __forceinline__ void await_atomic(uint64_t v) { __asm__ volatile("" :
 // of the line that the atomics are queueing for waits in their queue (with one in every workgroup a
 // 2048^2 coastal step took 69 us instead of 40).
 template <typename K>
-__device__ __forceinline__ void grid_reduce_and_plan(K key, GsClock* c, const Plan& p, bool advance) {
+__device__ __forceinline__ void grid_reduce_and_plan(K key, GsClock* c, const Plan& p, bool advance,
+                                                     double next_dt = 0.0) {
   __shared__ K s_w[16];
   const K top = wave_max(key);
   const int wave = threadIdx.x >> 6;
@@ -297,7 +297,7 @@ __device__ __forceinline__ void grid_reduce_and_plan(K key, GsClock* c, const Pl
   if (m)
     await_atomic(__hip_atomic_fetch_max(&c->lam_acc, lam_key_bits64(m), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
   const unsigned int prev = __hip_atomic_fetch_add(&c->blocks_done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  if (prev == gridDim.x - 1) plan_finish(c, p, clock_read(c), advance);
+  if (prev == gridDim.x - 1) plan_finish(c, p, clock_read(c), advance, next_dt);
 }
 
 // ---------------------------------------------------------------------------

@@ -34,10 +34,14 @@ constexpr int kSweepWaves = sizeof(T) == 4 ? 8 : 4;
 template <typename T>
 constexpr int kSBlock = 64 * kSweepWaves<T>;
 
+// One domain, as its kernels read it; also a member's view in the ensemble's table, of which
+// gs_ens_run_noalloc keeps a promised number in a fixed scratch: what belongs to one launch alone is
+// in FlatLaunch.
 template <typename T>
 struct FlatK {
   int64_t n;
   int n_runs, nyp, ngh;
+  int wave;         // kWave* flags of P; 0 too where a tile's rows may span 2 GiB
   int64_t nchunks;
   T* buf[2][3];
   const T* bed;
@@ -56,7 +60,6 @@ struct FlatK {
   const int32_t* run_d;
   const int32_t* chunk_run;
   Phys<T> P;
-  int wave;         // kWave* flags of P; 0 too where a tile's rows may span 2 GiB
   int rain_mode;
   const T* rain_frames;
   int64_t frame_stride, rain_pitch;
@@ -88,14 +91,20 @@ struct FlatK {
   const int64_t* fring;
   const int32_t* fring_row;  // nullable: gauge-ring row of each entry, -1 for none
   int ring_ng, ring_nt;
-  const int64_t* smp_ids;  // lean sweep: depths of the step's input state at smp_n ids into smp_out
-  int smp_n;
-  T* smp_out;
-  unsigned ring_blocks;  // first workgroups of a sweep that take the ring cells (a multiple of 8, 0: none)
   const T* ring_bed;
   const T* ring_w;
   const double* ring_t;
   const T* ring_stage;
+};
+
+// What one launch of a step adds.
+template <typename T>
+struct FlatLaunch {
+  double next_dt = 0.0;               // > 0: the dt that the step's plan takes for the step after it
+  const int64_t* smp_ids = nullptr;   // lean sweep: depths of the step's input state at smp_n ids into smp_out
+  T* smp_out = nullptr;
+  int smp_n = 0;
+  unsigned ring_blocks = 0;           // first workgroups of a sweep that take the ring cells (a multiple of 8, 0: none)
 };
 
 
@@ -317,6 +326,18 @@ __device__ __forceinline__ const GS_C FlatK<T>* kernel_arg() {   // a kernel who
   return (const GS_C FlatK<T>*)__builtin_amdgcn_kernarg_segment_ptr();
 #else
   return nullptr;
+#endif
+}
+
+// The next_dt of a kernel whose arguments are a FlatK<T> and a FlatLaunch<T>, read where it is used
+// (held through the row loop it cost the lean sweep spilled lanes: 290 lane reads instead of 219).
+template <typename T>
+__device__ __forceinline__ double next_dt_arg() {
+#if defined(__HIP_DEVICE_COMPILE__)
+  static_assert(sizeof(FlatK<T>) % alignof(FlatLaunch<T>) == 0, "the second argument follows the first");
+  return ((const GS_C FlatLaunch<T>*)(cold_ptr<T>(kernel_arg<T>()) + 1))->next_dt;
+#else
+  return 0.0;
 #endif
 }
 
@@ -986,7 +1007,7 @@ __device__ __forceinline__ unsigned xcd_rank(unsigned b, unsigned nb) {
 
 // One step of one flat domain on a resident grid, each wavefront striding over chunks.
 template <typename T, int MODE>
-__global__ __launch_bounds__(kFBlock) void k_flat_step(FlatK<T> a) {
+__global__ __launch_bounds__(kFBlock) void k_flat_step(FlatK<T> a, double next_dt) {
   const FlatClk<T> ck = flat_clock<T, MODE>(a);
   if (!ck.live) return;   // the whole grid sees the same clock
   FlatCtx<T> x;
@@ -1002,7 +1023,7 @@ __global__ __launch_bounds__(kFBlock) void k_flat_step(FlatK<T> a) {
   for (int64_t chunk = (int64_t)xcd_rank(blockIdx.x, gridDim.x) * (kFBlock / 64) + (threadIdx.x >> 6);
        chunk < a.nchunks; chunk += nwaves)
     flat_chunk<T, MODE>(x, chunk, lane, lam);
-  if (MODE == 1) grid_reduce_and_plan(lam, a.clock, a.plan, true);
+  if (MODE == 1) grid_reduce_and_plan(lam, a.clock, a.plan, true, next_dt);
 }
 
 // The forcings on the ring cells of the band (stored, not active): out = force(in), one thread per
@@ -1075,7 +1096,7 @@ __global__ __launch_bounds__(kFBlock) void k_flat_ring_force(FlatK<T> a) {
 // and wavefront forms now: 2048^2 coastal domain (lean) 63 and 40, 1500^2 with the forcing tail
 // (below) 69 and 57.
 template <typename T, bool PRE, bool LEAN = false>
-__global__ __launch_bounds__(kSBlock<T>) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 6 : 1))) void k_flat_sweep(FlatK<T> a) {
+__global__ __launch_bounds__(kSBlock<T>) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 6 : 1))) void k_flat_sweep(FlatK<T> a, FlatLaunch<T> l) {
   // What waits on nothing but the argument is asked for first: the tile's place, the Manning table
   // and the clock. Each wavefront keeps its own copy of the table, so that none waits for another
   // (2048^2 coastal step: 38.4 us against 39.5; the extended sweep, with fewer registers to spare,
@@ -1083,7 +1104,7 @@ __global__ __launch_bounds__(kSBlock<T>) __attribute__((amdgpu_waves_per_eu(size
   const GS_C FlatK<T>* k = kernel_arg<T>();
   const int lane = threadIdx.x & 63;
   const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const unsigned rb = LEAN || PRE ? 0u : a.ring_blocks;
+  const unsigned rb = LEAN || PRE ? 0u : l.ring_blocks;
   const bool ring = blockIdx.x < rb;
   const int64_t nwaves = (int64_t)(gridDim.x - rb) * kSweepWaves<T>;
   int64_t t = (int64_t)xcd_rank(blockIdx.x - rb, gridDim.x - rb) * kSweepWaves<T> + wv;
@@ -1091,9 +1112,9 @@ __global__ __launch_bounds__(kSBlock<T>) __attribute__((amdgpu_waves_per_eu(size
   __shared__ T s_ntab[kSweepWaves<T>][GS_MAX_CLASSES];
   const T n_mine = lane < a.n_classes ? gp(a.ntab)[lane] : T(0);
   const FlatClk<T> ck = flat_clock<T, 1>(a);
-  if (LEAN && a.smp_n > 0 && blockIdx.x == gridDim.x - 1 && wv == 0) {
+  if (LEAN && l.smp_n > 0 && blockIdx.x == gridDim.x - 1 && wv == 0) {
     const GS_G T* h0 = gp(ck.par ? a.buf[1][0] : a.buf[0][0]);
-    for (int i = lane; i < a.smp_n; i += 64) gp(a.smp_out)[i] = h0[gp(a.smp_ids)[i]];
+    for (int i = lane; i < l.smp_n; i += 64) gp(l.smp_out)[i] = h0[gp(l.smp_ids)[i]];
   }
   if (!ck.live) return;   // the whole grid sees the same clock
   FlatCtx<T> x;
@@ -1111,14 +1132,14 @@ __global__ __launch_bounds__(kSBlock<T>) __attribute__((amdgpu_waves_per_eu(size
     t += nwaves;
     if (t < a.n_tiles) h = tile_head<T>(cold_ptr<T>(k), t);
   }
-  grid_reduce_and_plan(lam, a.clock, a.plan, true);
+  grid_reduce_and_plan(lam, a.clock, a.plan, true, next_dt_arg<T>());
 }
 
 // The sweep with the extended forcings compiled in: Green-Ampt infiltration, drain-tau and
 // rain read through a per-cell lookup into a native-grid table (launched only when one of
 // them is set).
 template <typename T>
-__global__ __launch_bounds__(kSBlock<T>) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 6 : 1))) void k_flat_sweep_ext(FlatK<T> a) {
+__global__ __launch_bounds__(kSBlock<T>) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 6 : 1))) void k_flat_sweep_ext(FlatK<T> a, FlatLaunch<T> l) {
   const FlatClk<T> ck = flat_clock<T, 1>(a);
   if (!ck.live) return;
   FlatCtx<T> x;
@@ -1130,7 +1151,7 @@ __global__ __launch_bounds__(kSBlock<T>) __attribute__((amdgpu_waves_per_eu(size
   x.ntab = s_ntab;
   const int lane = threadIdx.x & 63;
   const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const unsigned rb = a.ring_blocks;
+  const unsigned rb = l.ring_blocks;
   const bool ring = blockIdx.x < rb;
   const int64_t nwaves = (int64_t)(gridDim.x - rb) * kSweepWaves<T>;
   lam_t<T> lam = 0;
@@ -1138,7 +1159,7 @@ __global__ __launch_bounds__(kSBlock<T>) __attribute__((amdgpu_waves_per_eu(size
   for (int64_t t = (int64_t)xcd_rank(blockIdx.x - rb, gridDim.x - rb) * kSweepWaves<T> + wv; !ring && t < a.n_tiles;
        t += nwaves)
     flat_tile<T, false, true>(x, tile_head<T>(cold_ptr<T>(x.k), t), lane, lam);
-  grid_reduce_and_plan(lam, a.clock, a.plan, true);
+  grid_reduce_and_plan(lam, a.clock, a.plan, true, next_dt_arg<T>());
 }
 
 // The ring modes of the cached replay on the step's input state, before the step reads
@@ -1369,7 +1390,7 @@ static void flat_launch_choice(const FlatK<T>& a, int* kernel, int64_t* blocks, 
 
 // The fused step: row-sweep tiles when the descriptor has them, else chunks of the run table.
 template <typename T>
-static int flat_step_launch(FlatK<T>& a, hipStream_t s) {
+static int flat_step_launch(const FlatK<T>& a, FlatLaunch<T> l, hipStream_t s) {
   if (a.n_rmode > 0) {
     const int64_t nb = (a.n_rmode + kFBlock - 1) / kFBlock;
     hipLaunchKernelGGL((k_flat_ring_mode<T>), dim3((unsigned)(nb < 1024 ? nb : 1024)), dim3(kFBlock), 0, s, a);
@@ -1381,7 +1402,7 @@ static int flat_step_launch(FlatK<T>& a, hipStream_t s) {
     // 8 us beside a 46 us sweep: 1500^2 with the forcing tail 547 -> 484 us for 10 steps); the lean
     // sweep, which only a gauge ring by itself would bring here, has no register for them
     const int64_t nb = (a.n_fring + kSBlock<T> - 1) / kSBlock<T>;
-    a.ring_blocks = (unsigned)(((nb < 1024 ? nb : 1024) + 7) / 8 * 8);
+    l.ring_blocks = (unsigned)(((nb < 1024 ? nb : 1024) + 7) / 8 * 8);
   } else if (a.n_fring > 0) {
     const int64_t nb = (a.n_fring + kFBlock - 1) / kFBlock;
     hipLaunchKernelGGL((k_flat_ring_force<T>), dim3((unsigned)(nb < 1024 ? nb : 1024)), dim3(kFBlock), 0, s, a);
@@ -1389,22 +1410,22 @@ static int flat_step_launch(FlatK<T>& a, hipStream_t s) {
   }
   if (a.n_tiles > 0 && a.pre[0] && !ext && flat_lean(a)) {
     // 1536^2 adjoint: 33.5 us against the general pre-friction sweep's 36
-    hipLaunchKernelGGL((k_flat_sweep<T, true, true>), dim3(sweep_grid<T>(a.n_tiles)), dim3(kSBlock<T>), 0, s, a);
+    hipLaunchKernelGGL((k_flat_sweep<T, true, true>), dim3(sweep_grid<T>(a.n_tiles)), dim3(kSBlock<T>), 0, s, a, l);
     GS_HIP(hipGetLastError(), "k_flat_sweep(pre, lean) launch");
   } else if (a.n_tiles > 0 && a.pre[0]) {
-    hipLaunchKernelGGL((k_flat_sweep<T, true>), dim3(sweep_grid<T>(a.n_tiles)), dim3(kSBlock<T>), 0, s, a);
+    hipLaunchKernelGGL((k_flat_sweep<T, true>), dim3(sweep_grid<T>(a.n_tiles)), dim3(kSBlock<T>), 0, s, a, l);
     GS_HIP(hipGetLastError(), "k_flat_sweep(pre) launch");
   } else if (a.n_tiles > 0 && ext) {
-    hipLaunchKernelGGL((k_flat_sweep_ext<T>), dim3(sweep_grid<T>(a.n_tiles) + a.ring_blocks), dim3(kSBlock<T>), 0, s, a);
+    hipLaunchKernelGGL((k_flat_sweep_ext<T>), dim3(sweep_grid<T>(a.n_tiles) + l.ring_blocks), dim3(kSBlock<T>), 0, s, a, l);
     GS_HIP(hipGetLastError(), "k_flat_sweep_ext launch");
   } else if (a.n_tiles > 0 && flat_lean(a)) {
-    hipLaunchKernelGGL((k_flat_sweep<T, false, true>), dim3(sweep_grid<T>(a.n_tiles)), dim3(kSBlock<T>), 0, s, a);
+    hipLaunchKernelGGL((k_flat_sweep<T, false, true>), dim3(sweep_grid<T>(a.n_tiles)), dim3(kSBlock<T>), 0, s, a, l);
     GS_HIP(hipGetLastError(), "k_flat_sweep(lean) launch");
   } else if (a.n_tiles > 0) {
-    hipLaunchKernelGGL((k_flat_sweep<T, false>), dim3(sweep_grid<T>(a.n_tiles) + a.ring_blocks), dim3(kSBlock<T>), 0, s, a);
+    hipLaunchKernelGGL((k_flat_sweep<T, false>), dim3(sweep_grid<T>(a.n_tiles) + l.ring_blocks), dim3(kSBlock<T>), 0, s, a, l);
     GS_HIP(hipGetLastError(), "k_flat_sweep launch");
   } else {
-    hipLaunchKernelGGL((k_flat_step<T, 1>), dim3(flat_grid<T, 1>(a.nchunks)), dim3(kFBlock), 0, s, a);
+    hipLaunchKernelGGL((k_flat_step<T, 1>), dim3(flat_grid<T, 1>(a.nchunks)), dim3(kFBlock), 0, s, a, l.next_dt);
     GS_HIP(hipGetLastError(), "k_flat_step launch");
   }
   return GS_OK;
@@ -1426,7 +1447,8 @@ static int flat_step_t(const GsFlat* f, const GsPhys* p, GsForcing fo, GsClock* 
   FlatK<T> a;
   int rc = build_flat<T>(f, p, fo, clk, a, true);
   if (rc) return rc;
-  a.plan.next_dt = next_dt;
+  FlatLaunch<T> l;
+  l.next_dt = next_dt;
   if ((pre0 || pre1 || pre2) && !(pre0 && pre1 && pre2)) return fail(GS_E_ARG, "pre: all three planes or none");
   if (pre0 && a.n_tiles == 0)
     return fail(GS_E_ARG, "the pre-friction state is written by the row-sweep traversal only (n_tiles > 0)");
@@ -1437,15 +1459,15 @@ static int flat_step_t(const GsFlat* f, const GsPhys* p, GsForcing fo, GsClock* 
       flat_lean(a)) {
     // by a wavefront of the sweep, on its way (not where a ring mode overwrites cells of the sweep's
     // input ahead of it)
-    a.smp_ids = smp->ids;
-    a.smp_n = smp->n;
-    a.smp_out = (T*)smp->out;
+    l.smp_ids = smp->ids;
+    l.smp_n = smp->n;
+    l.smp_out = (T*)smp->out;
   } else if (smp) {
     hipLaunchKernelGGL(k_flat_sample<T>, dim3((unsigned)((smp->n + 255) / 256)), dim3(256), 0, s, a, smp->ids, smp->n,
                        (T*)smp->out);
     GS_HIP(hipGetLastError(), "k_flat_sample launch");
   }
-  return flat_step_launch<T>(a, s);
+  return flat_step_launch<T>(a, l, s);
 }
 
 template <typename T>
@@ -1462,7 +1484,7 @@ static int flat_residual_t(const GsFlat* f, const GsPhys* p, int which, void* r0
   a.rhs[0] = (T*)r0;
   a.rhs[1] = (T*)r1;
   a.rhs[2] = (T*)r2;
-  hipLaunchKernelGGL((k_flat_step<T, 0>), dim3(flat_grid<T, 0>(a.nchunks)), dim3(kFBlock), 0, s, a);
+  hipLaunchKernelGGL((k_flat_step<T, 0>), dim3(flat_grid<T, 0>(a.nchunks)), dim3(kFBlock), 0, s, a, 0.0);
   GS_HIP(hipGetLastError(), "k_flat_step(residual) launch");
   return GS_OK;
 }
@@ -2132,10 +2154,11 @@ constexpr size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 // Bytes of scratch the no-allocation run needs for n members (0 if they do not fit).
 template <typename T>
-static size_t noalloc_bytes(int n) {
+static constexpr size_t noalloc_bytes(int n) {
   const size_t need = align256(256 + 8 * ((size_t)n + 1)) + sizeof(FlatK<T>) * (size_t)n;
   return need <= kScratchBytes ? need : 0;
 }
+static_assert(noalloc_bytes<float>(409) && noalloc_bytes<double>(384), "the members that the ABI promises");
 
 template <typename T>
 static int ens_run_noalloc_t(const GsFlat* members, const GsPhys* phys, const GsForcing* forcings,
