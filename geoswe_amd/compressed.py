@@ -576,8 +576,8 @@ class CompressedSolver:
 
     def launch_info(self) -> dict:
         """The step kernel's launch for this solver: ``kernel`` ("chunks", "sweep" or
-        "sweep_ext"), ``blocks`` (its grid) and ``resident`` (that kernel's resident grid on
-        this device; ``blocks > resident`` means one wavefront per tile)."""
+        "sweep_ext"), ``blocks`` (its grid: for a sweep one wavefront per tile, and the workgroups
+        that force ring cells) and ``resident`` (that kernel's resident grid on this device)."""
         k, b, r = C.c_int(0), C.c_int64(0), C.c_int64(0)
         L.call("gs_flat_launch_info", C.byref(self._desc()), C.byref(self._phys()), self._fo.s, C.byref(k),
                C.byref(b), C.byref(r))

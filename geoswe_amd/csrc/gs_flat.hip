@@ -1363,6 +1363,23 @@ static bool flat_lean(const FlatK<T>& a) {
   return !a.n_field && !a.cls && !a.max_h && !a.sponge && !a.clamp && !a.infil && !a.drain;
 }
 
+// The step takes the extended sweep.
+template <typename T>
+static bool flat_ext(const FlatK<T>& a) {
+  return a.ga_ks || a.ga_inv_tau || a.rain_mode == 3;
+}
+
+// The ring cells by workgroups of the sweep itself, ahead of its tiles (a launch of their own took
+// 8 us beside a 46 us sweep: 1500^2 with the forcing tail 547 -> 484 us for 10 steps); the lean sweep,
+// which only a gauge ring by itself would bring here, has no register for them. 0: a launch of their
+// own, or none to force.
+template <typename T>
+static unsigned sweep_ring_blocks(const FlatK<T>& a) {
+  if (a.n_fring <= 0 || a.n_tiles <= 0 || a.pre[0] || !(flat_ext(a) || !flat_lean(a))) return 0;
+  const int64_t nb = (a.n_fring + kSBlock<T> - 1) / kSBlock<T>;
+  return (unsigned)(((nb < 1024 ? nb : 1024) + 7) / 8 * 8);
+}
+
 // The launch gs_flat_step makes for `a` (without the pre-friction state): which kernel, its
 // grid and the kernel's resident grid on this device.
 template <typename T>
@@ -1372,9 +1389,9 @@ static void flat_launch_choice(const FlatK<T>& a, int* kernel, int64_t* blocks, 
     *kernel = 0;
     *blocks = flat_grid<T, 1>(a.nchunks);
     *resident = *blocks;
-  } else if (a.ga_ks || a.ga_inv_tau || a.rain_mode == 3) {
+  } else if (flat_ext(a)) {
     *kernel = 2;
-    *blocks = sweep_grid<T>(a.n_tiles);
+    *blocks = sweep_grid<T>(a.n_tiles) + sweep_ring_blocks(a);
     *resident = resident_grid(k_flat_sweep_ext<T>, c_ext, a.n_tiles, kSBlock<T>);
   } else if (flat_lean(a)) {
     static std::atomic<int> c_lean[64];
@@ -1383,7 +1400,7 @@ static void flat_launch_choice(const FlatK<T>& a, int* kernel, int64_t* blocks, 
     *resident = resident_grid(k_flat_sweep<T, false, true>, c_lean, a.n_tiles, kSBlock<T>);
   } else {
     *kernel = 1;
-    *blocks = sweep_grid<T>(a.n_tiles);
+    *blocks = sweep_grid<T>(a.n_tiles) + sweep_ring_blocks(a);
     *resident = resident_grid(k_flat_sweep<T, false>, c_plain, a.n_tiles, kSBlock<T>);
   }
 }
@@ -1396,14 +1413,9 @@ static int flat_step_launch(const FlatK<T>& a, FlatLaunch<T> l, hipStream_t s) {
     hipLaunchKernelGGL((k_flat_ring_mode<T>), dim3((unsigned)(nb < 1024 ? nb : 1024)), dim3(kFBlock), 0, s, a);
     GS_HIP(hipGetLastError(), "k_flat_ring_mode launch");
   }
-  const bool ext = a.ga_ks || a.ga_inv_tau || a.rain_mode == 3;
-  if (a.n_fring > 0 && a.n_tiles > 0 && !a.pre[0] && (ext || !flat_lean(a))) {
-    // the ring cells by workgroups of the sweep itself, ahead of its tiles (a launch of their own took
-    // 8 us beside a 46 us sweep: 1500^2 with the forcing tail 547 -> 484 us for 10 steps); the lean
-    // sweep, which only a gauge ring by itself would bring here, has no register for them
-    const int64_t nb = (a.n_fring + kSBlock<T> - 1) / kSBlock<T>;
-    l.ring_blocks = (unsigned)(((nb < 1024 ? nb : 1024) + 7) / 8 * 8);
-  } else if (a.n_fring > 0) {
+  const bool ext = flat_ext(a);
+  l.ring_blocks = sweep_ring_blocks(a);
+  if (a.n_fring > 0 && l.ring_blocks == 0) {
     const int64_t nb = (a.n_fring + kFBlock - 1) / kFBlock;
     hipLaunchKernelGGL((k_flat_ring_force<T>), dim3((unsigned)(nb < 1024 ? nb : 1024)), dim3(kFBlock), 0, s, a);
     GS_HIP(hipGetLastError(), "k_flat_ring_force launch");
@@ -1455,8 +1467,7 @@ static int flat_step_t(const GsFlat* f, const GsPhys* p, GsForcing fo, GsClock* 
   a.pre[0] = (T*)pre0;
   a.pre[1] = (T*)pre1;
   a.pre[2] = (T*)pre2;
-  if (smp && a.n_tiles > 0 && a.n_rmode == 0 && !pre0 && !(a.ga_ks || a.ga_inv_tau || a.rain_mode == 3) &&
-      flat_lean(a)) {
+  if (smp && a.n_tiles > 0 && a.n_rmode == 0 && !pre0 && !flat_ext(a) && flat_lean(a)) {
     // by a wavefront of the sweep, on its way (not where a ring mode overwrites cells of the sweep's
     // input ahead of it)
     l.smp_ids = smp->ids;

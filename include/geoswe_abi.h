@@ -351,8 +351,8 @@ int gs_flat_cfl(const GsFlat* f, const GsPhys* phys, GsForcing forc, GsClock* cl
 
 /* No reference counterpart (a launch query for tests and tuning): the kernel gs_flat_step
  * launches for this descriptor (0 chunk traversal, 1 plain row sweep, 2 extended row sweep),
- * its grid in workgroups and that kernel's resident grid on the current device (the grid
- * exceeds it when the step launches one wavefront per tile). No device work. */
+ * its grid in workgroups (for a row sweep one wavefront per tile, and the workgroups that force
+ * ring cells) and that kernel's resident grid on the current device. No device work. */
 int gs_flat_launch_info(const GsFlat* f, const GsPhys* phys, GsForcing forc, int* kernel, int64_t* blocks,
                         int64_t* resident);
 
