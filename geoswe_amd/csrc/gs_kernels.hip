@@ -191,8 +191,9 @@ __device__ __forceinline__ S load_b(const DenseK<T, S>& a, const DenseTile<T, S>
 }
 
 // What a cell's update reads from its planes. Lanes that write nothing read nothing. LEAN: the
-// domain has no flags, Manning, class and running-max plane and no gridded rain.
-template <bool LEAN, typename T, typename S>
+// domain has no flags, Manning, class and running-max plane and no gridded rain. The residual
+// (MODE 0) takes the flags alone: its launch fills in neither the rain nor the Manning table.
+template <int MODE, bool LEAN, typename T, typename S>
 __device__ __forceinline__ void cell_inputs(const DenseK<T, S>& a, const DenseTile<T, S>& x, int i, T& rh, T& rhu,
                                             T& rhv, T& rr0, T& n, uint8_t& fl) {
   fl = 0;
@@ -209,6 +210,7 @@ __device__ __forceinline__ void cell_inputs(const DenseK<T, S>& a, const DenseTi
     if (fl & GS_FLAG_INACTIVE) { rh = T(0); rhu = T(0); rhv = T(0); }
     rr0 = rh;
   }
+  if constexpr (MODE == 0) return;
   if (a.rain_mode == 1) {
     rr0 = rr0 + x.rain;
   } else if (a.rain_mode == 2) {
@@ -373,7 +375,7 @@ __device__ __forceinline__ int dense_rows(const DenseK<T, S>& a, const DenseTile
       mh = cr.mh;
       cb.load(min(i + 1, i_end - 1) - i0, cr);
     } else {
-      cell_inputs<LEAN, T>(a, x, i, rh, rhu, rhv, rr0, n, fl);
+      cell_inputs<MODE, LEAN, T>(a, x, i, rh, rhu, rhv, rr0, n, fl);
     }
     if (MODE == 0) {
       if (lm_any(odd)) return false;
@@ -474,7 +476,7 @@ __device__ __forceinline__ void dense_rows_general(const DenseK<T, S>& a, const 
     T rh, rhu, rhv, rr0, n;
     uint8_t fl;
     sum_faces<T>(fn, fx, fy, lFh, lFN, lFT, lsR, rh, rhu, rhv);
-    cell_inputs<LEAN, T>(a, x, i, rh, rhu, rhv, rr0, n, fl);
+    cell_inputs<MODE, LEAN, T>(a, x, i, rh, rhu, rhv, rr0, n, fl);
     if (MODE == 0) {
       if (x.col_ok) {
         const int64_t idx = (int64_t)i * a.pitch + x.c;
