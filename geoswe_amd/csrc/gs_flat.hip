@@ -317,6 +317,7 @@ __device__ __forceinline__ FlatCtx<T> cold(const FlatCtx<T>& x) {
   y.ga_fmax = gp((T*)k->ga_fmax);
   y.ga_inv_tau = gp((T*)k->ga_inv_tau);
   y.rain_lookup = gp((int32_t*)k->rain_lookup);
+  y.wave = k->wave;
   y.P = const_read((const Phys<T>*)(uint64_t)&k->P);
   return y;
 }
@@ -690,6 +691,16 @@ __device__ __forceinline__ void finish_cell(const FlatCtx<T>& x, const ForceIn<T
 // The tallest tile that flat_rows takes: its rows are addressed with 32-bit offsets.
 constexpr int kWaveRows = 1024;
 
+// The rows of a sweep. The lean sweeps have an instantiation of each: in the lean row the general wave
+// speed beside the quick one cost the L-inf steps 1 to 2 % (2048^2, 20 steps: 764 us against 755). The
+// others decide by the descriptor, in a branch that a forcing takes anyway.
+enum {
+  kRowsQuick,  // wavefront forms, with the L-inf wave speed that the update has made (kWaveLam)
+  kRowsAny,    // wavefront forms, any wave speed (the L2 norm, a CFL floor above h_min)
+};
+template <bool LEAN>
+constexpr int kRowsOf = LEAN ? kRowsQuick : kRowsAny;
+
 // One row of a sweep tile.
 struct FlatRow {
   uint32_t row;        // its first stored id, from the tile's first one (uniform)
@@ -713,7 +724,7 @@ __device__ __forceinline__ FlatRow flat_row(const GS_C uint64_t* e, uint32_t g0)
 // A row's state, flags and rain are loaded one row ahead of their use, its bed two rows ahead and
 // its entry before that. Lanes on unstored cells read 0: no face that an active cell uses reads
 // them.
-template <typename T, bool PRE, bool EXT, bool LEAN>
+template <typename T, bool PRE, bool EXT, bool LEAN, int ROWS>
 __device__ __forceinline__ int flat_rows(const FlatCtx<T>& x, const WaveC<T>& w, const GS_C uint64_t* E, int i0, int nr,
                                          int c0, int lane, lam_t<T>& lam) {
   constexpr uint32_t es = (uint32_t)sizeof(T);
@@ -841,15 +852,17 @@ __device__ __forceinline__ int flat_rows(const FlatCtx<T>& x, const WaveC<T>& w,
         h = lm_sel(stage, pos_w(x.eta - b0), h);
         hu = lm_sel(stage, T(0), hu);
         hv = lm_sel(stage, T(0), hv);
-        speed = speed_w<T>(h, hu, hv, w);
+        if (ROWS == kRowsQuick) speed = speed_w<T>(h, hu, hv, w);
       }
-      key = lam_key_w<T>(speed);
+      if constexpr (ROWS == kRowsQuick) key = lam_key_w<T>(speed);
+      else key = lam_key<T, true>(h, hu, hv, cold(x).P);
     } else {
       const FlatCtx<T> y = cold(x);
       if (lm_lane(act) && !left) finish_cell<T, EXT, LEAN>(y, fin, fg, gC, eC.below * es, b0, h, hu, hv);
       speed = speed_w<T>(h, hu, hv, w);
       key = lam_key_w<T>(speed);
-      if (lm_any(act & lm_not(lm_lt(speed, kMaxSpeed<T>)))) key = lam_key<T, true>(h, hu, hv, cold(x).P);
+      if (!(y.wave & kWaveLam) || lm_any(act & lm_not(lm_lt(speed, kMaxSpeed<T>))))
+        key = lam_key<T, true>(h, hu, hv, cold(x).P);
     }
     // in a row with an odd lane every lane's store is out of range, so that every way to the next
     // row's loads holds the same stores
@@ -984,15 +997,15 @@ __device__ __forceinline__ TileHead tile_head(const GS_C FlatK<T>* k, int64_t t)
 // plain step's scalar registers. LEAN: the domain has no per-cell Manning field or class plane, no
 // running maximum and no active-cell forcing, so none of their pointers is held (the host checks
 // that they are all null).
-template <typename T, bool PRE, bool EXT, bool LEAN = false>
+template <typename T, bool PRE, bool EXT, bool LEAN = false, int ROWS = kRowsOf<LEAN>>
 __device__ __forceinline__ void flat_tile(const FlatCtx<T>& x, const TileHead& h, int lane, lam_t<T>& lam) {
   const int i0 = h.i0, nr = h.nr, c0 = h.c0;
   const GS_C uint64_t* E = h.E;
   int r = 0;
-  constexpr int forms = kWaveFast | kWaveLam;
+  constexpr int forms = ROWS == kRowsQuick ? kWaveFast | kWaveLam : kWaveFast;
   if ((x.wave & forms) == forms && vabs(x.eta) < T(0x1p30) && nr <= kWaveRows) {
     const WaveC<T> w = wave_consts<T>(x.P, x.dt, x.wave);
-    r = __builtin_amdgcn_readfirstlane(flat_rows<T, PRE, EXT, LEAN>(x, w, E, i0, nr, c0, lane, lam));
+    r = __builtin_amdgcn_readfirstlane(flat_rows<T, PRE, EXT, LEAN, ROWS>(x, w, E, i0, nr, c0, lane, lam));
   }
   if (r < nr) flat_rows_general<T, PRE, EXT, LEAN>(x, E + 3 * r, i0 + r, nr - r, c0, lane, lam);
 }
@@ -1095,7 +1108,7 @@ __global__ __launch_bounds__(kFBlock) void k_flat_ring_force(FlatK<T> a) {
 // active-cell forcing) drops those paths. us per step, general functions with 4-row tiles before
 // and wavefront forms now: 2048^2 coastal domain (lean) 63 and 40, 1500^2 with the forcing tail
 // (below) 69 and 57.
-template <typename T, bool PRE, bool LEAN = false>
+template <typename T, bool PRE, bool LEAN = false, int ROWS = kRowsOf<LEAN>>
 __global__ __launch_bounds__(kSBlock<T>) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 6 : 1))) void k_flat_sweep(FlatK<T> a, FlatLaunch<T> l) {
   // What waits on nothing but the argument is asked for first: the tile's place, the Manning table
   // and the clock. Each wavefront keeps its own copy of the table, so that none waits for another
@@ -1128,7 +1141,7 @@ __global__ __launch_bounds__(kSBlock<T>) __attribute__((amdgpu_waves_per_eu(size
   // that a replay reads rain through the per-cell lookup exactly as the forward run's extended sweep
   if (ring) ring_cells<T>(a, x, blockIdx.x, rb);
   while (!ring && t < a.n_tiles) {
-    flat_tile<T, PRE, PRE && !LEAN, LEAN>(x, h, lane, lam);
+    flat_tile<T, PRE, PRE && !LEAN, LEAN, ROWS>(x, h, lane, lam);
     t += nwaves;
     if (t < a.n_tiles) h = tile_head<T>(cold_ptr<T>(k), t);
   }
@@ -1380,6 +1393,23 @@ static unsigned sweep_ring_blocks(const FlatK<T>& a) {
   return (unsigned)(((nb < 1024 ? nb : 1024) + 7) / 8 * 8);
 }
 
+// Its rows, where they may take the wavefront forms, know the wave speed from the update.
+template <typename T>
+static bool flat_quick(const FlatK<T>& a) {
+  return !(a.wave & kWaveFast) || (a.wave & kWaveLam);
+}
+
+// The rows of the lean sweep for `a`.
+template <typename T>
+static int lean_rows(const FlatK<T>& a) {
+  return flat_quick(a) ? kRowsQuick : kRowsAny;
+}
+
+template <typename T, bool PRE>
+static auto lean_sweep(int rows) -> void (*)(FlatK<T>, FlatLaunch<T>) {
+  return rows == kRowsAny ? k_flat_sweep<T, PRE, true, kRowsAny> : k_flat_sweep<T, PRE, true, kRowsQuick>;
+}
+
 // The launch gs_flat_step makes for `a` (without the pre-friction state): which kernel, its
 // grid and the kernel's resident grid on this device.
 template <typename T>
@@ -1394,10 +1424,11 @@ static void flat_launch_choice(const FlatK<T>& a, int* kernel, int64_t* blocks, 
     *blocks = sweep_grid<T>(a.n_tiles) + sweep_ring_blocks(a);
     *resident = resident_grid(k_flat_sweep_ext<T>, c_ext, a.n_tiles, kSBlock<T>);
   } else if (flat_lean(a)) {
-    static std::atomic<int> c_lean[64];
+    static std::atomic<int> c_lean[2][64];
+    const int rows = lean_rows(a);
     *kernel = 1;
     *blocks = sweep_grid<T>(a.n_tiles);
-    *resident = resident_grid(k_flat_sweep<T, false, true>, c_lean, a.n_tiles, kSBlock<T>);
+    *resident = resident_grid(lean_sweep<T, false>(rows), c_lean[rows], a.n_tiles, kSBlock<T>);
   } else {
     *kernel = 1;
     *blocks = sweep_grid<T>(a.n_tiles) + sweep_ring_blocks(a);
@@ -1422,7 +1453,7 @@ static int flat_step_launch(const FlatK<T>& a, FlatLaunch<T> l, hipStream_t s) {
   }
   if (a.n_tiles > 0 && a.pre[0] && !ext && flat_lean(a)) {
     // 1536^2 adjoint: 33.5 us against the general pre-friction sweep's 36
-    hipLaunchKernelGGL((k_flat_sweep<T, true, true>), dim3(sweep_grid<T>(a.n_tiles)), dim3(kSBlock<T>), 0, s, a, l);
+    hipLaunchKernelGGL((lean_sweep<T, true>(lean_rows(a))), dim3(sweep_grid<T>(a.n_tiles)), dim3(kSBlock<T>), 0, s, a, l);
     GS_HIP(hipGetLastError(), "k_flat_sweep(pre, lean) launch");
   } else if (a.n_tiles > 0 && a.pre[0]) {
     hipLaunchKernelGGL((k_flat_sweep<T, true>), dim3(sweep_grid<T>(a.n_tiles)), dim3(kSBlock<T>), 0, s, a, l);
@@ -1431,7 +1462,7 @@ static int flat_step_launch(const FlatK<T>& a, FlatLaunch<T> l, hipStream_t s) {
     hipLaunchKernelGGL((k_flat_sweep_ext<T>), dim3(sweep_grid<T>(a.n_tiles) + l.ring_blocks), dim3(kSBlock<T>), 0, s, a, l);
     GS_HIP(hipGetLastError(), "k_flat_sweep_ext launch");
   } else if (a.n_tiles > 0 && flat_lean(a)) {
-    hipLaunchKernelGGL((k_flat_sweep<T, false, true>), dim3(sweep_grid<T>(a.n_tiles)), dim3(kSBlock<T>), 0, s, a, l);
+    hipLaunchKernelGGL((lean_sweep<T, false>(lean_rows(a))), dim3(sweep_grid<T>(a.n_tiles)), dim3(kSBlock<T>), 0, s, a, l);
     GS_HIP(hipGetLastError(), "k_flat_sweep(lean) launch");
   } else if (a.n_tiles > 0) {
     hipLaunchKernelGGL((k_flat_sweep<T, false>), dim3(sweep_grid<T>(a.n_tiles) + l.ring_blocks), dim3(kSBlock<T>), 0, s, a, l);
@@ -1563,7 +1594,8 @@ __device__ __forceinline__ int ens_member_of(const int64_t* tile0, int n, int64_
 // of them), and its float32 build is held to 96 VGPRs (5 wavefronts per SIMD, nothing spilled; at
 // 80 and 6 the row loop reloads, and 16 members of 256 to 1024 cells a side took 90 us per step at
 // 8 rows a tile against 84).
-enum { kEnsPlain = 0, kEnsExt = 1, kEnsLean = 2 };
+// kEnsLeanAny is kEnsLean where some member's wave speed is not the quick one (kRowsAny).
+enum { kEnsPlain = 0, kEnsExt = 1, kEnsLean = 2, kEnsLeanAny = 3 };
 
 // The members' clock statuses side by side, for one copy to the host.
 template <typename T>
@@ -1572,7 +1604,7 @@ __global__ void k_ens_status(const FlatK<T>* mem, int n, int* out) {
 }
 
 template <typename T, int KIND>
-__global__ __launch_bounds__(kFBlock) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && KIND == kEnsLean ? 5 : 1)))
+__global__ __launch_bounds__(kFBlock) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && KIND >= kEnsLean ? 5 : 1)))
 void k_ens_step(EnsK<T> e, const FlatK<T>* __restrict__ mem, const int64_t* __restrict__ tile0) {
   const int lane = threadIdx.x & 63;
   const int64_t nwaves = (int64_t)gridDim.x * (kFBlock / 64);
@@ -1604,7 +1636,8 @@ void k_ens_step(EnsK<T> e, const FlatK<T>* __restrict__ mem, const int64_t* __re
       flat_ctx<T, 1>(v, ck, x);
       x.k = cp((const GS_G FlatK<T>*)(mem + mt));
       x.ntab = s_ntab[wv];
-      flat_tile<T, false, KIND == kEnsExt, KIND == kEnsLean>(x, tile_head<T>(x.k, gc - const_read(tile0 + mt)), lane, lam);
+      flat_tile<T, false, KIND == kEnsExt, (KIND >= kEnsLean), KIND == kEnsLean ? kRowsQuick : kRowsAny>(
+          x, tile_head<T>(x.k, gc - const_read(tile0 + mt)), lane, lam);
     }
   }
   __shared__ int s_m[kFBlock / 64];
@@ -1642,12 +1675,19 @@ void k_ens_step(EnsK<T> e, const FlatK<T>* __restrict__ mem, const int64_t* __re
 }
 
 template <typename T>
+static auto ens_kernel(int kind) -> void (*)(EnsK<T>, const FlatK<T>*, const int64_t*) {
+  switch (kind) {
+    case kEnsExt: return k_ens_step<T, kEnsExt>;
+    case kEnsLean: return k_ens_step<T, kEnsLean>;
+    case kEnsLeanAny: return k_ens_step<T, kEnsLeanAny>;
+    default: return k_ens_step<T, kEnsPlain>;
+  }
+}
+
+template <typename T>
 static int ens_occupancy(int kind) {
   int occ = 0;
-  const hipError_t h =
-      kind == kEnsExt    ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k_ens_step<T, kEnsExt>, kFBlock, 0)
-      : kind == kEnsLean ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k_ens_step<T, kEnsLean>, kFBlock, 0)
-                         : hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k_ens_step<T, kEnsPlain>, kFBlock, 0);
+  const hipError_t h = hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, ens_kernel<T>(kind), kFBlock, 0);
   if (h != hipSuccess || occ < 1) occ = 1;
   return occ;
 }
@@ -1656,22 +1696,18 @@ static int ens_occupancy(int kind) {
 // if every member may take the lean sweep, else plain.
 template <typename T>
 static int ens_kind(const FlatK<T>* views, int n) {
-  bool lean = true;
+  bool lean = true, quick = true;
   for (int m = 0; m < n; ++m) {
-    if (views[m].ga_ks || views[m].ga_inv_tau || views[m].rain_mode == 3) return kEnsExt;
+    if (flat_ext(views[m])) return kEnsExt;
     lean = lean && flat_lean(views[m]);
+    quick = quick && flat_quick(views[m]);
   }
-  return lean ? kEnsLean : kEnsPlain;
+  return !lean ? kEnsPlain : quick ? kEnsLean : kEnsLeanAny;
 }
 
 template <typename T>
 static void ens_launch_kind(int kind, int64_t blocks, hipStream_t s, const EnsK<T>& k) {
-  if (kind == kEnsExt)
-    hipLaunchKernelGGL((k_ens_step<T, kEnsExt>), dim3((unsigned)blocks), dim3(kFBlock), 0, s, k, k.mem, k.tile0);
-  else if (kind == kEnsLean)
-    hipLaunchKernelGGL((k_ens_step<T, kEnsLean>), dim3((unsigned)blocks), dim3(kFBlock), 0, s, k, k.mem, k.tile0);
-  else
-    hipLaunchKernelGGL((k_ens_step<T, kEnsPlain>), dim3((unsigned)blocks), dim3(kFBlock), 0, s, k, k.mem, k.tile0);
+  hipLaunchKernelGGL((ens_kernel<T>(kind)), dim3((unsigned)blocks), dim3(kFBlock), 0, s, k, k.mem, k.tile0);
 }
 
 int flat_step_next(const GsFlat* f, const GsPhys* phys, const GsForcing& forc, GsClock* clock_dev, void* const* pre,
