@@ -98,7 +98,7 @@ class CompressedSolver:
         nxp, nyp = nx + 2 * g, ny + 2 * g
         inside = np.zeros((nxp, nyp), bool)
         inside[g:g + nx, g:g + ny] = s.inside_mask if s.inside_mask is not None else True
-        fm = build_flat_mesh(inside, g, ring=2, sweep_rows=sweep_rows)
+        fm = build_flat_mesh(inside, g, ring=2, sweep_rows=sweep_rows, dtype=s.dtype)
         q_pad = s.q                                  # ghosts filled from the boundary kinds
         b_pad = s.b
         flags = np.zeros((nxp, nyp), np.uint8)

@@ -70,10 +70,13 @@ class FlatMesh:
 
 
 def build_flat_mesh(inside_padded: np.ndarray, ngh: int, ring: int = 2, sweep_rows: int = None,
-                    native: bool = True) -> FlatMesh:
+                    native: bool = True, dtype=np.float32) -> FlatMesh:
     """Stored set, flat order, run table and row-sweep tiles of an active mask given on the
     padded grid. `native`: the library's host builder (gs_flat_mesh_build, one pass with
-    rolling rows); otherwise the NumPy restatement below, which produces the same arrays."""
+    rolling rows); otherwise the NumPy restatement below, which produces the same arrays.
+    `dtype`: the state's, which the tile height goes with unless `sweep_rows` gives it."""
+    if sweep_rows is None and np.dtype(dtype) == np.float64:
+        sweep_rows = sweep_rows_for64(window_rows(inside_padded))
     if native:
         return _build_native(inside_padded, ngh, ring, sweep_rows)
     inside = np.asarray(inside_padded, dtype=bool)
@@ -202,6 +205,31 @@ def sweep_rows_for(busy: int) -> int:
     busy = int(busy)
     rows = max(math.isqrt(busy // 1000), busy // (2 * TILE_TARGET) + 1)
     return max(1, min(rows, busy // TILE_TARGET, MAX_SWEEP_ROWS))
+
+
+def sweep_rows_for64(busy: int) -> int:
+    """The same for the float64 sweeps, of which an MI355X holds 3072 wavefronts at once: the height that
+    makes one round of them (at least 2 rows from 1000 window rows on), up to 9 rows; beyond, the
+    float32 height.
+
+    A round that is nearly empty costs most: coastal domains, us per lean step at heights 1/2/3/4: 1100
+    busy rows 17.8/17.0, 3400 28.1/21.4/22.7, 5500 34.0/25.7/24.6/26.0, 7137 39.1/31.2/27.4/26.7, 10756
+    (from 2) 40.0/36.3/33.0, at 5 35.6; 14700 at 3/4/5/6 42.0/40.3/37.4/39.8, 19500 at 4/5/6/7/8
+    52.5/52.4/51.3/46.0/48.5, 25000 at 5/8/9/10 55.1/59.5/53.0/56.5; 51000 at 6/7/8/9 91.8/92.7/91.8/89.4 and
+    in one round of 17 86, but 43000 at 8/14/15 84/91/94. (The float32 rule gives 1 row up to 9215.)"""
+    rows = -(-int(busy) // 3000)
+    if rows > 9:
+        return sweep_rows_for(busy)
+    return max(rows, 2 if busy >= 1000 else 1)
+
+
+def window_rows(inside: np.ndarray) -> int:
+    """Rows of the windows of the column grid (written lanes 2..61 of 64 columns from CHUNK*k) with an
+    active cell: what sweep_rows_for counts."""
+    inside = np.asarray(inside, dtype=bool)
+    if inside.ndim != 2 or inside.shape[1] <= 2:
+        return 0
+    return int(np.count_nonzero(np.logical_or.reduceat(inside, np.arange(2, inside.shape[1], CHUNK), axis=1)))
 
 
 def mesh_sweep_tiles(fm: "FlatMesh", rows: int):
