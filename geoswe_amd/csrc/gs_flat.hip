@@ -695,8 +695,9 @@ constexpr int kWaveRows = 1024;
 // speed beside the quick one cost the L-inf steps 1 to 2 % (2048^2, 20 steps: 764 us against 755). The
 // others decide by the descriptor, in a branch that a forcing takes anyway.
 enum {
-  kRowsQuick,  // wavefront forms, with the L-inf wave speed that the update has made (kWaveLam)
-  kRowsAny,    // wavefront forms, any wave speed (the L2 norm, a CFL floor above h_min)
+  kRowsQuick,    // wavefront forms, with the L-inf wave speed that the update has made (kWaveLam)
+  kRowsAny,      // wavefront forms, any wave speed (the L2 norm, a CFL floor above h_min)
+  kRowsGeneral,  // the general functions alone
 };
 template <bool LEAN>
 constexpr int kRowsOf = LEAN ? kRowsQuick : kRowsAny;
@@ -1002,10 +1003,12 @@ __device__ __forceinline__ void flat_tile(const FlatCtx<T>& x, const TileHead& h
   const int i0 = h.i0, nr = h.nr, c0 = h.c0;
   const GS_C uint64_t* E = h.E;
   int r = 0;
-  constexpr int forms = ROWS == kRowsQuick ? kWaveFast | kWaveLam : kWaveFast;
-  if ((x.wave & forms) == forms && vabs(x.eta) < T(0x1p30) && nr <= kWaveRows) {
-    const WaveC<T> w = wave_consts<T>(x.P, x.dt, x.wave);
-    r = __builtin_amdgcn_readfirstlane(flat_rows<T, PRE, EXT, LEAN, ROWS>(x, w, E, i0, nr, c0, lane, lam));
+  if constexpr (ROWS != kRowsGeneral) {
+    constexpr int forms = ROWS == kRowsQuick ? kWaveFast | kWaveLam : kWaveFast;
+    if ((x.wave & forms) == forms && vabs(x.eta) < T(0x1p30) && nr <= kWaveRows) {
+      const WaveC<T> w = wave_consts<T>(x.P, x.dt, x.wave);
+      r = __builtin_amdgcn_readfirstlane(flat_rows<T, PRE, EXT, LEAN, ROWS>(x, w, E, i0, nr, c0, lane, lam));
+    }
   }
   if (r < nr) flat_rows_general<T, PRE, EXT, LEAN>(x, E + 3 * r, i0 + r, nr - r, c0, lane, lam);
 }
@@ -1399,14 +1402,20 @@ static bool flat_quick(const FlatK<T>& a) {
   return !(a.wave & kWaveFast) || (a.wave & kWaveLam);
 }
 
-// The rows of the lean sweep for `a`.
+// The rows of the lean sweep for `a`. A float64 step of up to one wavefront per SIMD is one tile's
+// latency, which the general functions alone have less of (us per step with and without the forms:
+// 64^2 14.1 and 13.4, 150^2 14.3 and 13.6, 400^2 of 864 tiles 18.2 and 18.0; but 500^2 of 1230 tiles 20.7
+// and 20.7, 700^2 of 2250 23.8 and 25.1).
 template <typename T>
 static int lean_rows(const FlatK<T>& a) {
+  if (sizeof(T) == 8 && a.n_tiles <= 1024) return kRowsGeneral;
   return flat_quick(a) ? kRowsQuick : kRowsAny;
 }
 
 template <typename T, bool PRE>
 static auto lean_sweep(int rows) -> void (*)(FlatK<T>, FlatLaunch<T>) {
+  if constexpr (sizeof(T) == 8)
+    if (rows == kRowsGeneral) return k_flat_sweep<T, PRE, true, kRowsGeneral>;
   return rows == kRowsAny ? k_flat_sweep<T, PRE, true, kRowsAny> : k_flat_sweep<T, PRE, true, kRowsQuick>;
 }
 
@@ -1424,7 +1433,7 @@ static void flat_launch_choice(const FlatK<T>& a, int* kernel, int64_t* blocks, 
     *blocks = sweep_grid<T>(a.n_tiles) + sweep_ring_blocks(a);
     *resident = resident_grid(k_flat_sweep_ext<T>, c_ext, a.n_tiles, kSBlock<T>);
   } else if (flat_lean(a)) {
-    static std::atomic<int> c_lean[2][64];
+    static std::atomic<int> c_lean[3][64];
     const int rows = lean_rows(a);
     *kernel = 1;
     *blocks = sweep_grid<T>(a.n_tiles);
