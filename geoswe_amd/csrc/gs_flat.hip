@@ -892,11 +892,12 @@ __device__ __forceinline__ int flat_rows(const FlatCtx<T>& x, const WaveC<T>& w,
   return r;
 }
 
-// The same rows by the general functions of gs_device.h, for every operand.
-template <typename T, bool PRE, bool EXT, bool LEAN>
+// The same rows by the general functions of gs_device.h, for every operand. HOT: nothing ran before
+// them, so the context is taken as it is.
+template <typename T, bool PRE, bool EXT, bool LEAN, bool HOT>
 __device__ __forceinline__ void flat_rows_general(const FlatCtx<T>& hot, const GS_C uint64_t* E, int i0, int nr, int c0,
                                                   int lane, lam_t<T>& lam) {
-  const FlatCtx<T> x = cold(hot);
+  const FlatCtx<T> x = HOT ? hot : cold(hot);
   const Phys<T>& P = x.P;
   const T ix = P.inv_dx, iy = P.inv_dy, hdx = P.half_dx, hdy = P.half_dy, g = P.g, hm = P.h_min;
   bool sm2, sm1, sC, sN;
@@ -1010,7 +1011,7 @@ __device__ __forceinline__ void flat_tile(const FlatCtx<T>& x, const TileHead& h
       r = __builtin_amdgcn_readfirstlane(flat_rows<T, PRE, EXT, LEAN, ROWS>(x, w, E, i0, nr, c0, lane, lam));
     }
   }
-  if (r < nr) flat_rows_general<T, PRE, EXT, LEAN>(x, E + 3 * r, i0 + r, nr - r, c0, lane, lam);
+  if (r < nr) flat_rows_general<T, PRE, EXT, LEAN, ROWS == kRowsGeneral>(x, E + 3 * r, i0 + r, nr - r, c0, lane, lam);
 }
 
 // Workgroup b's place in an XCD-major order: workgroups are dealt round-robin to the 8
@@ -1402,47 +1403,50 @@ static bool flat_quick(const FlatK<T>& a) {
   return !(a.wave & kWaveFast) || (a.wave & kWaveLam);
 }
 
-// The rows of the lean sweep for `a`. A float64 step of up to one wavefront per SIMD is one tile's
-// latency, which the general functions alone have less of (us per step with and without the forms:
-// 64^2 14.1 and 13.4, 150^2 14.3 and 13.6, 400^2 of 864 tiles 18.2 and 18.0; but 500^2 of 1230 tiles 20.7
-// and 20.7, 700^2 of 2250 23.8 and 25.1).
+// A float64 step of up to one wavefront per SIMD is one tile's latency, of which the general functions
+// alone have less (us per lean step with and without the forms: 64^2 14.0 and 12.8, 150^2 14.2 and 13.1,
+// 400^2 of 864 tiles 18.2 and 17.8; but 500^2 of 1230 tiles 20.7 and 20.7, 700^2 of 2250 23.8 and 25.1).
 template <typename T>
-static int lean_rows(const FlatK<T>& a) {
-  if (sizeof(T) == 8 && a.n_tiles <= 1024) return kRowsGeneral;
-  return flat_quick(a) ? kRowsQuick : kRowsAny;
+static bool flat_small(const FlatK<T>& a) {
+  return sizeof(T) == 8 && a.n_tiles <= 1024;
 }
 
+// The lean and the plain sweep for `a`. (The extended one gains nothing from rows of their own: 400^2 with
+// the forcing tail 22.8 us against 21.5.)
 template <typename T, bool PRE>
-static auto lean_sweep(int rows) -> void (*)(FlatK<T>, FlatLaunch<T>) {
+static auto lean_sweep(const FlatK<T>& a) -> void (*)(FlatK<T>, FlatLaunch<T>) {
   if constexpr (sizeof(T) == 8)
-    if (rows == kRowsGeneral) return k_flat_sweep<T, PRE, true, kRowsGeneral>;
-  return rows == kRowsAny ? k_flat_sweep<T, PRE, true, kRowsAny> : k_flat_sweep<T, PRE, true, kRowsQuick>;
+    if (flat_small(a)) return k_flat_sweep<T, PRE, true, kRowsGeneral>;
+  return flat_quick(a) ? k_flat_sweep<T, PRE, true, kRowsQuick> : k_flat_sweep<T, PRE, true, kRowsAny>;
+}
+template <typename T>
+static auto plain_sweep(const FlatK<T>& a) -> void (*)(FlatK<T>, FlatLaunch<T>) {
+  if constexpr (sizeof(T) == 8)
+    if (flat_small(a)) return k_flat_sweep<T, false, false, kRowsGeneral>;
+  return k_flat_sweep<T, false, false>;
+}
+// Each one's number, for a cache by kernel.
+template <typename T>
+static int sweep_slot(const FlatK<T>& a) {
+  const int rows = flat_small(a) ? kRowsGeneral : flat_quick(a) ? kRowsQuick : kRowsAny;
+  return (flat_ext(a) ? 6 : flat_lean(a) ? 0 : 3) + rows;
 }
 
 // The launch gs_flat_step makes for `a` (without the pre-friction state): which kernel, its
 // grid and the kernel's resident grid on this device.
 template <typename T>
 static void flat_launch_choice(const FlatK<T>& a, int* kernel, int64_t* blocks, int64_t* resident) {
-  static std::atomic<int> c_plain[64], c_ext[64];
+  static std::atomic<int> cache[9][64];
   if (a.n_tiles <= 0) {
     *kernel = 0;
     *blocks = flat_grid<T, 1>(a.nchunks);
     *resident = *blocks;
-  } else if (flat_ext(a)) {
-    *kernel = 2;
-    *blocks = sweep_grid<T>(a.n_tiles) + sweep_ring_blocks(a);
-    *resident = resident_grid(k_flat_sweep_ext<T>, c_ext, a.n_tiles, kSBlock<T>);
-  } else if (flat_lean(a)) {
-    static std::atomic<int> c_lean[3][64];
-    const int rows = lean_rows(a);
-    *kernel = 1;
-    *blocks = sweep_grid<T>(a.n_tiles);
-    *resident = resident_grid(lean_sweep<T, false>(rows), c_lean[rows], a.n_tiles, kSBlock<T>);
-  } else {
-    *kernel = 1;
-    *blocks = sweep_grid<T>(a.n_tiles) + sweep_ring_blocks(a);
-    *resident = resident_grid(k_flat_sweep<T, false>, c_plain, a.n_tiles, kSBlock<T>);
+    return;
   }
+  auto kern = flat_ext(a) ? k_flat_sweep_ext<T> : flat_lean(a) ? lean_sweep<T, false>(a) : plain_sweep(a);
+  *kernel = flat_ext(a) ? 2 : 1;
+  *blocks = sweep_grid<T>(a.n_tiles) + sweep_ring_blocks(a);
+  *resident = resident_grid(kern, cache[sweep_slot(a)], a.n_tiles, kSBlock<T>);
 }
 
 // The fused step: row-sweep tiles when the descriptor has them, else chunks of the run table.
@@ -1462,7 +1466,7 @@ static int flat_step_launch(const FlatK<T>& a, FlatLaunch<T> l, hipStream_t s) {
   }
   if (a.n_tiles > 0 && a.pre[0] && !ext && flat_lean(a)) {
     // 1536^2 adjoint: 33.5 us against the general pre-friction sweep's 36
-    hipLaunchKernelGGL((lean_sweep<T, true>(lean_rows(a))), dim3(sweep_grid<T>(a.n_tiles)), dim3(kSBlock<T>), 0, s, a, l);
+    hipLaunchKernelGGL((lean_sweep<T, true>(a)), dim3(sweep_grid<T>(a.n_tiles)), dim3(kSBlock<T>), 0, s, a, l);
     GS_HIP(hipGetLastError(), "k_flat_sweep(pre, lean) launch");
   } else if (a.n_tiles > 0 && a.pre[0]) {
     hipLaunchKernelGGL((k_flat_sweep<T, true>), dim3(sweep_grid<T>(a.n_tiles)), dim3(kSBlock<T>), 0, s, a, l);
@@ -1471,10 +1475,10 @@ static int flat_step_launch(const FlatK<T>& a, FlatLaunch<T> l, hipStream_t s) {
     hipLaunchKernelGGL((k_flat_sweep_ext<T>), dim3(sweep_grid<T>(a.n_tiles) + l.ring_blocks), dim3(kSBlock<T>), 0, s, a, l);
     GS_HIP(hipGetLastError(), "k_flat_sweep_ext launch");
   } else if (a.n_tiles > 0 && flat_lean(a)) {
-    hipLaunchKernelGGL((lean_sweep<T, false>(lean_rows(a))), dim3(sweep_grid<T>(a.n_tiles)), dim3(kSBlock<T>), 0, s, a, l);
+    hipLaunchKernelGGL((lean_sweep<T, false>(a)), dim3(sweep_grid<T>(a.n_tiles)), dim3(kSBlock<T>), 0, s, a, l);
     GS_HIP(hipGetLastError(), "k_flat_sweep(lean) launch");
   } else if (a.n_tiles > 0) {
-    hipLaunchKernelGGL((k_flat_sweep<T, false>), dim3(sweep_grid<T>(a.n_tiles) + l.ring_blocks), dim3(kSBlock<T>), 0, s, a, l);
+    hipLaunchKernelGGL(plain_sweep(a), dim3(sweep_grid<T>(a.n_tiles) + l.ring_blocks), dim3(kSBlock<T>), 0, s, a, l);
     GS_HIP(hipGetLastError(), "k_flat_sweep launch");
   } else {
     hipLaunchKernelGGL((k_flat_step<T, 1>), dim3(flat_grid<T, 1>(a.nchunks)), dim3(kFBlock), 0, s, a, l.next_dt);
