@@ -822,7 +822,7 @@ __device__ __forceinline__ int flat_rows(const FlatCtx<T>& x, const WaveC<T>& w,
     } else {
       const FlatCtx<T> y = cold(x);
       if (EXT && x.rain_mode == 3 && lm_lane(act)) rr0 = rh + x.frame[gat(y.rain_lookup + gC, eC.below * 4u)];
-      if (x.P.friction) {
+      if (EXT ? y.P.friction : x.P.friction) {
         if (y.n_field || y.cls) {
           if (lm_lane(act)) n = y.n_field ? gat(y.n_field + gC, eC.below * es) : x.ntab[gat(y.cls + gC, eC.below)];
         } else {
@@ -837,7 +837,10 @@ __device__ __forceinline__ int flat_rows(const FlatCtx<T>& x, const WaveC<T>& w,
       if (lm_lane(act)) fin = force_load<T, EXT>(y, fg, gC, eC.below * es, eC.below);
     }
     T h, hu, hv, speed;
-    update_w<T>(hC, huC, hvC, rr0, rhu, rhv, n, act, x.P, w, h, hu, hv, speed, odd);
+    // the extended sweep has no scalar registers for the physics switches either (held, they cost 20 lane
+    // reads more in float32 and 144 in float64: 2500^2 with the forcing tail 87 us per step against 86)
+    if constexpr (EXT) update_w<T>(hC, huC, hvC, rr0, rhu, rhv, n, act, cold(x).P, w, h, hu, hv, speed, odd);
+    else update_w<T>(hC, huC, hvC, rr0, rhu, rhv, n, act, x.P, w, h, hu, hv, speed, odd);
     const bool left = lm_any(odd);
     if (PRE) {   // the first three statements of update(), kept for its reverse
       const FlatCtx<T> y = cold(x);
