@@ -646,16 +646,18 @@ GS_HD void update_w(T q0, T q1, T q2, T rr0, T r1, T r2, T n, lmask act, const P
     const T v = quot_w(hv, hs, yh);
     const T m2 = u * u + v * v;
     T modU = root0_w(m2);
+    const T h43 = pow_m43(hs);
+    // one branch for what few rows hold: velocities below 2^-48, which take the general root (still
+    // water, 0, is in order), and those above the cap
     lmask creep = lm_lt(m2, Range<T>::root()) & live;
-    if (lm_any(creep)) {   // still water is in order; velocities below 2^-48 take the general root
+    if (lm_any(creep | (lm_gt(modU, w.vcap) & live))) {
       creep = creep & lm_gt(m2, T(0));
       if (lm_any(creep)) modU = lm_sel(creep, vsqrt(here(m2)), modU);
-    }
-    const T h43 = pow_m43(hs);
-    const lmask fastw = lm_gt(modU, w.vcap) & live;
-    if (lm_any(fastw)) {
-      const T n_cri = vsqrt(vdiv(T(1), (((T(1.0e-10) + here(w.dt)) * P.g) * h43) * (modU + T(1.0e-30))));
-      n = lm_sel(fastw & lm_gt(n_cri, n), n_cri, n);
+      const lmask fastw = lm_gt(modU, w.vcap) & live;
+      if (lm_any(fastw)) {
+        const T n_cri = vsqrt(vdiv(T(1), (((T(1.0e-10) + here(w.dt)) * P.g) * h43) * (modU + T(1.0e-30))));
+        n = lm_sel(fastw & lm_gt(n_cri, n), n_cri, n);
+      }
     }
     const T Cf = ((w.g * n) * n) * h43;
     T alpha;
