@@ -137,7 +137,7 @@ def flat_layout_leg(nx, ny, bed, steps, warmup, dense_depth=None) -> dict:
     out = {"value": cells * steps / wall, "unit": "cell-updates/s", "steps": steps, "ms_per_step": 1e3 * wall / steps,
            "kernel_ms": kern_ms, "tiles": int(len(s.fm.tile_e0)),
            "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                        "frac": achieved / HBM_PEAK_GBS, "kernel": "gs::k_flat_sweep<float, false, true>",
+                        "frac": achieved / HBM_PEAK_GBS, "kernel": "gs::k_flat_sweep<float, false, true, 0>",
                         "bytes_per_cell": BYTES_PER_CELL["flat"]}}
     if dense_depth is not None:
         out["equals_dense"] = bool(np.array_equal(s.depth(), dense_depth))
@@ -312,7 +312,7 @@ def coastal_leg(n: int, steps: int, sweep_rows=None, forcings: bool = False) -> 
                    "layout": "flat", "active_cells": int(nact), "stored_cells": int(fm.n_stored),
                    "sweep_tiles": int(len(fm.tile_e0)), "sweep_rows": int(fm.tile_irc[:, 1].max(initial=0))},
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                     "frac": achieved / HBM_PEAK_GBS, "traffic": traffic, "kernel": "gs::k_flat_sweep<float, false, true>",
+                     "frac": achieved / HBM_PEAK_GBS, "traffic": traffic, "kernel": "gs::k_flat_sweep<float, false, true, 0>",
                      "kernel_ms": ms_f, "bytes_per_cell": bpc},
         "dense_ms_per_step": ms_d,
         "dense_equals_flat": ok,
@@ -863,7 +863,7 @@ def main():
         # against the device's measured float32 issue rate; achieved/peak/frac are the HBM figures
         "roofline": {"bound": "valu" if valu else "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
-                     "kernel": "gs::k_dense_sweep<float, 1, true, float, unsigned int>" if args.layout == "dense" else "gs::k_flat_sweep<float, false, true>",
+                     "kernel": "gs::k_dense_sweep<float, 1, true, float, unsigned int>" if args.layout == "dense" else "gs::k_flat_sweep<float, false, true, 0>",
                      "kernel_ms": kern_ms, "bytes_per_cell": BYTES_PER_CELL[args.layout], "valu": valu,
                      "copy_GBps": copy["GBps_read_plus_write"],
                      "frac_of_copy": achieved / copy["GBps_read_plus_write"]},

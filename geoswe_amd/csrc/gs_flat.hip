@@ -1113,8 +1113,8 @@ __global__ __launch_bounds__(kFBlock) void k_flat_ring_force(FlatK<T> a) {
 // float32 steps are held to 80 VGPRs (6 wavefronts per SIMD), where no row reloads a spilled
 // register. LEAN (a domain with no per-cell Manning field or class plane, running maximum or
 // active-cell forcing) drops those paths. us per step, general functions with 4-row tiles before
-// and wavefront forms now: 2048^2 coastal domain (lean) 63 and 40, 1500^2 with the forcing tail
-// (below) 69 and 57.
+// and wavefront forms now: 2048^2 coastal domain (lean) 63 and 38, 1500^2 with the forcing tail
+// (below) 69 and 45.
 template <typename T, bool PRE, bool LEAN = false, int ROWS = kRowsOf<LEAN>>
 __global__ __launch_bounds__(kSBlock<T>) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 6 : 1))) void k_flat_sweep(FlatK<T> a, FlatLaunch<T> l) {
   // What waits on nothing but the argument is asked for first: the tile's place, the Manning table

@@ -135,8 +135,6 @@ __device__ __forceinline__ void take_loaded(double& a, double& b, double& c, dou
 }
 // the mask of each lane's upper neighbour (lane l gets bit l + 1; the top lane's is not used)
 __device__ __forceinline__ lmask lm_upper(lmask m) { return m >> 1; }
-// a uniform value in a vector register: fast instructions that read a scalar register run at
-// half rate
 // A uniform value in scalar registers.
 __device__ __forceinline__ float sreg(float x) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(x))); }
 __device__ __forceinline__ double sreg(double x) {
@@ -154,6 +152,8 @@ __device__ __forceinline__ double here(double x) {
   asm volatile("" : "+v"(x));
   return x;
 }
+// A uniform value in a vector register: fast instructions that read a scalar register run at half
+// rate.
 __device__ __forceinline__ float vreg(float x) {
   float y;
   __asm__("v_mov_b32 %0, %1" : "=v"(y) : "s"(x));

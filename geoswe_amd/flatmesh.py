@@ -199,9 +199,10 @@ def sweep_rows_for(busy: int) -> int:
     gives TILE_TARGET to 2*TILE_TARGET tiles, at most MAX_SWEEP_ROWS.
 
     A tile pays for a row and a half of lead-in, few tall tiles leave SIMDs idle. Coastal domains on
-    MI355X, us for 20 lean steps at heights 2/4/6/8/12/16: 21207 busy rows 841/699/661/743/844/1094,
-    36626 rows 1132/1017/865/960/1118/1260, 77431 rows (from 4) 1595/1537/1465/1533/1508; 139562 rows
-    2373 at 12, 2425 at 16, 2532 at 20; 300224 rows within 4 % from 10 to 32."""
+    MI355X, us for 20 lean steps at heights 2/4/6/8/12/16: 21207 busy rows 841/699/661/743/844/1094
+    (where the lower bound on the tiles gives 4), 36626 rows 1132/1017/865/960/1118/1260, 77431 rows
+    (from 4) 1595/1537/1465/1533/1508; 139562 rows 2373 at 12, 2425 at 16, 2532 at 20; 300224 rows within
+    4 % from 10 to 32."""
     busy = int(busy)
     rows = max(math.isqrt(busy // 1000), busy // (2 * TILE_TARGET) + 1)
     return max(1, min(rows, busy // TILE_TARGET, MAX_SWEEP_ROWS))
