@@ -1406,33 +1406,33 @@ static bool flat_quick(const FlatK<T>& a) {
   return !(a.wave & kWaveFast) || (a.wave & kWaveLam);
 }
 
-// A float64 step of up to one wavefront per SIMD is one tile's latency, of which the general functions
-// alone have less (us per lean step with and without the forms: 64^2 14.0 and 12.8, 150^2 14.2 and 13.1,
-// 400^2 of 864 tiles 18.2 and 17.8; but 500^2 of 1230 tiles 20.7 and 20.7, 700^2 of 2250 23.8 and 25.1).
+// The rows of the lean and the plain sweep for `a`. The general functions alone where the forms may not
+// be taken at all (h_min below 2^-21 in float32), and for a float64 step of up to one wavefront per
+// SIMD, which is one tile's latency (us per lean step with and without the forms: 64^2 14.0 and 12.8,
+// 150^2 14.2 and 13.1, 400^2 of 864 tiles 18.2 and 17.8; but 500^2 of 1230 tiles 20.7 and 20.7, 700^2 of 2250
+// 23.8 and 25.1). The extended sweep gains nothing from it: 400^2 with the forcing tail 22.8 us against 21.5.
 template <typename T>
-static bool flat_small(const FlatK<T>& a) {
-  return sizeof(T) == 8 && a.n_tiles <= 1024;
+static int sweep_rows_kind(const FlatK<T>& a) {
+  if (!(a.wave & kWaveFast) || (sizeof(T) == 8 && a.n_tiles <= 1024)) return kRowsGeneral;
+  return flat_quick(a) ? kRowsQuick : kRowsAny;
 }
 
-// The lean and the plain sweep for `a`. (The extended one gains nothing from rows of their own: 400^2 with
-// the forcing tail 22.8 us against 21.5.)
 template <typename T, bool PRE>
 static auto lean_sweep(const FlatK<T>& a) -> void (*)(FlatK<T>, FlatLaunch<T>) {
-  if constexpr (sizeof(T) == 8)
-    if (flat_small(a)) return k_flat_sweep<T, PRE, true, kRowsGeneral>;
-  return flat_quick(a) ? k_flat_sweep<T, PRE, true, kRowsQuick> : k_flat_sweep<T, PRE, true, kRowsAny>;
+  switch (sweep_rows_kind(a)) {
+    case kRowsGeneral: return k_flat_sweep<T, PRE, true, kRowsGeneral>;
+    case kRowsAny: return k_flat_sweep<T, PRE, true, kRowsAny>;
+    default: return k_flat_sweep<T, PRE, true, kRowsQuick>;
+  }
 }
 template <typename T>
 static auto plain_sweep(const FlatK<T>& a) -> void (*)(FlatK<T>, FlatLaunch<T>) {
-  if constexpr (sizeof(T) == 8)
-    if (flat_small(a)) return k_flat_sweep<T, false, false, kRowsGeneral>;
-  return k_flat_sweep<T, false, false>;
+  return sweep_rows_kind(a) == kRowsGeneral ? k_flat_sweep<T, false, false, kRowsGeneral> : k_flat_sweep<T, false, false>;
 }
 // Each one's number, for a cache by kernel.
 template <typename T>
 static int sweep_slot(const FlatK<T>& a) {
-  const int rows = flat_small(a) ? kRowsGeneral : flat_quick(a) ? kRowsQuick : kRowsAny;
-  return (flat_ext(a) ? 6 : flat_lean(a) ? 0 : 3) + rows;
+  return (flat_ext(a) ? 6 : flat_lean(a) ? 0 : 3) + sweep_rows_kind(a);
 }
 
 // The launch gs_flat_step makes for `a` (without the pre-friction state): which kernel, its

@@ -27,10 +27,11 @@ def _state(nx, ny, dtype, odd):
     return q, bed, rng
 
 
-def _solver(shape, rows, speed, dtype, odd, maxh, ext):
+def _solver(shape, rows, speed, dtype, odd, maxh, ext, h_min=None):
     nx, ny = shape
     q, bed, rng = _state(nx, ny, dtype, odd)
-    cfg = Config(bc_x="fall", bc_y="fall", dtype=dtype, friction="manning", manning_n=0.03, rainfall=20.0 / 3.6e6)
+    cfg = Config(bc_x="fall", bc_y="fall", dtype=dtype, friction="manning", manning_n=0.03, rainfall=20.0 / 3.6e6,
+                 **({} if h_min is None else {"h_min": h_min}))
     s = Solver2D(Mesh2D(nx, ny, 2.0, 2.0), cfg, q, bed)
     mask = rng.random((nx, ny)) > 0.06
     mask[nx // 2, ny // 2] = True
@@ -58,6 +59,21 @@ def test_tiles_equal_chunks(gpu, shape, rows, speed, maxh, ext, dtype, odd):
     a, b = out
     assert a[1:4] == b[1:4] and np.array_equal(a[0], b[0])
     assert not maxh or np.array_equal(a[4], b[4])
+
+
+@pytest.mark.parametrize("dtype,h_min", [("float32", 1.0e-7), ("float64", 1.0e-13)])
+@pytest.mark.parametrize("maxh,ext", [(False, False), (True, False), (True, True)])
+@pytest.mark.parametrize("speed", SPEEDS[:2])
+@pytest.mark.parametrize("shape,rows", [((17, 61), 2), ((2100, 70), 1)])
+def test_dry_floors_that_the_forms_do_not_take(gpu, shape, rows, speed, maxh, ext, dtype, h_min):
+    """Below 2^-21 (float32) and 2^-36 (float64) the sweeps step by the general functions alone."""
+    out = []
+    for trav in ("tiles", "chunks"):
+        c = _solver(shape, rows, speed, dtype, False, maxh, ext, h_min)
+        c.traversal = trav
+        c.advance(3)
+        out.append((c.q_flat(), c.t, c._clockv().lam_bits))
+    assert out[0][1:] == out[1][1:] and np.array_equal(out[0][0], out[1][0])
 
 
 @pytest.mark.parametrize("dtype", ["float32", "float64"])
