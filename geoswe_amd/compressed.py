@@ -57,6 +57,7 @@ class CompressedSolver:
         self._infil = self._drain = self._ga = None
         self._rain_lookup = None
         self._rmode = None
+        self._auto_rows = False            # the tile height was picked for this domain alone
         self._tables_taken = False         # an Ensemble or GaugeMisfit holds this solver's device pointers
         t = np.zeros(L.MAX_CLASSES_PLANE, self.dtype)
         t[:len(ntab)] = ntab
@@ -114,6 +115,7 @@ class CompressedSolver:
             cp = np.zeros((nxp, nyp), np.uint8)
             cp[g:g + nx, g:g + ny] = s._cls.download()[:, :ny]
         out = cls(mesh, cfg, fm, q_pad, b_pad, flags, ntab, nf, cfl_linf, track_max_depth, h_min_cfl, cls_pad=cp)
+        out._auto_rows = sweep_rows is None
         c = s._clockv()
         if c.t != 0.0:
             L.call("gs_clock_reset", C.c_void_p(out._clock.ptr), C.c_double(float(c.t)), None)

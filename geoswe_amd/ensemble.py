@@ -16,9 +16,11 @@ import ctypes as C
 import math
 from typing import Optional, Sequence
 
+import numpy as np
+
 from . import _lib as L
 from .compressed import CompressedSolver
-from .flatmesh import mesh_sweep_tiles, sweep_rows_for
+from .flatmesh import mesh_sweep_tiles, sweep_rows_for, sweep_rows_for64
 
 
 class Ensemble:
@@ -59,13 +61,15 @@ class Ensemble:
         # alone); autotune(heights=...) may pick another.
         if sweep_rows is not None and not (1 <= int(sweep_rows) <= 1024):
             raise ValueError(f"sweep_rows must be in 1..1024, got {sweep_rows}")
+        rows_for = sweep_rows_for64 if np.dtype(dt0) == np.float64 else sweep_rows_for
         self._build(int(sweep_rows) if sweep_rows is not None
-                    else sweep_rows_for(sum(int(m.fm.tile_irc[:, 1].sum()) for m in members)),
+                    else rows_for(sum(int(m.fm.tile_irc[:, 1].sum()) for m in members)),
                     exact=sweep_rows is not None)
 
     def _build(self, rows: int, exact: bool = True) -> None:
         """The native ensemble over the members' tiles of `rows` rows (`exact`: every member
-        re-tiled to that height; else members already at least as tall keep their tiles)."""
+        re-tiled to that height; else members already at least as tall keep their tiles, unless they are
+        float64 domains tall enough to make one round of wavefronts by themselves)."""
         self.close()
         members = self.members
         self.sweep_rows = int(rows)
@@ -73,7 +77,8 @@ class Ensemble:
         tiles = []
         for k, m in enumerate(members):
             tall = int(m.fm.tile_irc[:, 1].max(initial=0))
-            if m.n_active == 0 or (tall == rows if exact else tall >= rows):
+            alone = m._auto_rows and np.dtype(m.dtype) == np.float64
+            if m.n_active == 0 or (tall == rows if exact or alone else tall >= rows):
                 continue                       # keep the member's own tiles
             key = (k, rows)
             if key not in self._tile_cache:

@@ -112,3 +112,25 @@ def test_pre_friction_state(gpu, shape, rows, dtype, speed):
     L.sync(None)
     assert np.array_equal(a.q_flat(), b.q_flat()) and a._clockv().lam_bits == b._clockv().lam_bits
     assert (pre[0].download()[a.fm.active] > 0).any()
+
+
+def test_float64_members_at_one_height(gpu):
+    """Float64 members whose own tile heights differ (3, 1 and 2 rows) step at the height their total
+    calls for, with their own tables left as they are; a height that the caller gave a member stays."""
+    from geoswe_amd.ensemble import Ensemble
+    from geoswe_amd.flatmesh import sweep_rows_for64
+    shapes = ((110, 3700), (40, 130), (60, 1200), (30, 200))
+    members, plain = ([_solver(sh, 5 if k == 3 else None, SPEEDS[0], "float64", False, False, False)
+                       for k, sh in enumerate(shapes)] for _ in range(2))
+    own = [int(m.fm.tile_irc[:, 1].max()) for m in members]
+    assert own == [3, 1, 2, 5]
+    rows = sweep_rows_for64(sum(int(m.fm.tile_irc[:, 1].sum()) for m in members))
+    assert rows == 3
+    e = Ensemble(members, graph_batch=2)
+    assert e.sweep_rows == rows and len(e._tiles) == 2      # the second and the third member
+    assert [int(m.fm.tile_irc[:, 1].max()) for m in members] == own
+    e.advance(5)
+    for m, p in zip(members, plain):
+        p.advance(5)
+        assert m.t == p.t and np.array_equal(m.q_flat(), p.q_flat())
+    e.close()
